@@ -242,3 +242,56 @@ def test_srnl_backward_tiny_stage3_shape(device):
     got = srnl_packed_backward(tuple(torch.from_numpy(m).to(device) for m in mems), x.to(device), q.to(device),
                                [14] * 4, dy.to(device), q_raw=True)
     _check([g.float() for g in got], want, "Tiny stage 3", tol=1e-2)
+
+
+def _block_form_case(device, head_dim, chunks, length, *, heads=1, batch=1, dtype=torch.float32, kind="perturbed",
+                     gate_scale=1.0, offset=0, q_raw=True):
+    """Gradients of random lines and the tolerance for them: every gradient is a sum of
+    products along at most one chunk (the gains never expand), so an FP32 evaluation is
+    within (chunk + 4 d) roundings of 2^-24, doubled, of the gradient's scale; 16-bit inputs
+    round the returned dx and dq once more (2^-8 for bf16, 2^-11 for fp16)."""
+    from visionhope_amd.models.srnl_core.chunk import srnl_packed_backward
+
+    def place(t):
+        """t on the GPU, starting ``offset`` elements into its storage."""
+        flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)
+        flat[offset:] = t.reshape(-1).to(device)
+        return flat[offset:].view(t.shape)
+
+    directions = len(chunks)
+    mems = list(memories(directions, heads, head_dim, kind=kind, seed=head_dim + 201))
+    mems[3:] = [m * gate_scale for m in mems[3:]]
+    x = randn(batch, directions, heads, length, head_dim, seed=202).to(dtype)
+    q = (randn(batch, directions, length, heads * head_dim, seed=203).to(dtype) if q_raw else
+         torch.nn.functional.normalize(randn(batch, directions, heads, length, head_dim, seed=203), dim=-1))
+    dy = randn(batch, directions, heads, length, head_dim, seed=204)
+    want = _oracle_grads(x.float(), q.float(), mems, chunks, dy, q_raw)
+    got = srnl_packed_backward(tuple(torch.from_numpy(m).to(device) for m in mems), place(x), place(q), chunks,
+                               place(dy), q_raw=q_raw)
+    tol = 2.0 ** -23 * (max(chunks) + 4 * head_dim)
+    rounding = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    what = f"d={head_dim} chunks={chunks} {dtype}"
+    _check(got[:5], want[:5], what, tol)
+    for name, g, w in zip(("dx", "dq"), got[5:], want[5:]):
+        assert_close(g.double().cpu().numpy(), w, tol + rounding, f"{what} {name}")
+
+
+@pytest.mark.parametrize("head_dim,chunks,length", [
+    (16, [1, 2, 15, 16], 35), (16, [17, 31, 32, 33], 70), (16, [63, 64, 65, 3], 140), (16, [127, 128, 129, 16], 290),
+    (16, [256, 200, 255, 130], 530), (16, [39, 40, 64, 128], 40), (32, [1, 15, 16, 7], 33), (32, [17, 32, 33, 48], 100),
+    (32, [64, 65, 100, 128], 210), (32, [256, 129, 192, 16], 520)])
+def test_srnl_backward_block_edges(device, head_dim, chunks, length):
+    """The block-form kernels (head_dim 16 and 32) around their tile, wave-count and segment
+    edges: 1, 2, 4 or 8 waves, chunks of one slot to several segments, ragged last chunks,
+    directions with fewer blocks than waves, and lines of a single chunk."""
+    _block_form_case(device, head_dim, chunks, length, heads=2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim,directions", [(16, 1), (32, 2)])
+def test_srnl_backward_block_inputs(device, head_dim, directions, dtype):
+    """Every activation type, tensors that start at an odd element of their storage, one and
+    two directions, and saturated gates with strong memories (retentions down to the clamp)."""
+    chunks = [19, 40][:directions]
+    _block_form_case(device, head_dim, chunks, 90, heads=3, batch=2, dtype=dtype, offset=1)
+    _block_form_case(device, head_dim, chunks, 90, dtype=dtype, kind="strong", gate_scale=4.0, offset=3, q_raw=False)

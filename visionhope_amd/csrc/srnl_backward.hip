@@ -13,7 +13,11 @@
 // clamp routes it to alpha and |k|^2 only when it binds, and the query normalisation
 // drops its projection below the epsilon.
 //
-// Structure (one workgroup of D lanes per line, lane i holding row i of the d x d
+// head_dim 16 and 32 run the block form on the matrix cores (srnl_backward_blocks.hip); the
+// kernel here steps token by token and serves head_dim 4 and 8, whose matrices are smaller
+// than a matrix-core tile.
+//
+// Structure of the stepped kernel (D lanes per line, lane i holding row i of the d x d
 // matrices; all math fp32):
 //   1. forward state pass: the chunk-start state of every chunk goes to the workspace;
 //   2. chunks in reverse: the chunk's keys, values and gates are recomputed from its
@@ -30,32 +34,13 @@
 #include <cstdint>
 #include <type_traits>
 
-#include "vh_common.h"
+#include "srnl_backward.h"
 
 namespace vh {
-
-constexpr int kBwdMaxChunk = 64;     // chunks up to this length use the small-LDS variant
-constexpr int kBwdLongChunk = 256;   // longest chunk of the backward (lines.cu:252-760 range)
 
 // The chunk buffers of a workgroup hold CMAX tokens: 64, or 256 when a direction's chunk
 // is longer (the long-line backward; about 42 KB of LDS more at d = 16).
 inline int bwd_cmax(int64_t max_chunk) { return max_chunk <= kBwdMaxChunk ? kBwdMaxChunk : kBwdLongChunk; }
-
-struct BwdParams {
-    const void* x;      // [B, R, heads, N, D] io dtype
-    const void* q;      // raw: [B, R, N, heads * D] io dtype; else fp32 [B, R, heads, N, D]
-    const float* dy;    // [B, R, heads, N, D]
-    const float* m0[5]; // M_m, M_v, M_k [S, D, D]; M_eta, M_alpha [S, D]; S = R * heads, or one per line
-    int per_line;       // 1: state s = line; 0: s = line % (R * heads), shared over the batch
-    float* dx;          // [B, R, heads, N, D]
-    float* dq;          // layout of q, fp32
-    float* dline;       // [lines, 3 D^2 + 2 D] per-line gradient of the initial state
-    float* states;      // [lines, nc, 3 D^2 + 2 D] chunk-start states
-    float* gtraj;       // [lines, CMAX, D, D] gain trajectory of the current chunk
-    int64_t B, R, heads, N, nc;
-    int chunk[4];
-    vh_srnl_consts k;
-};
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -67,15 +52,10 @@ __device__ __forceinline__ float dpp_f(float v) {
 // mirror, quad xor 1 and 2, row xor), so all lanes of a group end with the same bits.
 template <int D>
 __device__ __forceinline__ float group_sum(float v) {
-    static_assert(D == 4 || D == 8 || D == 16 || D == 32, "group of 4, 8, 16 or 32 lanes");
-    if constexpr (D >= 16) v += dpp_f<0x140>(v);   // row_mirror: lane l <-> 15 - l
+    static_assert(D == 4 || D == 8, "group of 4 or 8 lanes");
     if constexpr (D >= 8) v += dpp_f<0x141>(v);    // row_half_mirror: l <-> 7 - l in each 8
     v += dpp_f<0xB1>(v);                           // quad_perm [1, 0, 3, 2]
     v += dpp_f<0x4E>(v);                           // quad_perm [2, 3, 0, 1]
-    if constexpr (D == 32) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(p16[0]) + __uint_as_float(p16[1]);
-    }
     return v;
 }
 
@@ -86,13 +66,6 @@ __device__ __forceinline__ void lds_fence() { asm volatile("" ::: "memory"); }
 template <typename T>
 __device__ __forceinline__ float ld(const void* p, int64_t i) {
     return to_f32(static_cast<const T*>(p)[i]);
-}
-
-// d(eta^)/d(cap) of eta^ = cap (1 - exp(-u)), u = eta / cap: (1 - e^-u) - u e^-u, by its
-// series u^2 (1/2 - u/3 + u^2/8 - u^3/30 + u^4/144) below u = 1e-3 (cancellation).
-__device__ __forceinline__ float softcap_dcap(float u, float e_neg) {
-    if (u < 1e-3f) return u * u * (0.5f + u * (-1.f / 3.f + u * (1.f / 8.f + u * (-1.f / 30.f + u / 144.f))));
-    return -expm1f(-u) - u * e_neg;
 }
 
 // LPW lines per workgroup, D lanes each (lines ln = LPW blockIdx.x + sub share (b, r), so
@@ -483,6 +456,7 @@ namespace {
 
 struct BwdLayout {
     int64_t lines, nc, sd, cmax;
+    int waves, segs;   // block form (head_dim 16 and 32), else 0
     size_t states, traj, dline, total;
 };
 
@@ -493,11 +467,18 @@ BwdLayout bwd_layout(int64_t B, int64_t R, int64_t heads, int64_t N, int d, cons
     for (int64_t r = 0; r < R; ++r) l.nc = std::max<int64_t>(l.nc, (N + chunks[r] - 1) / chunks[r]);
     l.sd = 3 * int64_t(d) * d + 2 * d;
     auto round = [](size_t v) { return (v + 63) / 64 * 64; };
-    l.states = round(static_cast<size_t>(l.lines * l.nc * l.sd));
     int64_t cmax = 0;
     for (int64_t r = 0; r < R; ++r) cmax = std::max<int64_t>(cmax, chunks[r]);
-    l.cmax = bwd_cmax(cmax);
-    l.traj = round(static_cast<size_t>(l.lines * l.cmax * d * d));
+    if (d >= 16) {
+        l.waves = bwd_block_waves(d, cmax);
+        l.segs = bwd_block_segs(l.waves, cmax);
+        l.states = round(static_cast<size_t>(l.lines * l.nc * d * d));
+        l.traj = l.segs > 1 ? round(static_cast<size_t>(l.lines * l.waves * l.segs * d * d)) : 0;
+    } else {
+        l.cmax = bwd_cmax(cmax);
+        l.states = round(static_cast<size_t>(l.lines * l.nc * l.sd));
+        l.traj = round(static_cast<size_t>(l.lines * l.cmax * d * d));
+    }
     l.dline = round(static_cast<size_t>(l.lines * l.sd));
     l.total = (l.states + l.traj + l.dline) * sizeof(float);
     return l;
@@ -553,20 +534,20 @@ int vh_srnl_backward(const void* x, const void* q, int32_t io_dtype, int32_t q_r
     bp.dline = ws + lay.states + lay.traj;
     bp.B = B; bp.R = R; bp.heads = heads; bp.N = N; bp.nc = lay.nc;
     for (int r = 0; r < 4; ++r) bp.chunk[r] = static_cast<int>(chunks[r < R ? r : R - 1]);
+    bp.segs = lay.segs;
+    bp.io_dtype = io_dtype; bp.q_raw = q_raw ? 1 : 0;
     bp.k = *consts;
     hipStream_t s = static_cast<hipStream_t>(stream);
     VH_REQUIRE(lay.lines < (int64_t(1) << 31), VH_ERR_SHAPE, "SRNL backward: too many lines");
-    // Lines per workgroup: consecutive heads of one (b, r), as many as LDS allows (one line
-    // of d = 16 with 64-token buffers needs about 19 KB; 256-token buffers 43 KB; d = 32
-    // about 52 and 105 KB).
+    // Lines per workgroup: consecutive heads of one (b, r) when 4 (2 with 256-token buffers)
+    // divide the heads.
     auto launch = [&](auto kern, int lpw, int d) {
         hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(lay.lines / lpw)), dim3(d * lpw), 0, s, bp);
     };
     auto go = [&](auto dc, auto tv) {
         constexpr int D = decltype(dc)::value;
         using T = decltype(tv);
-        constexpr int LS = D <= 16 ? 4 : 2;   // 64-token buffers
-        constexpr int LL = D <= 16 ? 2 : 1;   // 256-token buffers
+        constexpr int LS = 4, LL = 2;
         if (lay.cmax == kBwdMaxChunk) {
             const bool packed = heads % LS == 0;
             if (q_raw) {
@@ -594,13 +575,14 @@ int vh_srnl_backward(const void* x, const void* q, int32_t io_dtype, int32_t q_r
             default: go(dc, f16_t{}); break;
         }
     };
-    switch (head_dim) {
-        case 4: by_type(std::integral_constant<int, 4>{}); break;
-        case 8: by_type(std::integral_constant<int, 8>{}); break;
-        case 16: by_type(std::integral_constant<int, 16>{}); break;
-        default: by_type(std::integral_constant<int, 32>{}); break;
+    int rc;
+    if (head_dim >= 16) {
+        rc = launch_backward_blocks(bp, head_dim, lay.waves, lay.lines, s);
+    } else {
+        if (head_dim == 4) by_type(std::integral_constant<int, 4>{});
+        else by_type(std::integral_constant<int, 8>{});
+        rc = check_launch("srnl_backward_kernel");
     }
-    int rc = check_launch("srnl_backward_kernel");
     if (rc) return rc;
     // Shared states: sum the B lines of each; one state per line: copy.
     const int64_t S = memories_per_line ? lay.lines : R * heads, batch = memories_per_line ? 1 : B;

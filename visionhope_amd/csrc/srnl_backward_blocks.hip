@@ -1,0 +1,902 @@
+// SRNL backward for head_dim 16 and 32: the recurrence and its adjoint in 16-token block
+// form on the FP32 matrix cores.
+//
+// Forward of one line (srnl_backward.hip states it token by token).  With Gamma_c the
+// product of the chunk gains before chunk c, the chunk-start state is S_0 Gamma_c, so only
+// Gamma_c (d x d) is carried: z = Gamma_c x, k~ = M_k z, v = M_v z, gate pre-activations
+// e.z and a.z, y = M_m (Gamma_c q^).  Inside a chunk, for a block of 16 token slots entered
+// with gain G, with a_t the product of the block's retentions before slot t, a the product
+// of all 16, and the strictly upper triangle L[s][t] = eta^_s (a_t / a_{s+1}) (k_s . k_t):
+//   R (I + L) = G K D_a + Delta             (columns r_t; Delta = k - v, D_a = diag(a_t))
+//   G' = a G - R D_e K^T = G X + Y          (D_e = diag(eta^_t a / a_{t+1}))
+//   X = a I - K D_a S, Y = -Delta S, (I + L) S = D_e K^T.
+// Adjoint, with H' = dG' the gradient of the block's exit gain (H_C = Gamma^T dGamma_{c+1}):
+//   Rb (I + L^T) = -H' K D_e                (columns r_bar_t)
+//   H = a H' + Rb D_a K^T = H' X^T
+//   dK = -H'^T R D_e + G^T Rb D_a - K (W + W^T) + Rb + ...,  W[s][t] = eta^_s (a_t / a_{s+1}) (r_s . r_bar_t), s < t
+//   d alpha_t = (phi_{t+1} - r_bar_t . r_t) / alpha_t,  phi_t = <H_t, G_t> = phi_0 + sum_{s < t} r_bar_s . delta_s
+// (the last line replaces the token-by-token inner products <H_{t+1}, G_t>; phi is taken
+// afresh at every block start, so it carries no error from block to block).  Then
+//   dz = M_v^T dv + M_k^T dk~ + e d_pre_eta + a d_pre_alpha,  dx = Gamma^T dz,
+//   dGamma_c = dGamma_{c+1} G_C^T + sum_t (dz_t x_t^T + (M_m^T dy_t) q^_t^T).
+// The regrouping is exact in real arithmetic; every product is FP32
+// (v_mfma_f32_16x16x4_f32), nothing is split or rounded to 16 bits.
+//
+// Mapping.  One workgroup per line, wave w holding block w of the current 16 W-token
+// segment of a chunk (W = 1, 2, 4 or 8 waves; longer chunks take several segments).  A
+// tile is 4 registers: lane (g = l / 16, c = l % 16) holds rows 4g..4g+3 of column c, which
+// is what the matrix core returns, the B operand of that matrix and the A operand of its
+// transpose; so mm(A, B) = A^T B needs no data movement, and where a transpose is needed it
+// goes through 1.3 KB of wave-private LDS.  Token slots are permuted: slot index n stands for
+// time 4 (n % 4) + n / 4 of the block, which puts four consecutive times into one register
+// index, so one rank-4 matrix instruction eliminates them: a 16 x 16 triangular solve is 7
+// instructions (the 4 x 4 diagonal inverses are formed on the VALU).
+//
+// Bound: the dependency chain.  A chunk is one serial chain of solves and products per line,
+// and the chunks of a line follow one another; the compulsory matrix work and the bytes take
+// well under a tenth of the time.  Times on MI355X against the token-by-token kernel (which
+// head_dim 4 and 8 still run): 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 305 us;
+// 512 lines of 3,136 tokens, d = 16, chunks of 56: 24,500 -> 802 us; 48 lines of 960 tokens,
+// d = 32, chunks of 40 and 24: 11,800 -> 769 us; 4 lines of 196 tokens, d = 32, chunks of 64:
+// 1,690 -> 77 us.
+#include <algorithm>
+#include <cmath>
+
+#include "srnl_backward.h"
+#include "srnl_device.h"
+
+namespace vh {
+namespace {
+
+constexpr int kTrStride = 20;   // floats per row of the transpose scratch (16-byte aligned rows)
+
+// acc + A^T B
+__device__ __forceinline__ v4f mm(v4f a, v4f b, v4f acc) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = mfma4(a[j], b[j], acc);
+    return acc;
+}
+
+typedef v4f v4f_any __attribute__((aligned(4)));
+typedef unsigned short us4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// Four consecutive elements of an io-dtype row as FP32.  Rows start at any element (a
+// contiguous tensor may be a view at an odd offset), so the loads assume no alignment.
+__device__ __forceinline__ v4f load_io4(const void* p, int64_t idx, int io) {
+    if (io == VH_DTYPE_F32) return *reinterpret_cast<const v4f_any*>(static_cast<const float*>(p) + idx);
+    const us4_any u = *reinterpret_cast<const us4_any*>(static_cast<const uint16_t*>(p) + idx);
+    v4f r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = io == VH_DTYPE_BF16 ? to_f32(bf16_t{u[i]}) : to_f32(f16_t{u[i]});
+    return r;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp0(float v) {   // 0 where the source lane is outside the row
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// Prefix sums over the 16 slots of a block in time order (slot c = time 4 (c % 4) + c / 4),
+// the same in every row of lanes: inclusive, exclusive and the total.
+struct Prefix {
+    float incl, excl, total;
+};
+__device__ __forceinline__ Prefix time_prefix(float v, int c) {
+    float in = v + dpp0<0x114>(v);              // row_shr 4: the previous time of the same group of four
+    in += dpp0<0x118>(in);                      // row_shr 8
+    float t = v + dpp0<0x128>(v);               // row_ror 8, 4: the group's total
+    t += dpp0<0x124>(t);
+    // every lane moves before the selects: a move inside a branch would read inactive lanes
+    const int j = c & 3;
+    const float t1 = dpp0<0x90>(t);             // quad_perm [0, 0, 1, 2]
+    float s = t + (j >= 1 ? t1 : 0.f);
+    const float s2 = dpp0<0x40>(s);             // quad_perm [0, 0, 0, 1]
+    s += j >= 2 ? s2 : 0.f;
+    const float s1 = dpp0<0x90>(s), before = j >= 1 ? s1 : 0.f;
+    return {before + in, before + dpp0<0x114>(in), dpp0<0xFF>(s)};
+}
+
+__device__ __forceinline__ float wave_sum(float v) { return row_group_sum<16>(xor16_32_sum(v)); }
+
+template <int D, int W>
+struct Shared {
+    static constexpr int ND = D / 16, NT = ND * ND;
+    // Memories as tiles [tile][lane]: N(M^T) of M_k, M_v; N(M) of M_k, M_v, M_m.
+    v4f mem[5][NT][64];
+    float ev[2][D];
+    float E[D][D + 4];                 // dGamma of the next chunk, row major
+    float tr[W][16 * kTrStride];       // transpose scratch
+    float sc[W][5][16];                // per-slot scalars, read four rows at a time
+    float diag[W][64];                 // the 4 x 4 diagonal blocks of L
+    // Block maps X, X^T, Y^T of the segment (W > 1); also the waves' partial sums.
+    v4f maps[W > 1 ? W : 1][W > 1 ? 3 : 1][NT][64];
+};
+
+// Everything the recurrence needs from the 16 tokens of one block.
+template <int ND>
+struct Tokens {
+    v4f Z[ND], K[ND], Dl[ND];      // z, k, k - v: channel rows, slot columns
+    v4f KT[ND], DlT[ND];           // the last two transposed
+    v4f Mc;                        // eta^_s a_t / a_{s+1} for the earlier slot s and the later slot t of (row, column)
+    v4f nC;                        // -(that times k_s . k_t): L above, L^T below the diagonal, negated
+    v4f De_r, Da_r;                // D_e, D_a by row
+    float De, Da, a;               // by column; product of the block's retentions
+    float dl, du;                  // this lane's entry of the diagonal inverses (lower, upper solve)
+    float inv_k, eff, alpha;
+    float dn, denom, cap, deff_deta, deff_dcap, deff_dalpha, deff_dksq, s_eta, s_alpha;
+};
+
+template <int D, int W>
+struct Line {
+    static constexpr int ND = D / 16;
+    Shared<D, W>& sh;
+    const int w, lane, g, c, tau;   // tau: time of slot c within the block
+    const vh_srnl_consts& k;
+
+    __device__ __forceinline__ v4f transpose(v4f v) const {
+        float* s = sh.tr[w];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[(4 * g + i) * kTrStride + c] = v[i];
+        __builtin_amdgcn_wave_barrier();
+        const v4f r = *reinterpret_cast<const v4f*>(&s[c * kTrStride + 4 * g]);
+        __builtin_amdgcn_wave_barrier();
+        return r;
+    }
+    __device__ __forceinline__ v4f rows_of(const float* s) const { return *reinterpret_cast<const v4f*>(s + 4 * g); }
+    __device__ __forceinline__ int row_time(int i) const { return 4 * i + g; }
+
+    // B <- (I + L^T)^-1 B and B <- (I + L)^-1 B for token-row tiles.
+    __device__ __forceinline__ void solve_lower(const Tokens<ND>& t, v4f (&b)[ND]) const {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float a1 = (c & 3) == s ? t.dl : 0.f, a2 = (c & 3) > s ? t.nC[s] : 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][s], b[j]);
+            if (s < 3)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][s], b[j]);
+        }
+    }
+    __device__ __forceinline__ void solve_upper(const Tokens<ND>& t, v4f (&b)[ND]) const {
+#pragma unroll
+        for (int s = 3; s >= 0; --s) {
+            const float a1 = (c & 3) == s ? t.du : 0.f, a2 = (c & 3) < s ? t.nC[s] : 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][s], b[j]);
+            if (s > 0)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][s], b[j]);
+        }
+    }
+
+    // Keys, values and gates of the block from x (channel rows; zero in slots past the
+    // chunk) and Gamma^T.  Slots past the chunk act as the identity.
+    __device__ __forceinline__ void tokens(const v4f (&X)[ND], bool valid, const v4f (&GamT)[ND][ND],
+                                           Tokens<ND>& t) const {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            t.Z[i] = zero;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) t.Z[i] = mm(GamT[j][i], X[j], t.Z[i]);
+        }
+        v4f V[ND];
+        float pe = 0.f, pa = 0.f, ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            t.K[i] = zero;
+            V[i] = zero;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                t.K[i] = mm(sh.mem[0][j * ND + i][lane], t.Z[j], t.K[i]);
+                V[i] = mm(sh.mem[1][j * ND + i][lane], t.Z[j], V[i]);
+            }
+            const v4f e = rows_of(&sh.ev[0][16 * i]), a = rows_of(&sh.ev[1][16 * i]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                pe += e[r] * t.Z[i][r];
+                pa += a[r] * t.Z[i][r];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ss += t.K[i][r] * t.K[i][r];
+        const float pe_raw = xor16_32_sum(pe), pa_raw = xor16_32_sum(pa) + k.retention_bias;
+        t.inv_k = rsqrtf(xor16_32_sum(ss) + 1e-6f);
+        float dd = 0.f, kk = 0.f;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                t.K[i][r] *= t.inv_k;
+                t.Dl[i][r] = t.K[i][r] - V[i][r];
+                dd += t.Dl[i][r] * t.Dl[i][r];
+                kk += t.K[i][r] * t.K[i][r];
+            }
+        t.dn = sqrtf(xor16_32_sum(dd) + 1e-12f);
+        const float ksq = xor16_32_sum(kk);
+        const float amin = k.min_retention, mu = k.injection_margin, fac = k.spectral_factor;
+        const float ep = fminf(10.f, fmaxf(-10.f, pe_raw)), ap = fminf(10.f, fmaxf(-10.f, pa_raw));
+        const float eta = k.step_scale * logf(1.f + expf(ep));
+        const float sg = 1.f / (1.f + expf(-ap));
+        t.alpha = amin + (1.f - amin) * sg;
+        t.s_eta = fabsf(pe_raw) <= 10.f ? k.step_scale / (1.f + expf(-ep)) : 0.f;
+        t.s_alpha = fabsf(pa_raw) <= 10.f ? (1.f - amin) * sg * (1.f - sg) : 0.f;
+        t.denom = t.dn + 1e-6f;
+        t.cap = mu * (1.f - t.alpha) / t.denom;
+        const float u = eta / t.cap, e_neg = expf(-u);
+        t.eff = t.cap * (-expm1f(-u));
+        t.deff_deta = e_neg;
+        t.deff_dcap = softcap_dcap(u, e_neg);
+        t.deff_dalpha = 0.f;
+        t.deff_dksq = 0.f;
+        if (k.spectral_clamp) {
+            const float den = fmaxf(ksq, 1e-20f), lim = nextafterf(fac * t.alpha / den, 0.f);
+            if (t.eff > lim) {
+                t.eff = lim;
+                t.deff_deta = 0.f;
+                t.deff_dcap = 0.f;
+                t.deff_dalpha = fac / den;
+                if (ksq > 1e-20f) t.deff_dksq = -fac * t.alpha / (den * den);
+            }
+        }
+        if (!valid) {
+            t.eff = 0.f;
+            t.alpha = 1.f;
+        }
+        const Prefix la = time_prefix(log2f(t.alpha), c);
+        t.a = exp2f(la.total);
+        t.Da = exp2f(la.excl);
+        t.De = t.eff * exp2f(la.total - la.incl);
+        float(&sc)[5][16] = sh.sc[w];
+        sc[0][c] = t.eff;
+        sc[1][c] = la.incl;
+        sc[2][c] = la.excl;
+        sc[3][c] = t.De;
+        sc[4][c] = t.Da;
+        __builtin_amdgcn_wave_barrier();
+        const v4f eff_r = rows_of(sc[0]), incl_r = rows_of(sc[1]), excl_r = rows_of(sc[2]);
+        t.De_r = rows_of(sc[3]);
+        t.Da_r = rows_of(sc[4]);
+        __builtin_amdgcn_wave_barrier();
+        v4f gram = zero;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) gram = mm(t.K[i], t.K[i], gram);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool row_first = row_time(i) < tau;
+            const float m = (row_first ? eff_r[i] : t.eff) * exp2f(row_first ? la.excl - incl_r[i] : excl_r[i] - la.incl);
+            t.Mc[i] = row_time(i) == tau ? 0.f : m;
+            t.nC[i] = -t.Mc[i] * gram[i];
+        }
+        // Inverse of the 4 x 4 unit triangle of this slot's group of four times: this lane's
+        // entry is that of times min(g, f), max(g, f) of group c % 4, f = c / 4.
+        const int grp = c & 3, f = c >> 2;
+        float* dg = sh.diag[w];
+        dg[grp * 16 + 4 * g + f] = grp == 0 ? t.nC[0] : grp == 1 ? t.nC[1] : grp == 2 ? t.nC[2] : t.nC[3];
+        __builtin_amdgcn_wave_barrier();
+        const v4f r0 = *reinterpret_cast<const v4f*>(dg + grp * 16), r1 = *reinterpret_cast<const v4f*>(dg + grp * 16 + 4);
+        const v4f r2 = *reinterpret_cast<const v4f*>(dg + grp * 16 + 8);
+        __builtin_amdgcn_wave_barrier();
+        // r holds -L; (I - N)^-1 = I + N + N^2 + N^3 with N = -L
+        const float t02 = r0[2] + r0[1] * r1[2], t13 = r1[3] + r1[2] * r2[3];
+        const float t03 = r0[3] + r0[1] * t13 + r0[2] * r2[3];
+        const int lo = min(g, f), hi = max(g, f);
+        const float from0 = hi == 1 ? r0[1] : hi == 2 ? t02 : t03, from1 = hi == 2 ? r1[2] : t13;
+        const float inv = lo == 0 ? from0 : lo == 1 ? from1 : r2[3];
+        t.dl = g < f ? inv : 0.f;
+        t.du = f < g ? inv : 0.f;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            t.KT[i] = transpose(t.K[i]);
+            t.DlT[i] = transpose(t.Dl[i]);
+        }
+    }
+
+    __device__ __forceinline__ v4f diagonal(float v) const {   // v I as a tile
+        v4f r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = 4 * g + i == c ? v : 0.f;
+        return r;
+    }
+
+    // The block's maps into slot w of the segment's table: X, Y^T, and X^T for the adjoint.
+    template <bool ADJOINT>
+    __device__ __forceinline__ void store_maps(const Tokens<ND>& t) const {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        v4f S[ND], KD[ND];
+#pragma unroll
+        for (int j = 0; j < ND; ++j) {
+            S[j] = t.De_r * t.KT[j];
+            KD[j] = -(t.Da_r * t.KT[j]);
+        }
+        solve_upper(t, S);
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                const v4f start = i == j ? diagonal(t.a) : zero;
+                sh.maps[w][0][i * ND + j][lane] = mm(KD[i], S[j], start);
+                if constexpr (ADJOINT) sh.maps[w][1][i * ND + j][lane] = mm(S[i], KD[j], start);
+                sh.maps[w][2][i * ND + j][lane] = mm(-S[i], t.DlT[j], zero);
+            }
+    }
+    // G^T <- X^T G^T + Y^T of block b
+    __device__ __forceinline__ void apply_map(int b, v4f (&GT)[ND][ND]) const {
+        v4f out[ND][ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) out[i][j] = sh.maps[b][2][i * ND + j][lane];
+#pragma unroll
+        for (int m = 0; m < ND; ++m)
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const v4f x = sh.maps[b][0][m * ND + i][lane];
+#pragma unroll
+                for (int j = 0; j < ND; ++j) out[i][j] = mm(x, GT[m][j], out[i][j]);
+            }
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) GT[i][j] = out[i][j];
+    }
+    // H^T <- X H^T of block b
+    __device__ __forceinline__ void apply_adjoint(int b, v4f (&HT)[ND][ND]) const {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        v4f out[ND][ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) out[i][j] = zero;
+#pragma unroll
+        for (int m = 0; m < ND; ++m)
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const v4f x = sh.maps[b][1][m * ND + i][lane];
+#pragma unroll
+                for (int j = 0; j < ND; ++j) out[i][j] = mm(x, HT[m][j], out[i][j]);
+            }
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) HT[i][j] = out[i][j];
+    }
+};
+
+template <int ND>
+__device__ __forceinline__ void copy_tiles(const v4f (&from)[ND][ND], v4f (&to)[ND][ND]) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+        for (int j = 0; j < ND; ++j) to[i][j] = from[i][j];
+}
+
+template <int D, int W>
+__global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const BwdParams p) {
+    constexpr int ND = D / 16, NT = ND * ND, SD = 3 * D * D + 2 * D, DD = D * D;
+    using Tok = Tokens<ND>;
+    __shared__ Shared<D, W> sh;
+    const int w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int lane = static_cast<int>(threadIdx.x) & 63, g = lane >> 4, c = lane & 15;
+    const int tau = 4 * (c & 3) + (c >> 2);
+    const Line<D, W> L{sh, w, lane, g, c, tau, p.k};
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+
+    const int64_t ln = blockIdx.x;
+    const int64_t RH = p.R * p.heads, s = p.per_line ? ln : ln % RH;
+    const int r_dir = static_cast<int>((ln / p.heads) % p.R);
+    const int64_t b = ln / RH, head = ln % p.heads;
+    const int C = chunk_of(p.chunk, r_dir);
+    const int64_t N = p.N, nc = (N + C - 1) / C;
+    const int nb = (C + 15) / 16, nseg = (nb + W - 1) / W;
+    const int64_t xbase = ln * p.N * D;
+    const int64_t qbase = p.q_raw ? (b * p.R + r_dir) * p.N * (p.heads * D) + head * D : xbase;
+    const int64_t qstride = p.q_raw ? p.heads * D : D;
+    float* const my_gam = p.states + ln * p.nc * DD;
+    float* const my_seg = p.gtraj + (ln * W + w) * static_cast<int64_t>(p.segs) * DD;
+
+    // ---- memories into LDS -------------------------------------------------------------
+    for (int t = w; t < 5 * NT; t += W) {
+        const int m = t / NT, i = (t % NT) / ND, j = t % ND;
+        const float* src = p.m0[m == 0 || m == 2 ? 2 : m == 4 ? 0 : 1] + s * DD;
+        v4f v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)   // N(M^T): column 16 j + c of the tile is row 16 j + c of M
+            v[r] = m < 2 ? src[(16 * j + c) * D + 16 * i + 4 * g + r] : src[(16 * i + 4 * g + r) * D + 16 * j + c];
+        sh.mem[m][t % NT][lane] = v;
+    }
+    if (threadIdx.x < 2 * D)
+        sh.ev[threadIdx.x / D][threadIdx.x % D] = p.m0[3 + threadIdx.x / D][s * D + threadIdx.x % D];
+    __syncthreads();
+
+    auto load_x = [&](int64_t ch, int blk, bool& valid, v4f (&X)[ND]) {
+        const int tl = 16 * blk + tau;
+        const int64_t t = ch * C + tl;
+        valid = tl < C && t < N;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            X[i] = zero;
+            if (valid) X[i] = load_io4(p.x, xbase + t * D + 16 * i + 4 * g, p.io_dtype);
+        }
+    };
+    auto identity = [&](v4f (&M)[ND][ND]) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) M[i][j] = i == j ? L.diagonal(1.f) : zero;
+    };
+    // R^T from K^T G^T of the block's entry gain (R (I + L) = G K D_a + Delta).
+    auto solve_r = [&](const Tok& t, const v4f (&KG)[ND], v4f (&RT)[ND]) {
+#pragma unroll
+        for (int j = 0; j < ND; ++j) RT[j] = t.Da_r * KG[j] + t.DlT[j];
+        L.solve_lower(t, RT);
+    };
+
+    // ---- 1. forward: Gamma before every chunk ------------------------------------------
+    v4f GamT[ND][ND];
+    identity(GamT);
+    for (int64_t ch = 0; ch < nc - 1; ++ch) {
+        v4f G[ND][ND];
+        if constexpr (W == 1) {
+            v4f X[ND], RT[ND];
+            bool valid;
+            Tok t;
+            load_x(ch, 0, valid, X);
+            L.tokens(X, valid, GamT, t);
+            solve_r(t, t.KT, RT);
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j)
+                    G[i][j] = mm(-RT[i], t.De_r * t.KT[j], i == j ? L.diagonal(t.a) : zero);
+        } else {
+            v4f GT[ND][ND];
+            identity(GT);
+            for (int seg = 0; seg < nseg; ++seg) {
+                const int nbs = min(W, nb - seg * W);
+                if (w < nbs) {
+                    v4f X[ND];
+                    bool valid;
+                    Tok t;
+                    load_x(ch, seg * W + w, valid, X);
+                    L.tokens(X, valid, GamT, t);
+                    L.template store_maps<false>(t);
+                }
+                __syncthreads();
+                for (int blk = 0; blk < nbs; ++blk) L.apply_map(blk, GT);
+                __syncthreads();
+            }
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) G[i][j] = L.transpose(GT[j][i]);
+        }
+        // Gamma^T <- G^T Gamma^T
+        v4f next[ND][ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                next[i][j] = zero;
+#pragma unroll
+                for (int m = 0; m < ND; ++m) next[i][j] = mm(G[m][i], GamT[m][j], next[i][j]);
+            }
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                GamT[i][j] = next[i][j];
+                // row 16 j + c of Gamma, columns 16 i + 4 g ..
+                if ((i * ND + j) % W == w)
+                    *reinterpret_cast<v4f_any*>(my_gam + (ch + 1) * DD + (16 * j + c) * D + 16 * i +
+                                            4 * g) = next[i][j];
+            }
+    }
+    __syncthreads();   // Gamma of every chunk is written (each wave reads all of it below)
+
+    // ---- 2. chunks in reverse ----------------------------------------------------------
+    v4f dMm[ND][ND], dMv[ND][ND], dMk[ND][ND], dEv[ND], dAv[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        dEv[i] = dAv[i] = zero;
+#pragma unroll
+        for (int j = 0; j < ND; ++j) dMm[i][j] = dMv[i][j] = dMk[i][j] = zero;
+    }
+    for (int64_t ch = nc - 1; ch >= 0; --ch) {
+        v4f Gam[ND][ND];
+        if (ch == 0) {
+            identity(GamT);
+            identity(Gam);
+        } else {
+            const float* src = my_gam + ch * DD;
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) {
+                    GamT[i][j] = *reinterpret_cast<const v4f_any*>(src + (16 * j + c) * D + 16 * i + 4 * g);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) Gam[i][j][r] = src[(16 * i + 4 * g + r) * D + 16 * j + c];
+                }
+        }
+        v4f Ep[ND][ND], EG[ND][ND];   // this wave's part of dGamma_c; its tiles of dGamma_{c+1} G_C^T
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j) Ep[i][j] = EG[i][j] = zero;
+
+        // Gradients of this wave's block (chunk block blk) from the adjoint H of its exit
+        // gain; GTb: the transposed gain at its start (the identity when W is 1).
+        auto block_gradients = [&](int blk, const Tok& t, const v4f (&X)[ND], bool valid, const v4f (&RT)[ND],
+                                   const v4f (&KG)[ND], const v4f (&GTb)[ND][ND], const v4f (&HT)[ND][ND],
+                                   const v4f (&H)[ND][ND]) {
+            v4f RbT[ND], R[ND], Rb[ND];
+            float part = 0.f, hg = 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                v4f kh = zero;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) {
+                    kh = mm(t.K[i], HT[i][j], kh);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if constexpr (W > 1) hg += HT[i][j][r] * GTb[i][j][r];
+                        else if (i == j) hg += 4 * g + r == c ? HT[i][j][r] : 0.f;
+                    }
+                }
+                RbT[j] = -(t.De_r * kh);
+            }
+            L.solve_upper(t, RbT);
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) part += RbT[j][r] * (t.Da_r[r] * KG[j][r]);
+            const float phi0 = wave_sum(part + t.a * hg);   // <H, G> at the block start
+            float rr = 0.f, rd = 0.f;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                R[i] = L.transpose(RT[i]);
+                Rb[i] = L.transpose(RbT[i]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    rr += Rb[i][r] * R[i][r];
+                    rd += Rb[i][r] * t.Dl[i][r];
+                }
+            }
+            rr = xor16_32_sum(rr);
+            rd = xor16_32_sum(rd);
+            const float phi = phi0 + time_prefix(rd, c).incl;
+            const float d_eff = t.eff > 0.f ? rr / t.eff : 0.f;
+            const float d_cap = d_eff * t.deff_dcap;
+            const float d_alpha = (phi - rr) / t.alpha + d_cap * (-p.k.injection_margin / t.denom) + d_eff * t.deff_dalpha;
+            const float d_apre = valid ? d_alpha * t.s_alpha : 0.f;
+            const float d_epre = d_eff * t.deff_deta * t.s_eta;
+            const float cdn = d_cap * (-t.cap / t.denom) / t.dn, cks = 2.f * d_eff * t.deff_dksq;
+            v4f P = zero, PT = zero, Ws;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                P = mm(R[i], Rb[i], P);
+                PT = mm(Rb[i], R[i], PT);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Ws[r] = t.Mc[r] * (L.row_time(r) < tau ? P[r] : PT[r]);
+            v4f dk[ND], dv[ND], ZT[ND];
+            float kdot = 0.f;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                v4f hr = zero, gr = zero;
+#pragma unroll
+                for (int m = 0; m < ND; ++m) {
+                    hr = mm(H[m][i], R[m], hr);
+                    if constexpr (W > 1) gr = mm(L.transpose(GTb[i][m]), Rb[m], gr);
+                }
+                if constexpr (W == 1) gr = Rb[i];
+                const v4f kw = mm(t.KT[i], Ws, zero);
+                dk[i] = gr * t.Da - hr * t.De - kw + Rb[i] + t.Dl[i] * cdn + t.K[i] * cks;
+                dv[i] = -Rb[i] - t.Dl[i] * cdn;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) kdot += dk[i][r] * t.K[i][r];
+            }
+            kdot = xor16_32_sum(kdot);
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                dk[i] = (dk[i] - t.K[i] * kdot) * t.inv_k;
+                dEv[i] += t.Z[i] * d_epre;
+                dAv[i] += t.Z[i] * d_apre;
+                ZT[i] = L.transpose(t.Z[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const v4f dvT = L.transpose(dv[i]), dkT = L.transpose(dk[i]);
+#pragma unroll
+                for (int j = 0; j < ND; ++j) {
+                    dMv[i][j] = mm(dvT, ZT[j], dMv[i][j]);
+                    dMk[i][j] = mm(dkT, ZT[j], dMk[i][j]);
+                }
+            }
+            v4f dz[ND], XT[ND];
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                dz[j] = L.rows_of(&sh.ev[0][16 * j]) * d_epre + L.rows_of(&sh.ev[1][16 * j]) * d_apre;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) {
+                    dz[j] = mm(sh.mem[3][i * ND + j][lane], dv[i], dz[j]);
+                    dz[j] = mm(sh.mem[2][i * ND + j][lane], dk[i], dz[j]);
+                }
+                XT[j] = L.transpose(X[j]);
+            }
+            const int64_t at = xbase + (ch * C + 16 * blk + tau) * D + 4 * g;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                v4f dx = zero;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) dx = mm(Gam[i][j], dz[i], dx);
+                if (valid) *reinterpret_cast<v4f_any*>(p.dx + at + 16 * j) = dx;
+                const v4f dzT = L.transpose(dz[j]);
+#pragma unroll
+                for (int i = 0; i < ND; ++i) Ep[j][i] = mm(dzT, XT[i], Ep[j][i]);
+            }
+        };
+
+        if (ch < nc - 1) {
+            Tok t;
+            v4f X[ND], RT[ND], GT[ND][ND], HT[ND][ND], H[ND][ND];
+            v4f GTb[ND][ND];   // G^T at the start of this wave's block of the segment
+            bool valid = false;
+            if constexpr (W == 1) {
+                load_x(ch, 0, valid, X);
+                L.tokens(X, valid, GamT, t);
+                solve_r(t, t.KT, RT);
+#pragma unroll
+                for (int i = 0; i < ND; ++i)
+#pragma unroll
+                    for (int j = 0; j < ND; ++j)
+                        GT[i][j] = mm(t.De_r * t.KT[i], -RT[j], i == j ? L.diagonal(t.a) : zero);
+            } else {
+                identity(GT);
+                for (int seg = 0; seg < nseg; ++seg) {
+                    const int nbs = min(W, nb - seg * W);
+                    if (nseg > 1)
+#pragma unroll
+                        for (int i = 0; i < NT; ++i)
+                            *reinterpret_cast<v4f_any*>(my_seg + seg * DD + i * 256 + 4 * lane) = GT[i / ND][i % ND];
+                    if (seg > 0) __syncthreads();   // every wave has read the previous segment's maps
+                    if (w < nbs) {
+                        load_x(ch, seg * W + w, valid, X);
+                        L.tokens(X, valid, GamT, t);
+                        L.template store_maps<true>(t);
+                    }
+                    __syncthreads();
+                    for (int blk = 0; blk < nbs; ++blk) {
+                        if (blk == w) copy_tiles(GT, GTb);
+                        L.apply_map(blk, GT);
+                    }
+                }
+            }
+            // dGamma_{c+1} G_C^T and the adjoint of the chunk gain, dG_C = Gamma^T dGamma_{c+1}
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) HT[i][j] = H[i][j] = zero;
+#pragma unroll
+            for (int m = 0; m < ND; ++m)
+#pragma unroll
+                for (int i = 0; i < ND; ++i) {
+                    v4f e;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) e[r] = sh.E[16 * m + 4 * g + r][16 * i + c];
+                    const v4f et = *reinterpret_cast<const v4f*>(&sh.E[16 * i + c][16 * m + 4 * g]);
+#pragma unroll
+                    for (int j = 0; j < ND; ++j) {
+                        HT[i][j] = mm(e, Gam[m][j], HT[i][j]);
+                        if constexpr (W == 1) H[j][i] = mm(Gam[m][j], e, H[j][i]);
+                        if ((i * ND + j) % W == w) EG[i][j] = mm(et, GT[m][j], EG[i][j]);
+                    }
+                }
+            if constexpr (W == 1) {
+                block_gradients(0, t, X, valid, RT, t.KT, GT, HT, H);
+            } else {
+                for (int seg = nseg - 1; seg >= 0; --seg) {
+                    const int nbs = min(W, nb - seg * W);
+                    if (seg != nseg - 1) {
+#pragma unroll
+                        for (int i = 0; i < NT; ++i)
+                            GTb[i / ND][i % ND] = *reinterpret_cast<const v4f_any*>(my_seg + seg * DD + i * 256 + 4 * lane);
+                        __syncthreads();   // every wave has read the later segment's maps
+                        if (w < nbs) {
+                            load_x(ch, seg * W + w, valid, X);
+                            L.tokens(X, valid, GamT, t);
+                            L.template store_maps<true>(t);
+                        }
+                        __syncthreads();
+                        for (int blk = 0; blk < w; ++blk) L.apply_map(blk, GTb);   // a segment with a successor is full
+                    }
+                    // H^T from the segment's exit to this block's exit (and on to the segment's
+                    // start when an earlier segment continues from there)
+                    v4f HTb[ND][ND];
+                    for (int blk = nbs - 1; blk >= 0; --blk) {
+                        if (blk == w) copy_tiles(HT, HTb);
+                        if (seg == 0 && blk <= w) break;
+                        L.apply_adjoint(blk, HT);
+                    }
+                    if (w < nbs) {
+#pragma unroll
+                        for (int i = 0; i < ND; ++i)
+#pragma unroll
+                            for (int j = 0; j < ND; ++j) H[i][j] = L.transpose(HTb[j][i]);
+                        v4f KG[ND];
+#pragma unroll
+                        for (int j = 0; j < ND; ++j) {
+                            KG[j] = zero;
+#pragma unroll
+                            for (int i = 0; i < ND; ++i) KG[j] = mm(t.K[i], GTb[i][j], KG[j]);
+                        }
+                        solve_r(t, KG, RT);
+                        block_gradients(seg * W + w, t, X, valid, RT, KG, GTb, HTb, H);
+                    }
+                }
+            }
+        }
+
+        // Readout: y = M_m Gamma q^ of every token of the chunk.
+        for (int blk = w; blk < nb; blk += W) {
+            const int tl = 16 * blk + tau;
+            const int64_t tok = ch * C + tl;
+            const bool valid = tl < C && tok < N;
+            const int64_t at = xbase + tok * D + 4 * g, qat = qbase + tok * qstride + 4 * g;
+            v4f q[ND], dy[ND];
+            float qq = 0.f;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                q[i] = dy[i] = zero;
+                if (valid) {
+                    q[i] = load_io4(p.q, qat + 16 * i, p.q_raw ? p.io_dtype : VH_DTYPE_F32);
+                    dy[i] = *reinterpret_cast<const v4f_any*>(p.dy + at + 16 * i);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) qq += q[i][r] * q[i][r];
+            }
+            float qinv = 1.f;
+            if (p.q_raw) qinv = 1.f / fmaxf(sqrtf(xor16_32_sum(qq)), 1e-12f);
+            v4f dp[ND], qT[ND], dpT[ND];
+#pragma unroll
+            for (int i = 0; i < ND; ++i) q[i] *= qinv;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                dp[j] = zero;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) dp[j] = mm(sh.mem[4][i * ND + j][lane], dy[i], dp[j]);
+                qT[j] = L.transpose(q[j]);
+                dpT[j] = L.transpose(dp[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                v4f pT = zero;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) pT = mm(q[i], GamT[i][j], pT);
+#pragma unroll
+                for (int i = 0; i < ND; ++i) {
+                    dMm[i][j] = mm(L.transpose(dy[i]), pT, dMm[i][j]);
+                    Ep[i][j] = mm(dpT[i], qT[j], Ep[i][j]);
+                }
+            }
+            v4f dq[ND];
+            float qdot = 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                dq[j] = zero;
+#pragma unroll
+                for (int i = 0; i < ND; ++i) dq[j] = mm(Gam[i][j], dp[i], dq[j]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) qdot += dq[j][r] * q[j][r];
+            }
+            qdot = xor16_32_sum(qdot);
+#pragma unroll
+            for (int j = 0; j < ND; ++j) {
+                if (p.q_raw) dq[j] = (qinv > 9.999e11f ? dq[j] : dq[j] - q[j] * qdot) * qinv;
+                if (valid) {
+                    *reinterpret_cast<v4f_any*>(p.dq + qat + 16 * j) = dq[j];
+                    // the last chunk's x reaches no output
+                    if (ch == nc - 1) *reinterpret_cast<v4f_any*>(p.dx + at + 16 * j) = zero;
+                }
+            }
+        }
+
+        // dGamma_c: the waves' parts and dGamma_{c+1} G_C^T, in wave order.
+        if constexpr (W > 1) {
+            __syncthreads();   // every wave has read the maps and dGamma_{c+1}
+#pragma unroll
+            for (int i = 0; i < NT; ++i) sh.maps[w][0][i][lane] = Ep[i / ND][i % ND];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+                if ((i * ND + j) % W == w) {
+                    v4f e = EG[i][j];
+                    if constexpr (W == 1) e += Ep[i][j];
+                    else
+                        for (int v = 0; v < W; ++v) e += sh.maps[v][0][i * ND + j][lane];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sh.E[16 * i + 4 * g + r][16 * j + c] = e[r];
+                }
+        __syncthreads();
+    }
+
+    // ---- 3. the line's gradient of its initial memories ----------------------------------
+    float* const dst = p.dline + ln * SD;
+    auto store_matrix = [&](int m, const v4f (&M)[ND][ND]) {
+        if constexpr (W > 1) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) sh.maps[w][0][i][lane] = M[i / ND][i % ND];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+            if (i % W == w) {
+                v4f e = M[i / ND][i % ND];
+                if constexpr (W > 1) {
+                    e = zero;
+                    for (int v = 0; v < W; ++v) e += sh.maps[v][0][i][lane];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[m * DD + (16 * (i / ND) + 4 * g + r) * D + 16 * (i % ND) + c] = e[r];
+            }
+        if constexpr (W > 1) __syncthreads();
+    };
+    store_matrix(0, dMm);
+    store_matrix(1, dMv);
+    store_matrix(2, dMk);
+    // gate vectors: the 16 slot columns, then the waves (through the transpose scratch)
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float e = row_group_sum<16>(dEv[i][r]), a = row_group_sum<16>(dAv[i][r]);
+            sh.tr[w][16 * i + 4 * g + r] = e;
+            sh.tr[w][D + 16 * i + 4 * g + r] = a;
+        }
+    __syncthreads();
+    if (threadIdx.x < 2 * D) {
+        float v = 0.f;
+        for (int u = 0; u < W; ++u) v += sh.tr[u][threadIdx.x];
+        dst[3 * DD + threadIdx.x] = v;
+    }
+}
+
+}  // namespace
+
+// Waves per line: one 16-token block each, up to 8 (4 at d = 32, where a wave's registers
+// and the map table are four times as large); longer chunks run in segments.
+int bwd_block_waves(int head_dim, int64_t max_chunk) {
+    const int most = head_dim == 16 ? 8 : 4;
+    int w = 1;
+    while (w < most && 16 * w < max_chunk) w *= 2;
+    return w;
+}
+
+int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream) {
+    auto go = [&](auto d, auto w) {
+        constexpr int D = decltype(d)::value, W = decltype(w)::value;
+        hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W>), dim3(static_cast<unsigned>(lines)), dim3(64 * W), 0,
+                           stream, p);
+    };
+    auto by_waves = [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        switch (waves) {
+            case 1: go(d, std::integral_constant<int, 1>{}); break;
+            case 2: go(d, std::integral_constant<int, 2>{}); break;
+            case 4: go(d, std::integral_constant<int, 4>{}); break;
+            default:
+                if constexpr (D == 16) go(d, std::integral_constant<int, 8>{});
+                break;
+        }
+    };
+    if (head_dim == 16) by_waves(std::integral_constant<int, 16>{});
+    else by_waves(std::integral_constant<int, 32>{});
+    return check_launch("srnl_backward_blocks_kernel");
+}
+
+}  // namespace vh
