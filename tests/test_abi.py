@@ -318,6 +318,30 @@ def test_srnl_backward_validates_directions_and_constants(lib):
     assert _spatial(lib, consts=bad_margin) == hip.VH_ERR_ARG
 
 
+def test_srnl_spatial_backward_validates(lib):
+    """The spatial backward takes head_dim 16 and 32, chunks of 1 to 256, and a workspace of
+    the size it reports (0 for what it does not take)."""
+    p = ctypes.c_void_p(0x1000)
+
+    def call(head_dim=16, chunk=4, C=32, H=4, dtype=hip.VH_DTYPE_F32, nbytes=None, x=p):
+        arr, keep = hip.int64_array([chunk] * 4)
+        size = lib.vh_srnl_spatial_backward_workspace_bytes(1, H, 4, C, head_dim, dtype, arr)
+        rc = lib.vh_srnl_spatial_backward(x, p, dtype, p, p, p, p, p, p, p, 0, p, p, p, p, p, p, p, p, p, p,
+                                          1, H, 4, C, head_dim, arr, _consts(), p,
+                                          size if nbytes is None else nbytes, None)
+        return size, rc
+
+    assert call(head_dim=8) == (0, hip.VH_ERR_HEAD_DIM)
+    assert call(head_dim=64, C=64) == (0, hip.VH_ERR_HEAD_DIM)
+    assert call(chunk=257) == (0, hip.VH_ERR_ARG)
+    assert call(chunk=0) == (0, hip.VH_ERR_ARG)
+    assert call(C=40) == (0, hip.VH_ERR_SHAPE)
+    assert call(H=0) == (0, hip.VH_ERR_SHAPE)
+    assert call(dtype=9) == (0, hip.VH_ERR_DTYPE)
+    assert call(x=None)[1] == hip.VH_ERR_ARG
+    assert call(nbytes=64)[0] > 64 and call(nbytes=64)[1] == hip.VH_ERR_WORKSPACE
+
+
 def test_dispatch_overrides_are_validated(lib):
     """Kernel choices are forced only through vh_set_dispatch_override, which rejects unknown
     names and malformed values; nothing is read from the environment."""

@@ -27,6 +27,14 @@ struct BwdParams {
     int io_dtype, q_raw;
     int chunk[4];
     vh_srnl_consts k;
+    // Spatial form (block form only): x, q, dy are channels-last maps [B, H, W, heads * D]
+    // (x and q io dtype, dy the FP32 gradient of the fused output), R = 4 scan orders; dx and
+    // dq become four planes of such maps in the io dtype, one per direction, and the M_m part
+    // of dline the gradient for unit direction weights.
+    const float* scale;   // [4, heads * D] direction weights; null: packed lines
+    int64_t H, W;
+    float inv_h;
+    void *dx_planes, *dq_planes;
 };
 
 // d(eta^)/d(cap) of eta^ = cap (1 - exp(-u)), u = eta / cap: (1 - e^-u) - u e^-u, by its

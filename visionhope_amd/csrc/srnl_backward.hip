@@ -47,9 +47,9 @@ __device__ __forceinline__ float dpp_f(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
-// Sum over the D-lane group of this lane, on the VALU (DPP and the gfx950 row swap; no LDS
-// round trip).  Every step adds lane pairs that exchange values (row mirror, half-row
-// mirror, quad xor 1 and 2, row xor), so all lanes of a group end with the same bits.
+// Sum over the D-lane group of this lane, on the VALU (DPP; no LDS round trip).  Every step
+// adds lane pairs that exchange values (half-row mirror, quad xor 1 and 2), so all lanes of
+// a group end with the same bits.
 template <int D>
 __device__ __forceinline__ float group_sum(float v) {
     static_assert(D == 4 || D == 8, "group of 4 or 8 lanes");
@@ -434,22 +434,175 @@ __global__ __launch_bounds__(D * LPW) void srnl_backward_kernel(const BwdParams 
     }
 }
 
-// dM[s] = sum over b of the per-line gradients of lines b * S + s, in b order.
+// dM[s] = sum over b of the per-line gradients of lines b * S + s.  A workgroup takes 32
+// consecutive values of one state and 8 interleaved parts of the batch (each in b order),
+// then adds the parts in order: deterministic, and 8 times the loads in flight of one thread
+// per value (4,096 lines, 32 states of 800 values: 35 us with one thread per value, 4.7 us so).
 __global__ __launch_bounds__(256) void srnl_backward_reduce_kernel(const float* dline, int64_t batch, int64_t S,
                                                                    int d, float* dmm, float* dmv, float* dmk,
                                                                    float* dme, float* dma) {
+    __shared__ float parts[8][32];
     const int64_t SD = 3 * d * d + 2 * d;
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= S * SD) return;
-    const int64_t s = idx / SD, e = idx % SD;
+    const int lane = static_cast<int>(threadIdx.x) & 31, part = static_cast<int>(threadIdx.x) >> 5;
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * 32 + lane;
+    const bool live = idx < S * SD;
+    const int64_t s = live ? idx / SD : 0, e = live ? idx % SD : 0;
     float acc = 0.f;
-    for (int64_t b = 0; b < batch; ++b) acc += dline[(b * S + s) * SD + e];
+    if (live) {
+#pragma unroll 4
+        for (int64_t b = part; b < batch; b += 8) acc += dline[(b * S + s) * SD + e];
+    }
+    parts[part][lane] = acc;
+    __syncthreads();
+    if (part != 0 || !live) return;
+#pragma unroll
+    for (int p = 1; p < 8; ++p) acc += parts[p][lane];
     const int64_t dd = static_cast<int64_t>(d) * d;
     if (e < dd) dmm[s * dd + e] = acc;
     else if (e < 2 * dd) dmv[s * dd + e - dd] = acc;
     else if (e < 3 * dd) dmk[s * dd + e - 2 * dd] = acc;
     else if (e < 3 * dd + d) dme[s * d + e - 3 * dd] = acc;
     else dma[s * d + e - 3 * dd - d] = acc;
+}
+
+typedef float f8_any __attribute__((ext_vector_type(8), aligned(4)));
+typedef unsigned short us8_any __attribute__((ext_vector_type(8), aligned(2)));
+
+// Eight consecutive elements of a map row that may start at any element.
+template <typename T>
+__device__ __forceinline__ void load8_any(const void* p, int64_t i, float (&v)[8]) {
+    if constexpr (sizeof(T) == 4) {
+        const f8_any r = *reinterpret_cast<const f8_any*>(static_cast<const float*>(p) + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = r[j];
+    } else {
+        const us8_any r = *reinterpret_cast<const us8_any*>(static_cast<const uint16_t*>(p) + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = to_f32(T{r[j]});
+    }
+}
+template <typename T>
+__device__ __forceinline__ void store8_any(void* p, int64_t i, const float (&v)[8]) {
+    if constexpr (sizeof(T) == 4) {
+        f8_any r;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[j] = v[j];
+        *reinterpret_cast<f8_any*>(static_cast<float*>(p) + i) = r;
+    } else {
+        us8_any r;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[j] = from_f32<T>(v[j]).bits;
+        *reinterpret_cast<us8_any*>(static_cast<uint16_t*>(p) + i) = r;
+    }
+}
+
+struct MergeParams {
+    const void *dx_planes, *dq_planes, *x;
+    const float *dout, *skip, *scale;   // skip [C] or [4, C], scale [4, C]
+    int skip_per_direction;
+    void *dx, *dq;
+    float* part;                        // [gridDim.x, C]: sums of dout x over a workgroup's pixels
+    int64_t pixels, C;
+    int groups;                         // channel groups of 8 per workgroup
+};
+
+// The spatial backward's sum over the directions: dx = sum_r dx_r + dout sum_r s_r k_r,
+// dq = sum_r dq_r, and the per-channel sums of dout x that the gradients of the skip and of
+// the direction weights need.  One thread per 8 channels of a pixel, pixels strided over the
+// grid.  Bound by HBM: 8 planes, dout and x in, dx and dq out: 83 MB at B = 128, 14 x 14 x 128,
+// bf16, in 15 us (5.4 TB/s; a plain copy reaches 5.2).  With the spatial addressing of the
+// block-form kernel it replaces the fusion backward (164 us), four flips, the restoring and
+// converting copies and the sums of the four scan orders (about 250 us) of that step.
+template <typename T>
+__global__ __launch_bounds__(256) void srnl_backward_merge_kernel(const MergeParams p) {
+    __shared__ float red[256][9];
+    const int rows = 256 / p.groups, row = static_cast<int>(threadIdx.x) / p.groups;
+    const int64_t c0 = (static_cast<int64_t>(blockIdx.y) * p.groups + threadIdx.x % p.groups) * 8;
+    const int64_t plane = p.pixels * p.C;
+    float sums[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sums[j] = 0.f;
+    if (row < rows && c0 < p.C) {
+        float through[8];   // sum_r s_r k_r
+#pragma unroll
+        for (int j = 0; j < 8; ++j) through[j] = 0.f;
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                through[j] += p.scale[r * p.C + c0 + j] * p.skip[(p.skip_per_direction ? r * p.C : 0) + c0 + j];
+        for (int64_t i = static_cast<int64_t>(blockIdx.x) * rows + row; i < p.pixels;
+             i += static_cast<int64_t>(gridDim.x) * rows) {
+            const int64_t at = i * p.C + c0;
+            float g[8], x[8], a[8], b[8], dx[8], dq[8];
+            load8_any<float>(p.dout, at, g);
+            load8_any<T>(p.x, at, x);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                dx[j] = g[j] * through[j];
+                dq[j] = 0.f;
+                sums[j] += g[j] * x[j];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                load8_any<T>(p.dx_planes, r * plane + at, a);
+                load8_any<T>(p.dq_planes, r * plane + at, b);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    dx[j] += a[j];
+                    dq[j] += b[j];
+                }
+            }
+            store8_any<T>(p.dx, at, dx);
+            store8_any<T>(p.dq, at, dq);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) red[threadIdx.x][j] = sums[j];
+    __syncthreads();
+    if (row == 0 && c0 < p.C) {
+        for (int k = 1; k < rows; ++k)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sums[j] += red[threadIdx.x + k * p.groups][j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p.part[blockIdx.x * p.C + c0 + j] = sums[j];
+    }
+}
+
+// Gradients of the skip and the direction weights of channel c = blockIdx.x, from
+// sgx = sum dout x (parts of the workgroups above) and U = the gradient of M_m for unit
+// weights: sum dout y_r = M_m . U row by row, so
+//   d scale[r, c] = M_m[r, c, :] . U[r, c, :] + k_r[c] sgx, d skip = s_r[c] sgx (summed over r
+// when shared); U is scaled to the gradient of M_m in place.
+__global__ __launch_bounds__(256) void srnl_backward_params_kernel(const float* part, int64_t parts, int64_t C, int d,
+                                                                  const float* Mm, float* dMm, const float* skip,
+                                                                  int skip_per_direction, const float* scale,
+                                                                  float* dskip, float* dscale) {
+    __shared__ float red[256];
+    const int64_t c = blockIdx.x;
+    float acc = 0.f;
+    for (int64_t i = threadIdx.x; i < parts; i += 256) acc += part[i * C + c];
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    for (int n = 128; n > 0; n >>= 1) {
+        if (static_cast<int>(threadIdx.x) < n) red[threadIdx.x] += red[threadIdx.x + n];
+        __syncthreads();
+    }
+    const float sgx = red[0];
+    if (threadIdx.x < 4) {
+        const int r = static_cast<int>(threadIdx.x);
+        const int64_t at = r * C + c;
+        const float s = scale[at], k = skip[skip_per_direction ? at : c];
+        float dot = 0.f;
+        for (int j = 0; j < d; ++j) {   // row c % d of head c / d of direction r
+            const float u = dMm[at * d + j];
+            dot += Mm[at * d + j] * u;
+            dMm[at * d + j] = s * u;
+        }
+        dscale[at] = dot + k * sgx;
+        if (skip_per_direction) dskip[at] = s * sgx;
+    }
+    if (threadIdx.x == 0 && !skip_per_direction)
+        dskip[c] = (scale[c] + scale[C + c]) * sgx + (scale[2 * C + c] + scale[3 * C + c]) * sgx;
 }
 
 namespace {
@@ -482,6 +635,43 @@ BwdLayout bwd_layout(int64_t B, int64_t R, int64_t heads, int64_t N, int d, cons
     l.dline = round(static_cast<size_t>(l.lines * l.sd));
     l.total = (l.states + l.traj + l.dline) * sizeof(float);
     return l;
+}
+
+struct SpatialBwdLayout {
+    BwdLayout lines;
+    int groups;        // channel groups of 8 per merge workgroup
+    int64_t blocks;    // merge workgroups over the pixels
+    size_t dx_planes, dq_planes, parts, total;   // byte offsets
+};
+
+SpatialBwdLayout spatial_bwd_layout(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim, int32_t io_dtype,
+                                    const int64_t* chunks) {
+    SpatialBwdLayout l{};
+    if (B <= 0 || H <= 0 || W <= 0 || C <= 0 || chunks == nullptr || (head_dim != 16 && head_dim != 32) ||
+        C % head_dim != 0)
+        return l;
+    for (int r = 0; r < 4; ++r)
+        if (chunks[r] <= 0 || chunks[r] > kBwdLongChunk) return l;
+    l.lines = bwd_layout(B, 4, C / head_dim, H * W, head_dim, chunks);
+    l.groups = static_cast<int>(std::min<int64_t>(C / 8, 256));
+    const int64_t rows = 256 / l.groups, pixels = B * H * W;
+    // about four pixels per thread, at most four workgroups per CU
+    l.blocks = std::max<int64_t>(1, std::min<int64_t>(1024, (pixels + 4 * rows - 1) / (4 * rows)));
+    auto round = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t plane = round(static_cast<size_t>(4 * pixels * C) * (io_dtype == VH_DTYPE_F32 ? 4 : 2));
+    l.dx_planes = round(l.lines.total);
+    l.dq_planes = l.dx_planes + plane;
+    l.parts = l.dq_planes + plane;
+    l.total = l.parts + round(static_cast<size_t>(l.blocks * C) * sizeof(float));
+    return l;
+}
+
+int launch_backward_reduce(const float* dline, int64_t batch, int64_t S, int32_t head_dim, float* dM_m, float* dM_v,
+                           float* dM_k, float* dM_eta, float* dM_alpha, hipStream_t s) {
+    const int64_t total = S * (3 * head_dim * head_dim + 2 * head_dim);
+    hipLaunchKernelGGL(srnl_backward_reduce_kernel, dim3(static_cast<unsigned>((total + 31) / 32)), dim3(256), 0, s,
+                       dline, batch, S, head_dim, dM_m, dM_v, dM_k, dM_eta, dM_alpha);
+    return check_launch("srnl_backward_reduce_kernel");
 }
 
 }  // namespace
@@ -586,10 +776,83 @@ int vh_srnl_backward(const void* x, const void* q, int32_t io_dtype, int32_t q_r
     if (rc) return rc;
     // Shared states: sum the B lines of each; one state per line: copy.
     const int64_t S = memories_per_line ? lay.lines : R * heads, batch = memories_per_line ? 1 : B;
-    const int64_t total = S * lay.sd;
-    hipLaunchKernelGGL(srnl_backward_reduce_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s,
-                       bp.dline, batch, S, head_dim, dM_m, dM_v, dM_k, dM_eta, dM_alpha);
-    return check_launch("srnl_backward_reduce_kernel");
+    return launch_backward_reduce(bp.dline, batch, S, head_dim, dM_m, dM_v, dM_k, dM_eta, dM_alpha, s);
+}
+
+size_t vh_srnl_spatial_backward_workspace_bytes(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim,
+                                                int32_t io_dtype, const int64_t* chunks) {
+    if (!valid_dtype(io_dtype)) return 0;
+    return spatial_bwd_layout(B, H, W, C, head_dim, io_dtype, chunks).total;
+}
+
+int vh_srnl_spatial_backward(const void* x, const void* q, int32_t io_dtype, const float* dout, const float* M_m,
+                             const float* M_v, const float* M_k, const float* M_eta, const float* M_alpha,
+                             const float* d_skip, int32_t skip_per_direction, const float* dir_weight, void* dx,
+                             void* dq, float* dM_m, float* dM_v, float* dM_k, float* dM_eta, float* dM_alpha,
+                             float* dd_skip, float* ddir_weight, int64_t B, int64_t H, int64_t W, int64_t C,
+                             int32_t head_dim, const int64_t chunks[4], const vh_srnl_consts* consts, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+    VH_REQUIRE(x && q && dout && M_m && M_v && M_k && M_eta && M_alpha && d_skip && dir_weight && dx && dq && dM_m &&
+                   dM_v && dM_k && dM_eta && dM_alpha && dd_skip && ddir_weight && chunks && consts,
+               VH_ERR_ARG, "spatial SRNL backward pointers must not be null");
+    VH_REQUIRE(B > 0 && H > 0 && W > 0 && C > 0, VH_ERR_SHAPE, "spatial SRNL backward needs nonempty [B, H, W, C]");
+    {
+        const int rc = check_srnl_consts(consts);
+        if (rc) return rc;
+    }
+    VH_REQUIRE(head_dim == 16 || head_dim == 32, VH_ERR_HEAD_DIM,
+               "spatial SRNL backward supports head_dim 16 and 32; got %d", head_dim);
+    VH_REQUIRE(C % head_dim == 0, VH_ERR_SHAPE, "C=%lld is not a multiple of head_dim=%d", (long long)C, head_dim);
+    VH_REQUIRE(H * W < (int64_t(1) << 24), VH_ERR_SHAPE, "spatial SRNL supports H*W < 2^24 pixels, got %lld",
+               (long long)(H * W));
+    VH_REQUIRE(valid_dtype(io_dtype), VH_ERR_DTYPE, "unsupported io dtype code %d", io_dtype);
+    for (int r = 0; r < 4; ++r)
+        VH_REQUIRE(chunks[r] > 0 && chunks[r] <= kBwdLongChunk, VH_ERR_ARG,
+                   "SRNL backward chunk lengths must be in [1, %d], got %lld", kBwdLongChunk, (long long)chunks[r]);
+    const SpatialBwdLayout lay = spatial_bwd_layout(B, H, W, C, head_dim, io_dtype, chunks);
+    VH_REQUIRE(workspace && workspace_bytes >= lay.total, VH_ERR_WORKSPACE,
+               "spatial SRNL backward workspace needs %zu bytes, got %zu", lay.total,
+               workspace ? workspace_bytes : (size_t)0);
+    VH_REQUIRE(lay.lines.lines * lay.lines.nc * lay.lines.sd < (int64_t(1) << 40) && lay.lines.lines < (int64_t(1) << 31),
+               VH_ERR_SHAPE, "SRNL backward problem too large");
+    char* const ws = static_cast<char*>(workspace);
+    BwdParams bp{};
+    bp.x = x; bp.q = q; bp.dy = dout;
+    bp.m0[0] = M_m; bp.m0[1] = M_v; bp.m0[2] = M_k; bp.m0[3] = M_eta; bp.m0[4] = M_alpha;
+    bp.states = reinterpret_cast<float*>(ws);
+    bp.gtraj = bp.states + lay.lines.states;
+    bp.dline = bp.states + lay.lines.states + lay.lines.traj;
+    bp.dx_planes = ws + lay.dx_planes;
+    bp.dq_planes = ws + lay.dq_planes;
+    bp.B = B; bp.R = 4; bp.heads = C / head_dim; bp.N = H * W; bp.nc = lay.lines.nc;
+    bp.segs = lay.lines.segs;
+    bp.io_dtype = io_dtype; bp.q_raw = 1;
+    for (int r = 0; r < 4; ++r) bp.chunk[r] = static_cast<int>(chunks[r]);
+    bp.k = *consts;
+    bp.scale = dir_weight;
+    bp.H = H; bp.W = W; bp.inv_h = 1.0f / static_cast<float>(H);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    int rc = launch_backward_blocks(bp, head_dim, lay.lines.waves, lay.lines.lines, s);
+    if (rc) return rc;
+    rc = launch_backward_reduce(bp.dline, B, 4 * bp.heads, head_dim, dM_m, dM_v, dM_k, dM_eta, dM_alpha, s);
+    if (rc) return rc;
+    MergeParams mp{};
+    mp.dx_planes = bp.dx_planes; mp.dq_planes = bp.dq_planes; mp.x = x;
+    mp.dout = dout; mp.skip = d_skip; mp.scale = dir_weight;
+    mp.skip_per_direction = skip_per_direction ? 1 : 0;
+    mp.dx = dx; mp.dq = dq;
+    mp.part = reinterpret_cast<float*>(ws + lay.parts);
+    mp.pixels = B * H * W; mp.C = C;
+    mp.groups = lay.groups;
+    const dim3 grid(static_cast<unsigned>(lay.blocks), static_cast<unsigned>((C / 8 + lay.groups - 1) / lay.groups));
+    if (io_dtype == VH_DTYPE_F32) hipLaunchKernelGGL(srnl_backward_merge_kernel<float>, grid, dim3(256), 0, s, mp);
+    else if (io_dtype == VH_DTYPE_BF16) hipLaunchKernelGGL(srnl_backward_merge_kernel<bf16_t>, grid, dim3(256), 0, s, mp);
+    else hipLaunchKernelGGL(srnl_backward_merge_kernel<f16_t>, grid, dim3(256), 0, s, mp);
+    rc = check_launch("srnl_backward_merge_kernel");
+    if (rc) return rc;
+    hipLaunchKernelGGL(srnl_backward_params_kernel, dim3(static_cast<unsigned>(C)), dim3(256), 0, s, mp.part, lay.blocks,
+                       C, head_dim, M_m, dM_m, d_skip, mp.skip_per_direction, dir_weight, dd_skip, ddir_weight);
+    return check_launch("srnl_backward_params_kernel");
 }
 
 }  // extern "C"

@@ -71,6 +71,17 @@ __device__ __forceinline__ v4f load_io4(const void* p, int64_t idx, int io) {
     return r;
 }
 
+__device__ __forceinline__ void store_io4(void* p, int64_t idx, int io, v4f v) {
+    if (io == VH_DTYPE_F32) {
+        *reinterpret_cast<v4f_any*>(static_cast<float*>(p) + idx) = v;
+        return;
+    }
+    us4_any u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = io == VH_DTYPE_BF16 ? from_f32<bf16_t>(v[i]).bits : from_f32<f16_t>(v[i]).bits;
+    *reinterpret_cast<us4_any*>(static_cast<uint16_t*>(p) + idx) = u;
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp0(float v) {   // 0 where the source lane is outside the row
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
@@ -373,7 +384,7 @@ __device__ __forceinline__ void copy_tiles(const v4f (&from)[ND][ND], v4f (&to)[
         for (int j = 0; j < ND; ++j) to[i][j] = from[i][j];
 }
 
-template <int D, int W>
+template <int D, int W, bool SPATIAL>
 __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const BwdParams p) {
     constexpr int ND = D / 16, NT = ND * ND, SD = 3 * D * D + 2 * D, DD = D * D;
     using Tok = Tokens<ND>;
@@ -391,9 +402,20 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
     const int C = chunk_of(p.chunk, r_dir);
     const int64_t N = p.N, nc = (N + C - 1) / C;
     const int nb = (C + 15) / 16, nseg = (nb + W - 1) / W;
-    const int64_t xbase = ln * p.N * D;
-    const int64_t qbase = p.q_raw ? (b * p.R + r_dir) * p.N * (p.heads * D) + head * D : xbase;
-    const int64_t qstride = p.q_raw ? p.heads * D : D;
+    // Element offsets of token t (this lane's first channel): of x, dy and dx, and of q and dq.
+    const bool q_raw = SPATIAL || p.q_raw;
+    const int64_t C_all = p.heads * D;
+    const int64_t xbase = (SPATIAL ? b * N * C_all + head * D : ln * N * D) + 4 * g;
+    const int64_t qbase = SPATIAL ? xbase : p.q_raw ? (b * p.R + r_dir) * N * C_all + head * D + 4 * g : xbase;
+    auto x_at = [&](int64_t t) {
+        if constexpr (SPATIAL) return xbase + scan_to_pixel(r_dir, t, p.H, p.W, p.inv_h) * C_all;
+        else return xbase + t * D;
+    };
+    auto q_at = [&](int64_t t, int64_t x_off) {
+        if constexpr (SPATIAL) return x_off;
+        else return qbase + t * (p.q_raw ? C_all : D);
+    };
+    const int64_t plane = SPATIAL ? r_dir * p.B * N * C_all : 0;
     float* const my_gam = p.states + ln * p.nc * DD;
     float* const my_seg = p.gtraj + (ln * W + w) * static_cast<int64_t>(p.segs) * DD;
 
@@ -405,6 +427,9 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
         for (int r = 0; r < 4; ++r)   // N(M^T): column 16 j + c of the tile is row 16 j + c of M
             v[r] = m < 2 ? src[(16 * j + c) * D + 16 * i + 4 * g + r] : src[(16 * i + 4 * g + r) * D + 16 * j + c];
+        // the gradient of y_r is the direction weight times dy: folded into the rows of M_m
+        if (SPATIAL && m == 4)
+            v *= *reinterpret_cast<const v4f_any*>(p.scale + r_dir * C_all + head * D + 16 * i + 4 * g);
         sh.mem[m][t % NT][lane] = v;
     }
     if (threadIdx.x < 2 * D)
@@ -415,11 +440,16 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
         const int tl = 16 * blk + tau;
         const int64_t t = ch * C + tl;
         valid = tl < C && t < N;
+        const int64_t at = x_at(valid ? t : 0);
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
             X[i] = zero;
-            if (valid) X[i] = load_io4(p.x, xbase + t * D + 16 * i + 4 * g, p.io_dtype);
+            if (valid) X[i] = load_io4(p.x, at + 16 * i, p.io_dtype);
         }
+    };
+    auto store_dx = [&](int64_t at, v4f v) {
+        if constexpr (SPATIAL) store_io4(p.dx_planes, plane + at, p.io_dtype, v);
+        else *reinterpret_cast<v4f_any*>(p.dx + at) = v;
     };
     auto identity = [&](v4f (&M)[ND][ND]) {
 #pragma unroll
@@ -626,13 +656,13 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 }
                 XT[j] = L.transpose(X[j]);
             }
-            const int64_t at = xbase + (ch * C + 16 * blk + tau) * D + 4 * g;
+            const int64_t at = x_at(valid ? ch * C + 16 * blk + tau : 0);
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
                 v4f dx = zero;
 #pragma unroll
                 for (int i = 0; i < ND; ++i) dx = mm(Gam[i][j], dz[i], dx);
-                if (valid) *reinterpret_cast<v4f_any*>(p.dx + at + 16 * j) = dx;
+                if (valid) store_dx(at + 16 * j, dx);
                 const v4f dzT = L.transpose(dz[j]);
 #pragma unroll
                 for (int i = 0; i < ND; ++i) Ep[j][i] = mm(dzT, XT[i], Ep[j][i]);
@@ -744,21 +774,21 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
             const int tl = 16 * blk + tau;
             const int64_t tok = ch * C + tl;
             const bool valid = tl < C && tok < N;
-            const int64_t at = xbase + tok * D + 4 * g, qat = qbase + tok * qstride + 4 * g;
+            const int64_t at = x_at(valid ? tok : 0), qat = q_at(valid ? tok : 0, at);
             v4f q[ND], dy[ND];
             float qq = 0.f;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
                 q[i] = dy[i] = zero;
                 if (valid) {
-                    q[i] = load_io4(p.q, qat + 16 * i, p.q_raw ? p.io_dtype : VH_DTYPE_F32);
+                    q[i] = load_io4(p.q, qat + 16 * i, q_raw ? p.io_dtype : VH_DTYPE_F32);
                     dy[i] = *reinterpret_cast<const v4f_any*>(p.dy + at + 16 * i);
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) qq += q[i][r] * q[i][r];
             }
             float qinv = 1.f;
-            if (p.q_raw) qinv = 1.f / fmaxf(sqrtf(xor16_32_sum(qq)), 1e-12f);
+            if (q_raw) qinv = 1.f / fmaxf(sqrtf(xor16_32_sum(qq)), 1e-12f);
             v4f dp[ND], qT[ND], dpT[ND];
 #pragma unroll
             for (int i = 0; i < ND; ++i) q[i] *= qinv;
@@ -794,11 +824,11 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
             qdot = xor16_32_sum(qdot);
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                if (p.q_raw) dq[j] = (qinv > 9.999e11f ? dq[j] : dq[j] - q[j] * qdot) * qinv;
+                if (q_raw) dq[j] = (qinv > 9.999e11f ? dq[j] : dq[j] - q[j] * qdot) * qinv;
                 if (valid) {
-                    *reinterpret_cast<v4f_any*>(p.dq + qat + 16 * j) = dq[j];
-                    // the last chunk's x reaches no output
-                    if (ch == nc - 1) *reinterpret_cast<v4f_any*>(p.dx + at + 16 * j) = zero;
+                    if constexpr (SPATIAL) store_io4(p.dq_planes, plane + qat + 16 * j, p.io_dtype, dq[j]);
+                    else *reinterpret_cast<v4f_any*>(p.dq + qat + 16 * j) = dq[j];
+                    if (ch == nc - 1) store_dx(at + 16 * j, zero);   // the last chunk's x reaches no output
                 }
             }
         }
@@ -880,8 +910,9 @@ int bwd_block_waves(int head_dim, int64_t max_chunk) {
 int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream) {
     auto go = [&](auto d, auto w) {
         constexpr int D = decltype(d)::value, W = decltype(w)::value;
-        hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W>), dim3(static_cast<unsigned>(lines)), dim3(64 * W), 0,
-                           stream, p);
+        const dim3 grid(static_cast<unsigned>(lines)), block(64 * W);
+        if (p.scale) hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, false>), grid, block, 0, stream, p);
     };
     auto by_waves = [&](auto d) {
         constexpr int D = decltype(d)::value;

@@ -11,8 +11,9 @@ messages.  The implementation has three execution paths:
   one readout; no serialized copy of x or q is made;
 * sequence (inference, any other fixed chunk length): the packed native scan over
   serialized copies, then the native direction fusion;
-* ordinary (training or gradients enabled): the same packed scan and fusion through
-  their autograd Functions.
+* ordinary (training or gradients enabled): the spatial entry and its backward as one
+  autograd Function where the block-form kernels apply (head_dim 16 or 32, chunks of at
+  most 256), else the packed scan and fusion through theirs.
 """
 
 import torch
@@ -21,6 +22,7 @@ from torch.nn import functional as F
 from torch.nn.init import trunc_normal_
 
 from .srnl import SRNL
+from .srnl_core.spatial import spatial_training_supported, srnl_spatial
 from ..utils.cached_params import linear_weights
 from ..utils.cuda import on_tensor_device
 from ..utils.direction_fusion import visionhope_postprocess_scale
@@ -35,6 +37,15 @@ def scan_orders(seq_hw, height, width):
     batch, length, channels = seq_hw.shape
     col_major = seq_hw.reshape(batch, height, width, channels).transpose(1, 2).reshape(batch, length, channels)
     return torch.stack((seq_hw, seq_hw.flip(1), col_major, col_major.flip(1)), dim=1)
+
+
+def _observed(module):
+    """Whether hooks watch ``module``'s calls (its own or the global module hooks)."""
+    hooks = torch.nn.modules.module
+    return any(getattr(module, name) for name in ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks",
+                                                  "_backward_pre_hooks")) or any(
+        getattr(hooks, name) for name in ("_global_forward_hooks", "_global_forward_pre_hooks",
+                                          "_global_backward_hooks", "_global_backward_pre_hooks"))
 
 
 def _query_dtype(x):
@@ -158,9 +169,24 @@ class VisionHOPEOperator(nn.Module):
         ``memories`` (the inference sequence path) the scan is the gradient-free entry."""
         batch, _, height, width = x.shape
         seq_hw = x.flatten(2).transpose(1, 2)
+        if memories is None and self._spatial_training_ok():
+            q_hw = self.W_q(seq_hw)
+            chunks = self.srnl._chunk_lengths((height, width))
+            if spatial_training_supported(x, q_hw, self.head_dim, chunks):
+                states = self.srnl._validate_memories(x.device)
+                x_nhwc = x.permute(0, 2, 3, 1).contiguous()
+                if x_nhwc.data_ptr() == x.data_ptr() and not self.W_q.weight.requires_grad:
+                    x_nhwc = x_nhwc.clone()   # nothing else keeps x for the backward: the caller may overwrite it
+                out = srnl_spatial(states, x_nhwc,
+                                   q_hw.reshape(batch, height, width, self.dim), self.d_skip.float(),
+                                   self.direction_weights().float(), chunks).permute(0, 3, 1, 2)
+                return out.contiguous(memory_format=torch.channels_last if channels_last
+                                      else torch.contiguous_format)
+            queries = scan_orders(q_hw, height, width)
+        else:
+            queries = self.project_queries(seq_hw, height, width)
         lines = scan_orders(seq_hw, height, width)
         lines = lines.reshape(batch, 4, height * width, self.num_heads, self.head_dim).transpose(2, 3).contiguous()
-        queries = self.project_queries(seq_hw, height, width)
         if memories is None:
             y = self.srnl(lines, queries, spatial_shape=(height, width))
         else:
@@ -171,6 +197,13 @@ class VisionHOPEOperator(nn.Module):
         # reference's eligibility test is can_fuse_scale_postprocess, operator.py:116-119).
         return visionhope_postprocess_scale(y, lines, self.d_skip.float(), self.direction_weights().float(),
                                             height, width, channels_last)
+
+    def _spatial_training_ok(self):
+        """Whether the ordinary path may run without calling ``srnl`` and ``project_queries``
+        as such: both are this package's own and nothing watches the call of ``srnl``."""
+        return (type(self.srnl) is SRNL and type(self).project_queries is VisionHOPEOperator.project_queries
+                and "project_queries" not in self.__dict__ and "forward" not in self.srnl.__dict__
+                and not _observed(self.srnl))
 
     def _merge_weights(self):
         """FP32 merge weights for the inference kernels (no autograd)."""
