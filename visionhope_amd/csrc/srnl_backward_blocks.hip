@@ -23,14 +23,8 @@
 // (v_mfma_f32_16x16x4_f32), nothing is split or rounded to 16 bits.
 //
 // Mapping.  One workgroup per line, wave w holding block w of the current 16 W-token
-// segment of a chunk (W = 1, 2, 4 or 8 waves; longer chunks take several segments).  A
-// tile is 4 registers: lane (g = l / 16, c = l % 16) holds rows 4g..4g+3 of column c, which
-// is what the matrix core returns, the B operand of that matrix and the A operand of its
-// transpose; so mm(A, B) = A^T B needs no data movement, and where a transpose is needed it
-// goes through 1.3 KB of wave-private LDS.  Token slots are permuted: slot index n stands for
-// time 4 (n % 4) + n / 4 of the block, which puts four consecutive times into one register
-// index, so one rank-4 matrix instruction eliminates them: a 16 x 16 triangular solve is 7
-// instructions (the 4 x 4 diagonal inverses are formed on the VALU).
+// segment of a chunk (W = 1, 2, 4 or 8 waves; longer chunks take several segments).  Tiles,
+// slot order and solves: srnl_blocks.h.
 //
 // Bound: the dependency chain.  A chunk is one serial chain of solves and products per line,
 // and the chunks of a line follow one another; the compulsory matrix work and the bytes take
@@ -43,19 +37,11 @@
 #include <cmath>
 
 #include "srnl_backward.h"
-#include "srnl_device.h"
+#include "srnl_blocks.h"
 
 namespace vh {
+using namespace blocks;
 namespace {
-
-constexpr int kTrStride = 20;   // floats per row of the transpose scratch (16-byte aligned rows)
-
-// acc + A^T B
-__device__ __forceinline__ v4f mm(v4f a, v4f b, v4f acc) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc = mfma4(a[j], b[j], acc);
-    return acc;
-}
 
 typedef v4f v4f_any __attribute__((aligned(4)));
 typedef unsigned short us4_any __attribute__((ext_vector_type(4), aligned(2)));
@@ -82,29 +68,16 @@ __device__ __forceinline__ void store_io4(void* p, int64_t idx, int io, v4f v) {
     *reinterpret_cast<us4_any*>(static_cast<uint16_t*>(p) + idx) = u;
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp0(float v) {   // 0 where the source lane is outside the row
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+// 1 / x and e^x within about one ulp for the normal ranges met here, in 3 and 6 instructions
+// (hardware approximation and one correction) instead of the library's 10 and more.
+__device__ __forceinline__ float rcp1(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, r, 1.f), r, r);
 }
-
-// Prefix sums over the 16 slots of a block in time order (slot c = time 4 (c % 4) + c / 4),
-// the same in every row of lanes: inclusive, exclusive and the total.
-struct Prefix {
-    float incl, excl, total;
-};
-__device__ __forceinline__ Prefix time_prefix(float v, int c) {
-    float in = v + dpp0<0x114>(v);              // row_shr 4: the previous time of the same group of four
-    in += dpp0<0x118>(in);                      // row_shr 8
-    float t = v + dpp0<0x128>(v);               // row_ror 8, 4: the group's total
-    t += dpp0<0x124>(t);
-    // every lane moves before the selects: a move inside a branch would read inactive lanes
-    const int j = c & 3;
-    const float t1 = dpp0<0x90>(t);             // quad_perm [0, 0, 1, 2]
-    float s = t + (j >= 1 ? t1 : 0.f);
-    const float s2 = dpp0<0x40>(s);             // quad_perm [0, 0, 0, 1]
-    s += j >= 2 ? s2 : 0.f;
-    const float s1 = dpp0<0x90>(s), before = j >= 1 ? s1 : 0.f;
-    return {before + in, before + dpp0<0x114>(in), dpp0<0xFF>(s)};
+__device__ __forceinline__ float exp1(float x) {
+    constexpr float kLog2e = 1.44269504088896341f, kLog2eLow = 1.925963033500e-8f, kLn2 = 0.69314718055994531f;
+    const float t = x * kLog2e, rest = fmaf(x, kLog2e, -t) + x * kLog2eLow, e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e, rest * kLn2, e);
 }
 
 __device__ __forceinline__ float wave_sum(float v) { return row_group_sum<16>(xor16_32_sum(v)); }
@@ -116,9 +89,7 @@ struct Shared {
     v4f mem[5][NT][64];
     float ev[2][D];
     float E[D][D + 4];                 // dGamma of the next chunk, row major
-    float tr[W][16 * kTrStride];       // transpose scratch
-    float sc[W][5][16];                // per-slot scalars, read four rows at a time
-    float diag[W][64];                 // the 4 x 4 diagonal blocks of L
+    Scratch scratch[W];
     // Block maps X, X^T, Y^T of the segment (W > 1); also the waves' partial sums.
     v4f maps[W > 1 ? W : 1][W > 1 ? 3 : 1][NT][64];
 };
@@ -128,57 +99,19 @@ template <int ND>
 struct Tokens {
     v4f Z[ND], K[ND], Dl[ND];      // z, k, k - v: channel rows, slot columns
     v4f KT[ND], DlT[ND];           // the last two transposed
-    v4f Mc;                        // eta^_s a_t / a_{s+1} for the earlier slot s and the later slot t of (row, column)
-    v4f nC;                        // -(that times k_s . k_t): L above, L^T below the diagonal, negated
-    v4f De_r, Da_r;                // D_e, D_a by row
-    float De, Da, a;               // by column; product of the block's retentions
-    float dl, du;                  // this lane's entry of the diagonal inverses (lower, upper solve)
+    Decays d;
+    Triangle tri;
     float inv_k, eff, alpha;
-    float dn, denom, cap, deff_deta, deff_dcap, deff_dalpha, deff_dksq, s_eta, s_alpha;
+    float dn, inv_denom, cap, deff_deta, deff_dcap, deff_dalpha, deff_dksq, s_eta, s_alpha;
 };
 
 template <int D, int W>
 struct Line {
     static constexpr int ND = D / 16;
     Shared<D, W>& sh;
-    const int w, lane, g, c, tau;   // tau: time of slot c within the block
+    const int w;
+    const Block bl;
     const vh_srnl_consts& k;
-
-    __device__ __forceinline__ v4f transpose(v4f v) const {
-        float* s = sh.tr[w];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s[(4 * g + i) * kTrStride + c] = v[i];
-        __builtin_amdgcn_wave_barrier();
-        const v4f r = *reinterpret_cast<const v4f*>(&s[c * kTrStride + 4 * g]);
-        __builtin_amdgcn_wave_barrier();
-        return r;
-    }
-    __device__ __forceinline__ v4f rows_of(const float* s) const { return *reinterpret_cast<const v4f*>(s + 4 * g); }
-    __device__ __forceinline__ int row_time(int i) const { return 4 * i + g; }
-
-    // B <- (I + L^T)^-1 B and B <- (I + L)^-1 B for token-row tiles.
-    __device__ __forceinline__ void solve_lower(const Tokens<ND>& t, v4f (&b)[ND]) const {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const float a1 = (c & 3) == s ? t.dl : 0.f, a2 = (c & 3) > s ? t.nC[s] : 0.f;
-#pragma unroll
-            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][s], b[j]);
-            if (s < 3)
-#pragma unroll
-                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][s], b[j]);
-        }
-    }
-    __device__ __forceinline__ void solve_upper(const Tokens<ND>& t, v4f (&b)[ND]) const {
-#pragma unroll
-        for (int s = 3; s >= 0; --s) {
-            const float a1 = (c & 3) == s ? t.du : 0.f, a2 = (c & 3) < s ? t.nC[s] : 0.f;
-#pragma unroll
-            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][s], b[j]);
-            if (s > 0)
-#pragma unroll
-                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][s], b[j]);
-        }
-    }
 
     // Keys, values and gates of the block from x (channel rows; zero in slots past the
     // chunk) and Gamma^T.  Slots past the chunk act as the identity.
@@ -199,10 +132,10 @@ struct Line {
             V[i] = zero;
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                t.K[i] = mm(sh.mem[0][j * ND + i][lane], t.Z[j], t.K[i]);
-                V[i] = mm(sh.mem[1][j * ND + i][lane], t.Z[j], V[i]);
+                t.K[i] = mm(sh.mem[0][j * ND + i][bl.lane], t.Z[j], t.K[i]);
+                V[i] = mm(sh.mem[1][j * ND + i][bl.lane], t.Z[j], V[i]);
             }
-            const v4f e = rows_of(&sh.ev[0][16 * i]), a = rows_of(&sh.ev[1][16 * i]);
+            const v4f e = bl.rows_of(&sh.ev[0][16 * i]), a = bl.rows_of(&sh.ev[1][16 * i]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 pe += e[r] * t.Z[i][r];
@@ -225,91 +158,55 @@ struct Line {
                 dd += t.Dl[i][r] * t.Dl[i][r];
                 kk += t.K[i][r] * t.K[i][r];
             }
-        t.dn = sqrtf(xor16_32_sum(dd) + 1e-12f);
+        t.dn = __builtin_amdgcn_sqrtf(xor16_32_sum(dd) + 1e-12f);
         const float ksq = xor16_32_sum(kk);
         const float amin = k.min_retention, mu = k.injection_margin, fac = k.spectral_factor;
         const float ep = fminf(10.f, fmaxf(-10.f, pe_raw)), ap = fminf(10.f, fmaxf(-10.f, pa_raw));
-        const float eta = k.step_scale * logf(1.f + expf(ep));
-        const float sg = 1.f / (1.f + expf(-ap));
+        const float e_pre = exp1(ep);
+        const float eta = k.step_scale * (0.69314718055994531f * __builtin_amdgcn_logf(1.f + e_pre));
+        const float sg = rcp1(1.f + exp1(-ap));
         t.alpha = amin + (1.f - amin) * sg;
-        t.s_eta = fabsf(pe_raw) <= 10.f ? k.step_scale / (1.f + expf(-ep)) : 0.f;
+        t.s_eta = fabsf(pe_raw) <= 10.f ? k.step_scale * e_pre * rcp1(1.f + e_pre) : 0.f;
         t.s_alpha = fabsf(pa_raw) <= 10.f ? (1.f - amin) * sg * (1.f - sg) : 0.f;
-        t.denom = t.dn + 1e-6f;
-        t.cap = mu * (1.f - t.alpha) / t.denom;
-        const float u = eta / t.cap, e_neg = expf(-u);
-        t.eff = t.cap * (-expm1f(-u));
+        t.inv_denom = rcp1(t.dn + 1e-6f);
+        t.cap = mu * (1.f - t.alpha) * t.inv_denom;
+        // eta^ = cap (1 - e^-u) and its derivatives, u = eta / cap; Taylor series below 1/4,
+        // where the differences would cancel (truncated below 2e-9)
+        const float u = eta * rcp1(t.cap), e_neg = exp1(-u);
+        const float near1 = u * (1.f - u * (1.f / 2 - u * (1.f / 6 - u * (1.f / 24 - u * (1.f / 120 - u * (1.f / 720 -
+                            u * (1.f / 5040)))))));
+        const float near2 = u * u * (1.f / 2 - u * (1.f / 3 - u * (1.f / 8 - u * (1.f / 30 - u * (1.f / 144 - u * (1.f / 840 -
+                            u * (1.f / 5760)))))));
+        const float one_minus = u < 0.25f ? near1 : 1.f - e_neg;
+        t.eff = t.cap * one_minus;
         t.deff_deta = e_neg;
-        t.deff_dcap = softcap_dcap(u, e_neg);
+        t.deff_dcap = u < 0.25f ? near2 : one_minus - u * e_neg;
         t.deff_dalpha = 0.f;
         t.deff_dksq = 0.f;
         if (k.spectral_clamp) {
-            const float den = fmaxf(ksq, 1e-20f), lim = nextafterf(fac * t.alpha / den, 0.f);
-            if (t.eff > lim) {
-                t.eff = lim;
-                t.deff_deta = 0.f;
-                t.deff_dcap = 0.f;
-                t.deff_dalpha = fac / den;
-                if (ksq > 1e-20f) t.deff_dksq = -fac * t.alpha / (den * den);
-            }
+            const float inv = rcp1(fmaxf(ksq, 1e-20f)), bound = fac * t.alpha * inv;
+            const float lim = __uint_as_float(__float_as_uint(bound) - 1u);   // nextafter toward 0 (bound > 0)
+            const bool over = t.eff > lim;
+            t.eff = over ? lim : t.eff;
+            t.deff_deta = over ? 0.f : t.deff_deta;
+            t.deff_dcap = over ? 0.f : t.deff_dcap;
+            t.deff_dalpha = over ? fac * inv : 0.f;
+            t.deff_dksq = over && ksq > 1e-20f ? -bound * inv : 0.f;
         }
         if (!valid) {
             t.eff = 0.f;
             t.alpha = 1.f;
         }
-        const Prefix la = time_prefix(log2f(t.alpha), c);
-        t.a = exp2f(la.total);
-        t.Da = exp2f(la.excl);
-        t.De = t.eff * exp2f(la.total - la.incl);
-        float(&sc)[5][16] = sh.sc[w];
-        sc[0][c] = t.eff;
-        sc[1][c] = la.incl;
-        sc[2][c] = la.excl;
-        sc[3][c] = t.De;
-        sc[4][c] = t.Da;
-        __builtin_amdgcn_wave_barrier();
-        const v4f eff_r = rows_of(sc[0]), incl_r = rows_of(sc[1]), excl_r = rows_of(sc[2]);
-        t.De_r = rows_of(sc[3]);
-        t.Da_r = rows_of(sc[4]);
-        __builtin_amdgcn_wave_barrier();
+        t.d = bl.decays(t.eff, t.alpha);
         v4f gram = zero;
 #pragma unroll
         for (int i = 0; i < ND; ++i) gram = mm(t.K[i], t.K[i], gram);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool row_first = row_time(i) < tau;
-            const float m = (row_first ? eff_r[i] : t.eff) * exp2f(row_first ? la.excl - incl_r[i] : excl_r[i] - la.incl);
-            t.Mc[i] = row_time(i) == tau ? 0.f : m;
-            t.nC[i] = -t.Mc[i] * gram[i];
-        }
-        // Inverse of the 4 x 4 unit triangle of this slot's group of four times: this lane's
-        // entry is that of times min(g, f), max(g, f) of group c % 4, f = c / 4.
-        const int grp = c & 3, f = c >> 2;
-        float* dg = sh.diag[w];
-        dg[grp * 16 + 4 * g + f] = grp == 0 ? t.nC[0] : grp == 1 ? t.nC[1] : grp == 2 ? t.nC[2] : t.nC[3];
-        __builtin_amdgcn_wave_barrier();
-        const v4f r0 = *reinterpret_cast<const v4f*>(dg + grp * 16), r1 = *reinterpret_cast<const v4f*>(dg + grp * 16 + 4);
-        const v4f r2 = *reinterpret_cast<const v4f*>(dg + grp * 16 + 8);
-        __builtin_amdgcn_wave_barrier();
-        // r holds -L; (I - N)^-1 = I + N + N^2 + N^3 with N = -L
-        const float t02 = r0[2] + r0[1] * r1[2], t13 = r1[3] + r1[2] * r2[3];
-        const float t03 = r0[3] + r0[1] * t13 + r0[2] * r2[3];
-        const int lo = min(g, f), hi = max(g, f);
-        const float from0 = hi == 1 ? r0[1] : hi == 2 ? t02 : t03, from1 = hi == 2 ? r1[2] : t13;
-        const float inv = lo == 0 ? from0 : lo == 1 ? from1 : r2[3];
-        t.dl = g < f ? inv : 0.f;
-        t.du = f < g ? inv : 0.f;
+        t.tri = bl.triangle(t.d, gram);
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
-            t.KT[i] = transpose(t.K[i]);
-            t.DlT[i] = transpose(t.Dl[i]);
+            t.KT[i] = bl.transpose(t.K[i]);
+            t.DlT[i] = bl.transpose(t.Dl[i]);
         }
-    }
-
-    __device__ __forceinline__ v4f diagonal(float v) const {   // v I as a tile
-        v4f r;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = 4 * g + i == c ? v : 0.f;
-        return r;
     }
 
     // The block's maps into slot w of the segment's table: X, Y^T, and X^T for the adjoint.
@@ -319,18 +216,18 @@ struct Line {
         v4f S[ND], KD[ND];
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
-            S[j] = t.De_r * t.KT[j];
-            KD[j] = -(t.Da_r * t.KT[j]);
+            S[j] = t.d.De_r * t.KT[j];
+            KD[j] = -(t.d.Da_r * t.KT[j]);
         }
-        solve_upper(t, S);
+        bl.solve_upper(t.tri, S);
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                const v4f start = i == j ? diagonal(t.a) : zero;
-                sh.maps[w][0][i * ND + j][lane] = mm(KD[i], S[j], start);
-                if constexpr (ADJOINT) sh.maps[w][1][i * ND + j][lane] = mm(S[i], KD[j], start);
-                sh.maps[w][2][i * ND + j][lane] = mm(-S[i], t.DlT[j], zero);
+                const v4f start = i == j ? bl.diagonal(t.d.a) : zero;
+                sh.maps[w][0][i * ND + j][bl.lane] = mm(KD[i], S[j], start);
+                if constexpr (ADJOINT) sh.maps[w][1][i * ND + j][bl.lane] = mm(S[i], KD[j], start);
+                sh.maps[w][2][i * ND + j][bl.lane] = mm(-S[i], t.DlT[j], zero);
             }
     }
     // G^T <- X^T G^T + Y^T of block b
@@ -339,12 +236,12 @@ struct Line {
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
-            for (int j = 0; j < ND; ++j) out[i][j] = sh.maps[b][2][i * ND + j][lane];
+            for (int j = 0; j < ND; ++j) out[i][j] = sh.maps[b][2][i * ND + j][bl.lane];
 #pragma unroll
         for (int m = 0; m < ND; ++m)
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                const v4f x = sh.maps[b][0][m * ND + i][lane];
+                const v4f x = sh.maps[b][0][m * ND + i][bl.lane];
 #pragma unroll
                 for (int j = 0; j < ND; ++j) out[i][j] = mm(x, GT[m][j], out[i][j]);
             }
@@ -365,7 +262,7 @@ struct Line {
         for (int m = 0; m < ND; ++m)
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                const v4f x = sh.maps[b][1][m * ND + i][lane];
+                const v4f x = sh.maps[b][1][m * ND + i][bl.lane];
 #pragma unroll
                 for (int j = 0; j < ND; ++j) out[i][j] = mm(x, HT[m][j], out[i][j]);
             }
@@ -384,15 +281,19 @@ __device__ __forceinline__ void copy_tiles(const v4f (&from)[ND][ND], v4f (&to)[
         for (int j = 0; j < ND; ++j) to[i][j] = from[i][j];
 }
 
+// Waves per SIMD the register budget is cut for.
+template <int D, int W>
+constexpr int kMinWaves = D == 16 ? (W == 1 ? 3 : 2) : 1;
+
 template <int D, int W, bool SPATIAL>
-__global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const BwdParams p) {
+__global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_blocks_kernel(const BwdParams p) {
     constexpr int ND = D / 16, NT = ND * ND, SD = 3 * D * D + 2 * D, DD = D * D;
     using Tok = Tokens<ND>;
     __shared__ Shared<D, W> sh;
     const int w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const int lane = static_cast<int>(threadIdx.x) & 63, g = lane >> 4, c = lane & 15;
-    const int tau = 4 * (c & 3) + (c >> 2);
-    const Line<D, W> L{sh, w, lane, g, c, tau, p.k};
+    const Line<D, W> L{sh, w, Block(sh.scratch[w], static_cast<int>(threadIdx.x) & 63), p.k};
+    const Block& bl = L.bl;
+    const int lane = bl.lane, g = bl.g, c = bl.c, tau = bl.tau;
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
 
     const int64_t ln = blockIdx.x;
@@ -400,18 +301,27 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
     const int r_dir = static_cast<int>((ln / p.heads) % p.R);
     const int64_t b = ln / RH, head = ln % p.heads;
     const int C = chunk_of(p.chunk, r_dir);
-    const int64_t N = p.N, nc = (N + C - 1) / C;
+    using Index = std::conditional_t<SPATIAL, int, int64_t>;   // a map has fewer than 2^24 pixels
+    const Index N = static_cast<Index>(p.N), nc = (N + C - 1) / C;
     const int nb = (C + 15) / 16, nseg = (nb + W - 1) / W;
     // Element offsets of token t (this lane's first channel): of x, dy and dx, and of q and dq.
     const bool q_raw = SPATIAL || p.q_raw;
     const int64_t C_all = p.heads * D;
     const int64_t xbase = (SPATIAL ? b * N * C_all + head * D : ln * N * D) + 4 * g;
     const int64_t qbase = SPATIAL ? xbase : p.q_raw ? (b * p.R + r_dir) * N * C_all + head * D + 4 * g : xbase;
-    auto x_at = [&](int64_t t) {
-        if constexpr (SPATIAL) return xbase + scan_to_pixel(r_dir, t, p.H, p.W, p.inv_h) * C_all;
+    // Pixel of scan index t (scan_to_pixel in 32 bits).
+    auto pixel_of = [&](int t) {
+        const uint32_t orig = static_cast<uint32_t>((r_dir & 1) ? static_cast<int>(p.N) - 1 - t : t);
+        if (r_dir < 2) return orig;
+        uint32_t col, row;
+        divmod24(orig, static_cast<uint32_t>(p.H), p.inv_h, col, row);
+        return row * static_cast<uint32_t>(p.W) + col;
+    };
+    auto x_at = [&](Index t) {
+        if constexpr (SPATIAL) return xbase + static_cast<int64_t>(pixel_of(t)) * static_cast<uint32_t>(C_all);
         else return xbase + t * D;
     };
-    auto q_at = [&](int64_t t, int64_t x_off) {
+    auto q_at = [&](Index t, int64_t x_off) {
         if constexpr (SPATIAL) return x_off;
         else return qbase + t * (p.q_raw ? C_all : D);
     };
@@ -436,9 +346,9 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
         sh.ev[threadIdx.x / D][threadIdx.x % D] = p.m0[3 + threadIdx.x / D][s * D + threadIdx.x % D];
     __syncthreads();
 
-    auto load_x = [&](int64_t ch, int blk, bool& valid, v4f (&X)[ND]) {
+    auto load_x = [&](Index ch, int blk, bool& valid, v4f (&X)[ND]) {
         const int tl = 16 * blk + tau;
-        const int64_t t = ch * C + tl;
+        const Index t = ch * C + tl;
         valid = tl < C && t < N;
         const int64_t at = x_at(valid ? t : 0);
 #pragma unroll
@@ -455,19 +365,19 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
-            for (int j = 0; j < ND; ++j) M[i][j] = i == j ? L.diagonal(1.f) : zero;
+            for (int j = 0; j < ND; ++j) M[i][j] = i == j ? bl.diagonal(1.f) : zero;
     };
     // R^T from K^T G^T of the block's entry gain (R (I + L) = G K D_a + Delta).
     auto solve_r = [&](const Tok& t, const v4f (&KG)[ND], v4f (&RT)[ND]) {
 #pragma unroll
-        for (int j = 0; j < ND; ++j) RT[j] = t.Da_r * KG[j] + t.DlT[j];
-        L.solve_lower(t, RT);
+        for (int j = 0; j < ND; ++j) RT[j] = t.d.Da_r * KG[j] + t.DlT[j];
+        bl.solve_lower(t.tri, RT);
     };
 
     // ---- 1. forward: Gamma before every chunk ------------------------------------------
     v4f GamT[ND][ND];
     identity(GamT);
-    for (int64_t ch = 0; ch < nc - 1; ++ch) {
+    for (Index ch = 0; ch < nc - 1; ++ch) {
         v4f G[ND][ND];
         if constexpr (W == 1) {
             v4f X[ND], RT[ND];
@@ -480,7 +390,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
             for (int i = 0; i < ND; ++i)
 #pragma unroll
                 for (int j = 0; j < ND; ++j)
-                    G[i][j] = mm(-RT[i], t.De_r * t.KT[j], i == j ? L.diagonal(t.a) : zero);
+                    G[i][j] = mm(-RT[i], t.d.De_r * t.KT[j], i == j ? bl.diagonal(t.d.a) : zero);
         } else {
             v4f GT[ND][ND];
             identity(GT);
@@ -501,7 +411,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
             for (int i = 0; i < ND; ++i)
 #pragma unroll
-                for (int j = 0; j < ND; ++j) G[i][j] = L.transpose(GT[j][i]);
+                for (int j = 0; j < ND; ++j) G[i][j] = bl.transpose(GT[j][i]);
         }
         // Gamma^T <- G^T Gamma^T
         v4f next[ND][ND];
@@ -520,7 +430,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 GamT[i][j] = next[i][j];
                 // row 16 j + c of Gamma, columns 16 i + 4 g ..
                 if ((i * ND + j) % W == w)
-                    *reinterpret_cast<v4f_any*>(my_gam + (ch + 1) * DD + (16 * j + c) * D + 16 * i +
+                    *reinterpret_cast<v4f_any*>(my_gam + static_cast<int64_t>(ch + 1) * DD + (16 * j + c) * D + 16 * i +
                                             4 * g) = next[i][j];
             }
     }
@@ -534,13 +444,13 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
         for (int j = 0; j < ND; ++j) dMm[i][j] = dMv[i][j] = dMk[i][j] = zero;
     }
-    for (int64_t ch = nc - 1; ch >= 0; --ch) {
+    for (Index ch = nc - 1; ch >= 0; --ch) {
         v4f Gam[ND][ND];
         if (ch == 0) {
             identity(GamT);
             identity(Gam);
         } else {
-            const float* src = my_gam + ch * DD;
+            const float* src = my_gam + static_cast<int64_t>(ch) * DD;
 #pragma unroll
             for (int i = 0; i < ND; ++i)
 #pragma unroll
@@ -575,19 +485,19 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                         else if (i == j) hg += 4 * g + r == c ? HT[i][j][r] : 0.f;
                     }
                 }
-                RbT[j] = -(t.De_r * kh);
+                RbT[j] = -(t.d.De_r * kh);
             }
-            L.solve_upper(t, RbT);
+            bl.solve_upper(t.tri, RbT);
 #pragma unroll
             for (int j = 0; j < ND; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) part += RbT[j][r] * (t.Da_r[r] * KG[j][r]);
-            const float phi0 = wave_sum(part + t.a * hg);   // <H, G> at the block start
+                for (int r = 0; r < 4; ++r) part += RbT[j][r] * (t.d.Da_r[r] * KG[j][r]);
+            const float phi0 = wave_sum(part + t.d.a * hg);   // <H, G> at the block start
             float rr = 0.f, rd = 0.f;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                R[i] = L.transpose(RT[i]);
-                Rb[i] = L.transpose(RbT[i]);
+                R[i] = bl.transpose(RT[i]);
+                Rb[i] = bl.transpose(RbT[i]);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     rr += Rb[i][r] * R[i][r];
@@ -597,12 +507,12 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
             rr = xor16_32_sum(rr);
             rd = xor16_32_sum(rd);
             const float phi = phi0 + time_prefix(rd, c).incl;
-            const float d_eff = t.eff > 0.f ? rr / t.eff : 0.f;
+            const float d_eff = t.eff > 0.f ? rr * rcp1(t.eff) : 0.f;
             const float d_cap = d_eff * t.deff_dcap;
-            const float d_alpha = (phi - rr) / t.alpha + d_cap * (-p.k.injection_margin / t.denom) + d_eff * t.deff_dalpha;
+            const float d_alpha = (phi - rr) * rcp1(t.alpha) - d_cap * p.k.injection_margin * t.inv_denom + d_eff * t.deff_dalpha;
             const float d_apre = valid ? d_alpha * t.s_alpha : 0.f;
             const float d_epre = d_eff * t.deff_deta * t.s_eta;
-            const float cdn = d_cap * (-t.cap / t.denom) / t.dn, cks = 2.f * d_eff * t.deff_dksq;
+            const float cdn = -d_cap * t.cap * t.inv_denom * rcp1(t.dn), cks = 2.f * d_eff * t.deff_dksq;
             v4f P = zero, PT = zero, Ws;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
@@ -610,7 +520,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 PT = mm(Rb[i], R[i], PT);
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Ws[r] = t.Mc[r] * (L.row_time(r) < tau ? P[r] : PT[r]);
+            for (int r = 0; r < 4; ++r) Ws[r] = t.d.M[r] * (bl.row_time(r) < tau ? P[r] : PT[r]);
             v4f dk[ND], dv[ND], ZT[ND];
             float kdot = 0.f;
 #pragma unroll
@@ -619,11 +529,11 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
                 for (int m = 0; m < ND; ++m) {
                     hr = mm(H[m][i], R[m], hr);
-                    if constexpr (W > 1) gr = mm(L.transpose(GTb[i][m]), Rb[m], gr);
+                    if constexpr (W > 1) gr = mm(bl.transpose(GTb[i][m]), Rb[m], gr);
                 }
                 if constexpr (W == 1) gr = Rb[i];
                 const v4f kw = mm(t.KT[i], Ws, zero);
-                dk[i] = gr * t.Da - hr * t.De - kw + Rb[i] + t.Dl[i] * cdn + t.K[i] * cks;
+                dk[i] = gr * t.d.Da - hr * t.d.De - kw + Rb[i] + t.Dl[i] * cdn + t.K[i] * cks;
                 dv[i] = -Rb[i] - t.Dl[i] * cdn;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) kdot += dk[i][r] * t.K[i][r];
@@ -634,11 +544,11 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 dk[i] = (dk[i] - t.K[i] * kdot) * t.inv_k;
                 dEv[i] += t.Z[i] * d_epre;
                 dAv[i] += t.Z[i] * d_apre;
-                ZT[i] = L.transpose(t.Z[i]);
+                ZT[i] = bl.transpose(t.Z[i]);
             }
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                const v4f dvT = L.transpose(dv[i]), dkT = L.transpose(dk[i]);
+                const v4f dvT = bl.transpose(dv[i]), dkT = bl.transpose(dk[i]);
 #pragma unroll
                 for (int j = 0; j < ND; ++j) {
                     dMv[i][j] = mm(dvT, ZT[j], dMv[i][j]);
@@ -648,13 +558,13 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
             v4f dz[ND], XT[ND];
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                dz[j] = L.rows_of(&sh.ev[0][16 * j]) * d_epre + L.rows_of(&sh.ev[1][16 * j]) * d_apre;
+                dz[j] = bl.rows_of(&sh.ev[0][16 * j]) * d_epre + bl.rows_of(&sh.ev[1][16 * j]) * d_apre;
 #pragma unroll
                 for (int i = 0; i < ND; ++i) {
                     dz[j] = mm(sh.mem[3][i * ND + j][lane], dv[i], dz[j]);
                     dz[j] = mm(sh.mem[2][i * ND + j][lane], dk[i], dz[j]);
                 }
-                XT[j] = L.transpose(X[j]);
+                XT[j] = bl.transpose(X[j]);
             }
             const int64_t at = x_at(valid ? ch * C + 16 * blk + tau : 0);
 #pragma unroll
@@ -663,7 +573,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
                 for (int i = 0; i < ND; ++i) dx = mm(Gam[i][j], dz[i], dx);
                 if (valid) store_dx(at + 16 * j, dx);
-                const v4f dzT = L.transpose(dz[j]);
+                const v4f dzT = bl.transpose(dz[j]);
 #pragma unroll
                 for (int i = 0; i < ND; ++i) Ep[j][i] = mm(dzT, XT[i], Ep[j][i]);
             }
@@ -682,7 +592,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 for (int i = 0; i < ND; ++i)
 #pragma unroll
                     for (int j = 0; j < ND; ++j)
-                        GT[i][j] = mm(t.De_r * t.KT[i], -RT[j], i == j ? L.diagonal(t.a) : zero);
+                        GT[i][j] = mm(t.d.De_r * t.KT[i], -RT[j], i == j ? bl.diagonal(t.d.a) : zero);
             } else {
                 identity(GT);
                 for (int seg = 0; seg < nseg; ++seg) {
@@ -754,7 +664,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
                         for (int i = 0; i < ND; ++i)
 #pragma unroll
-                            for (int j = 0; j < ND; ++j) H[i][j] = L.transpose(HTb[j][i]);
+                            for (int j = 0; j < ND; ++j) H[i][j] = bl.transpose(HTb[j][i]);
                         v4f KG[ND];
 #pragma unroll
                         for (int j = 0; j < ND; ++j) {
@@ -772,7 +682,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
         // Readout: y = M_m Gamma q^ of every token of the chunk.
         for (int blk = w; blk < nb; blk += W) {
             const int tl = 16 * blk + tau;
-            const int64_t tok = ch * C + tl;
+            const Index tok = ch * C + tl;
             const bool valid = tl < C && tok < N;
             const int64_t at = x_at(valid ? tok : 0), qat = q_at(valid ? tok : 0, at);
             v4f q[ND], dy[ND];
@@ -797,8 +707,8 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 dp[j] = zero;
 #pragma unroll
                 for (int i = 0; i < ND; ++i) dp[j] = mm(sh.mem[4][i * ND + j][lane], dy[i], dp[j]);
-                qT[j] = L.transpose(q[j]);
-                dpT[j] = L.transpose(dp[j]);
+                qT[j] = bl.transpose(q[j]);
+                dpT[j] = bl.transpose(dp[j]);
             }
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
@@ -807,7 +717,7 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
                 for (int i = 0; i < ND; ++i) pT = mm(q[i], GamT[i][j], pT);
 #pragma unroll
                 for (int i = 0; i < ND; ++i) {
-                    dMm[i][j] = mm(L.transpose(dy[i]), pT, dMm[i][j]);
+                    dMm[i][j] = mm(bl.transpose(dy[i]), pT, dMm[i][j]);
                     Ep[i][j] = mm(dpT[i], qT[j], Ep[i][j]);
                 }
             }
@@ -885,13 +795,13 @@ __global__ __launch_bounds__(64 * W, 1) void srnl_backward_blocks_kernel(const B
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float e = row_group_sum<16>(dEv[i][r]), a = row_group_sum<16>(dAv[i][r]);
-            sh.tr[w][16 * i + 4 * g + r] = e;
-            sh.tr[w][D + 16 * i + 4 * g + r] = a;
+            sh.scratch[w].tr[16 * i + 4 * g + r] = e;
+            sh.scratch[w].tr[D + 16 * i + 4 * g + r] = a;
         }
     __syncthreads();
     if (threadIdx.x < 2 * D) {
         float v = 0.f;
-        for (int u = 0; u < W; ++u) v += sh.tr[u][threadIdx.x];
+        for (int u = 0; u < W; ++u) v += sh.scratch[u].tr[threadIdx.x];
         dst[3 * DD + threadIdx.x] = v;
     }
 }

@@ -1,0 +1,177 @@
+// The 16-token block form on the FP32 matrix cores: tile products, token order, decays and
+// triangular solves shared by the few-line scan (srnl_utw.hip) and the backward
+// (srnl_backward_blocks.hip).
+//
+// A tile is 4 registers: lane (g = l / 16, c = l % 16) holds rows 4g..4g+3 of column c, which
+// is what the matrix core returns, the B operand of that matrix and the A operand of its
+// transpose; so mm(A, B) = A^T B needs no data movement, and where a transpose is needed it
+// goes through wave-private LDS.  Token slots are permuted: slot index n stands for time
+// 4 (n % 4) + n / 4 of the block, which puts four consecutive times into one register index,
+// so one rank-4 matrix instruction eliminates them: a 16 x 16 triangular solve is 7
+// instructions, with the 4 x 4 diagonal inverses formed on the VALU (solving by columns on
+// the VALU took about 1,500 cycles against 350).
+#pragma once
+
+#include "srnl_device.h"
+
+namespace vh {
+namespace blocks {
+
+constexpr int kTrStride = 20;   // floats per row of the transpose scratch (16-byte aligned rows)
+
+// acc + A^T B
+__device__ __forceinline__ v4f mm(v4f a, v4f b, v4f acc) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = mfma4(a[j], b[j], acc);
+    return acc;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp0(float v) {   // 0 where the source lane is outside the row
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// Prefix sums over the 16 slots of a block in time order (slot c = time 4 (c % 4) + c / 4),
+// the same in every row of lanes: inclusive, exclusive and the total.
+struct Prefix {
+    float incl, excl, total;
+};
+__device__ __forceinline__ Prefix time_prefix(float v, int c) {
+    float in = v + dpp0<0x114>(v);              // row_shr 4: the previous time of the same group of four
+    in += dpp0<0x118>(in);                      // row_shr 8
+    float t = v + dpp0<0x128>(v);               // row_ror 8, 4: the group's total
+    t += dpp0<0x124>(t);
+    // every lane moves before the selects: a move inside a branch would read inactive lanes
+    const int j = c & 3;
+    const float t1 = dpp0<0x90>(t);             // quad_perm [0, 0, 1, 2]
+    float s = t + (j >= 1 ? t1 : 0.f);
+    const float s2 = dpp0<0x40>(s);             // quad_perm [0, 0, 0, 1]
+    s += j >= 2 ? s2 : 0.f;
+    const float s1 = dpp0<0x90>(s), before = j >= 1 ? s1 : 0.f;
+    return {before + in, before + dpp0<0x114>(in), dpp0<0xFF>(s)};
+}
+
+// Wave-private LDS of a block.
+struct Scratch {
+    float tr[16 * kTrStride];   // transposes
+    float sc[5][16];            // per-slot scalars, read four rows at a time
+    float diag[64];             // the 4 x 4 diagonal blocks of L, negated
+};
+
+// Decays of a block, from eta^ and the retentions of its slots (0 and 1 past the chunk): with
+// a_t the product of the retentions before slot t and a that of all 16,
+//   D_a = diag(a_t), D_e = diag(eta^_t a / a_{t+1}) by column and by row, and M[row][column] =
+//   eta^_s a_t / a_{s+1} for the earlier slot s and the later slot t of the two.
+struct Decays {
+    v4f M, De_r, Da_r;
+    float De, Da, a;
+};
+// L = M . (K^T K) above the diagonal: the symmetric tile -M . (K^T K), and this lane's entry
+// of the inverses of the 4 x 4 diagonal blocks for the lower and the upper solve.
+struct Triangle {
+    v4f nC;
+    float dl, du;
+};
+
+struct Block {
+    Scratch& s;
+    const int lane, g, c, tau;   // tau: time of slot c within the block
+
+    __device__ __forceinline__ Block(Scratch& scratch, int l)
+        : s(scratch), lane(l), g(l >> 4), c(l & 15), tau(4 * (l & 3) + ((l & 15) >> 2)) {}
+
+    __device__ __forceinline__ v4f transpose(v4f v) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s.tr[(4 * g + i) * kTrStride + c] = v[i];
+        __builtin_amdgcn_wave_barrier();
+        const v4f r = *reinterpret_cast<const v4f*>(&s.tr[c * kTrStride + 4 * g]);
+        __builtin_amdgcn_wave_barrier();
+        return r;
+    }
+    __device__ __forceinline__ v4f rows_of(const float* p) const { return *reinterpret_cast<const v4f*>(p + 4 * g); }
+    __device__ __forceinline__ int row_time(int i) const { return 4 * i + g; }
+    __device__ __forceinline__ v4f diagonal(float v) const {   // v I as a tile
+        v4f r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = 4 * g + i == c ? v : 0.f;
+        return r;
+    }
+
+    __device__ __forceinline__ Decays decays(float eff, float alpha) const {
+        Decays d;
+        const Prefix la = time_prefix(__builtin_amdgcn_logf(alpha), c);   // log2
+        d.a = __builtin_amdgcn_exp2f(la.total);
+        d.Da = __builtin_amdgcn_exp2f(la.excl);
+        d.De = eff * __builtin_amdgcn_exp2f(la.total - la.incl);
+        s.sc[0][c] = eff;
+        s.sc[1][c] = la.incl;
+        s.sc[2][c] = la.excl;
+        s.sc[3][c] = d.De;
+        s.sc[4][c] = d.Da;
+        __builtin_amdgcn_wave_barrier();
+        const v4f eff_r = rows_of(s.sc[0]), incl_r = rows_of(s.sc[1]), excl_r = rows_of(s.sc[2]);
+        d.De_r = rows_of(s.sc[3]);
+        d.Da_r = rows_of(s.sc[4]);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool row_first = row_time(i) < tau;
+            const float m = (row_first ? eff_r[i] : eff) *
+                            __builtin_amdgcn_exp2f(row_first ? la.excl - incl_r[i] : excl_r[i] - la.incl);
+            d.M[i] = row_time(i) == tau ? 0.f : m;
+        }
+        return d;
+    }
+
+    __device__ __forceinline__ Triangle triangle(const Decays& d, v4f gram) const {
+        Triangle t;
+        t.nC = -(d.M * gram);
+        // Inverse of the 4 x 4 unit triangle of this slot's group of four times: this lane's
+        // entry is that of times min(g, f), max(g, f) of group c % 4, f = c / 4.
+        const int grp = c & 3, f = c >> 2;
+        s.diag[grp * 16 + 4 * g + f] = grp == 0 ? t.nC[0] : grp == 1 ? t.nC[1] : grp == 2 ? t.nC[2] : t.nC[3];
+        __builtin_amdgcn_wave_barrier();
+        const v4f r0 = *reinterpret_cast<const v4f*>(s.diag + grp * 16);
+        const v4f r1 = *reinterpret_cast<const v4f*>(s.diag + grp * 16 + 4);
+        const v4f r2 = *reinterpret_cast<const v4f*>(s.diag + grp * 16 + 8);
+        __builtin_amdgcn_wave_barrier();
+        // r holds N = -L: (I - N)^-1 = I + N + N^2 + N^3
+        const float t02 = r0[2] + r0[1] * r1[2], t13 = r1[3] + r1[2] * r2[3];
+        const float t03 = r0[3] + r0[1] * t13 + r0[2] * r2[3];
+        const int lo = min(g, f), hi = max(g, f);
+        const float from0 = hi == 1 ? r0[1] : hi == 2 ? t02 : t03, from1 = hi == 2 ? r1[2] : t13;
+        const float inv = lo == 0 ? from0 : lo == 1 ? from1 : r2[3];
+        t.dl = g < f ? inv : 0.f;
+        t.du = f < g ? inv : 0.f;
+        return t;
+    }
+
+    // B <- (I + L^T)^-1 B and B <- (I + L)^-1 B for token-row tiles.
+    template <int ND>
+    __device__ __forceinline__ void solve_lower(const Triangle& t, v4f (&b)[ND]) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float a1 = (c & 3) == k ? t.dl : 0.f, a2 = (c & 3) > k ? t.nC[k] : 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][k], b[j]);
+            if (k < 3)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][k], b[j]);
+        }
+    }
+    template <int ND>
+    __device__ __forceinline__ void solve_upper(const Triangle& t, v4f (&b)[ND]) const {
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+            const float a1 = (c & 3) == k ? t.du : 0.f, a2 = (c & 3) < k ? t.nC[k] : 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; ++j) b[j] = mfma4(a1, b[j][k], b[j]);
+            if (k > 0)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) b[j] = mfma4(a2, b[j][k], b[j]);
+        }
+    }
+};
+
+}  // namespace blocks
+}  // namespace vh
