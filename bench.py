@@ -635,10 +635,12 @@ def main(argv=None):
                    "wall_s_timed_region": round(wall, 3)},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": BF16_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / BF16_PEAK_TFLOPS, 5), "traffic": srnl_bytes,
-                     "kernel": "vh_srnl_spatial_forward (srnl_scan16_ut_kernel + srnl_readout_tile_kernel)",
+                     "kernel": "vh_srnl_spatial_forward (srnl_scan16_utw_kernel, srnl_scan16_ut_kernel at 28x28, "
+                               "+ srnl_readout_tile_kernel)",
                      "scope": "sum over the 29 SRNL launches of one forward (3/4/18/4 blocks at "
                               "56/28/14/7); achieved = reference FLOP count / event-timed duration; "
-                              "peak = dense bf16 MFMA, the only matrix instruction the two kernels issue; "
+                              "peak = dense bf16 MFMA, the instruction of the two kernels' products (the "
+                              "scan's 16 x 16 triangular solves issue FP32 ones); "
                               "traffic = rocprofv3 FETCH_SIZE+WRITE_SIZE bytes, calibrated",
                      "srnl_ms_per_forward": round(srnl_ms_total, 3),
                      "algorithmic_gflop_per_forward": round(srnl_flops_total / 1e9, 2),

@@ -1311,11 +1311,16 @@ void launch_scan(const ScanParams& sp, hipStream_t stream) {
         const Override tb("scan_tb");
         if (tb.set()) token_blocks = tb.as_int() == 1 ? 1 : 2;
         if constexpr (D == 16) {
-            // Few lines: the block form with a chunk's blocks spread over the waves of one
-            // workgroup per line (srnl_utw.hip), unless a dispatch override forces the wide
-            // scan or the stepped form.
+            // One workgroup per line (srnl_utw.hip), unless a dispatch override forces another
+            // form: chunks of one 16-token block at any line count (4,096 lines of 14: 46.7
+            // against 51.7 us, 8,192 of 7: 40.7 against 48.5, 1,024 of 14: 21 against 46), longer
+            // chunks below 2,048 lines (1,024 lines of 56: 179 against 202 us, of 28: 59 against
+            // 96).  From there the waves of a chunk compete for the SIMDs and the packed form
+            // (srnl_ut.hip) is level or ahead: 2,048 lines of 28: 92 against 86 us, of 56: 323
+            // against 322, of 80: 828 against 646; 4,096 of 40: 368 against 345.
             const Override utw("scan_utw");   // "1": whenever the chunks allow, "0": never
-            const bool utw_on = utw.set() ? utw.value[0] == '1' : waves > 0;
+            const bool utw_on = utw.set() ? utw.value[0] == '1'
+                                          : !Override("scan_pack").set() && (max_chunk <= 16 || lines < 2048);
             if (utw_on && scan_ut_enabled() && !Override("scan_wide").set() && launch_scan16_utw<T>(sp, stream))
                 return;
         }

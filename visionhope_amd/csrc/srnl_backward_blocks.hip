@@ -216,15 +216,15 @@ struct Line {
         v4f S[ND], KD[ND];
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
-            S[j] = t.d.De_r * t.KT[j];
-            KD[j] = -(t.d.Da_r * t.KT[j]);
+            S[j] = t.d.De_r() * t.KT[j];
+            KD[j] = -(t.d.Da_r() * t.KT[j]);
         }
         bl.solve_upper(t.tri, S);
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                const v4f start = i == j ? bl.diagonal(t.d.a) : zero;
+                const v4f start = i == j ? bl.diagonal(t.d.a()) : zero;
                 sh.maps[w][0][i * ND + j][bl.lane] = mm(KD[i], S[j], start);
                 if constexpr (ADJOINT) sh.maps[w][1][i * ND + j][bl.lane] = mm(S[i], KD[j], start);
                 sh.maps[w][2][i * ND + j][bl.lane] = mm(-S[i], t.DlT[j], zero);
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
     // R^T from K^T G^T of the block's entry gain (R (I + L) = G K D_a + Delta).
     auto solve_r = [&](const Tok& t, const v4f (&KG)[ND], v4f (&RT)[ND]) {
 #pragma unroll
-        for (int j = 0; j < ND; ++j) RT[j] = t.d.Da_r * KG[j] + t.DlT[j];
+        for (int j = 0; j < ND; ++j) RT[j] = t.d.Da_r() * KG[j] + t.DlT[j];
         bl.solve_lower(t.tri, RT);
     };
 
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
             for (int i = 0; i < ND; ++i)
 #pragma unroll
                 for (int j = 0; j < ND; ++j)
-                    G[i][j] = mm(-RT[i], t.d.De_r * t.KT[j], i == j ? bl.diagonal(t.d.a) : zero);
+                    G[i][j] = mm(-RT[i], t.d.De_r() * t.KT[j], i == j ? bl.diagonal(t.d.a()) : zero);
         } else {
             v4f GT[ND][ND];
             identity(GT);
@@ -485,14 +485,15 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                         else if (i == j) hg += 4 * g + r == c ? HT[i][j][r] : 0.f;
                     }
                 }
-                RbT[j] = -(t.d.De_r * kh);
+                RbT[j] = -(t.d.De_r() * kh);
             }
             bl.solve_upper(t.tri, RbT);
+            const v4f Da_r = t.d.Da_r();
 #pragma unroll
             for (int j = 0; j < ND; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) part += RbT[j][r] * (t.d.Da_r[r] * KG[j][r]);
-            const float phi0 = wave_sum(part + t.d.a * hg);   // <H, G> at the block start
+                for (int r = 0; r < 4; ++r) part += RbT[j][r] * (Da_r[r] * KG[j][r]);
+            const float phi0 = wave_sum(part + t.d.a() * hg);   // <H, G> at the block start
             float rr = 0.f, rd = 0.f;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
@@ -520,7 +521,8 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                 PT = mm(Rb[i], R[i], PT);
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Ws[r] = t.d.M[r] * (bl.row_time(r) < tau ? P[r] : PT[r]);
+            for (int r = 0; r < 4; ++r) Ws[r] = bl.row_time(r) < tau ? P[r] : PT[r];
+            Ws = bl.decayed(t.d, Ws);
             v4f dk[ND], dv[ND], ZT[ND];
             float kdot = 0.f;
 #pragma unroll
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                 }
                 if constexpr (W == 1) gr = Rb[i];
                 const v4f kw = mm(t.KT[i], Ws, zero);
-                dk[i] = gr * t.d.Da - hr * t.d.De - kw + Rb[i] + t.Dl[i] * cdn + t.K[i] * cks;
+                dk[i] = gr * t.d.Da() - hr * t.d.De() - kw + Rb[i] + t.Dl[i] * cdn + t.K[i] * cks;
                 dv[i] = -Rb[i] - t.Dl[i] * cdn;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) kdot += dk[i][r] * t.K[i][r];
@@ -592,7 +594,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                 for (int i = 0; i < ND; ++i)
 #pragma unroll
                     for (int j = 0; j < ND; ++j)
-                        GT[i][j] = mm(t.d.De_r * t.KT[i], -RT[j], i == j ? bl.diagonal(t.d.a) : zero);
+                        GT[i][j] = mm(t.d.De_r() * t.KT[i], -RT[j], i == j ? bl.diagonal(t.d.a()) : zero);
             } else {
                 identity(GT);
                 for (int seg = 0; seg < nseg; ++seg) {

@@ -54,20 +54,36 @@ __device__ __forceinline__ Prefix time_prefix(float v, int c) {
 // Wave-private LDS of a block.
 struct Scratch {
     float tr[16 * kTrStride];   // transposes
-    float sc[5][16];            // per-slot scalars, read four rows at a time
+    float sc[2][16];            // per-slot scalars, read four rows at a time
     float diag[64];             // the 4 x 4 diagonal blocks of L, negated
 };
 
-// Decays of a block, from eta^ and the retentions of its slots (0 and 1 past the chunk): with
-// a_t the product of the retentions before slot t and a that of all 16,
-//   D_a = diag(a_t), D_e = diag(eta^_t a / a_{t+1}) by column and by row, and M[row][column] =
-//   eta^_s a_t / a_{s+1} for the earlier slot s and the later slot t of the two.
+// Decays of a block, from eta^ and the retentions of its slots (0 and 1 past the chunk).  With
+// a_t the product of the retentions before slot t and a = h^2 that of all 16,
+//   rho_s = eta^_s h / a_{s+1},  kappa_t = a_t / h,
+// so eta^_s a_t / a_{s+1} = rho_s kappa_t, D_e = diag(eta^_t a / a_{t+1}) = h rho and D_a =
+// diag(a_t) = h kappa.  Taken about the middle every factor stays inside 2^+-117 for the
+// smallest retention the gate clamps allow.  By column, and for the lane's four rows.
 struct Decays {
-    v4f M, De_r, Da_r;
-    float De, Da, a;
+    v4f rho_r, kappa_r;
+    float rho, kappa, h;
+    __device__ __forceinline__ float De() const { return rho * h; }
+    __device__ __forceinline__ float Da() const { return kappa * h; }
+    __device__ __forceinline__ v4f De_r() const { return rho_r * scalar_h(); }
+    __device__ __forceinline__ v4f Da_r() const { return kappa_r * scalar_h(); }
+    __device__ __forceinline__ float a() const { return h * h; }
+
+private:
+    // The asm keeps the compiler from widening the load of h to a vector, which left the struct
+    // in scratch memory.
+    __device__ __forceinline__ float scalar_h() const {
+        float v = h;
+        asm("" : "+v"(v));
+        return v;
+    }
 };
-// L = M . (K^T K) above the diagonal: the symmetric tile -M . (K^T K), and this lane's entry
-// of the inverses of the 4 x 4 diagonal blocks for the lower and the upper solve.
+// L[s][t] = rho_s kappa_t (k_s . k_t) above the diagonal: the symmetric tile -L - L^T, and this
+// lane's entry of the inverses of the 4 x 4 diagonal blocks for the lower and the upper solve.
 struct Triangle {
     v4f nC;
     float dl, du;
@@ -100,32 +116,35 @@ struct Block {
     __device__ __forceinline__ Decays decays(float eff, float alpha) const {
         Decays d;
         const Prefix la = time_prefix(__builtin_amdgcn_logf(alpha), c);   // log2
-        d.a = __builtin_amdgcn_exp2f(la.total);
-        d.Da = __builtin_amdgcn_exp2f(la.excl);
-        d.De = eff * __builtin_amdgcn_exp2f(la.total - la.incl);
-        s.sc[0][c] = eff;
-        s.sc[1][c] = la.incl;
-        s.sc[2][c] = la.excl;
-        s.sc[3][c] = d.De;
-        s.sc[4][c] = d.Da;
+        const float mid = 0.5f * la.total;
+        d.h = __builtin_amdgcn_exp2f(mid);
+        d.kappa = __builtin_amdgcn_exp2f(la.excl - mid);
+        d.rho = eff * __builtin_amdgcn_exp2f(mid - la.incl);
+        s.sc[0][c] = d.rho;
+        s.sc[1][c] = d.kappa;
         __builtin_amdgcn_wave_barrier();
-        const v4f eff_r = rows_of(s.sc[0]), incl_r = rows_of(s.sc[1]), excl_r = rows_of(s.sc[2]);
-        d.De_r = rows_of(s.sc[3]);
-        d.Da_r = rows_of(s.sc[4]);
+        d.rho_r = rows_of(s.sc[0]);
+        d.kappa_r = rows_of(s.sc[1]);
         __builtin_amdgcn_wave_barrier();
+        return d;
+    }
+    // v scaled by eta^_s a_t / a_{s+1} of the earlier slot s and the later slot t of (row,
+    // column); zero on the diagonal
+    __device__ __forceinline__ v4f decayed(Decays d, v4f v) const {
+        v4f r;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const bool row_first = row_time(i) < tau;
-            const float m = (row_first ? eff_r[i] : eff) *
-                            __builtin_amdgcn_exp2f(row_first ? la.excl - incl_r[i] : excl_r[i] - la.incl);
-            d.M[i] = row_time(i) == tau ? 0.f : m;
+            const float rho_r = d.rho_r[i], kappa_r = d.kappa_r[i], rho = d.rho, kappa = d.kappa;
+            const float first = row_first ? rho_r : rho, second = row_first ? kappa : kappa_r;
+            r[i] = row_time(i) == tau ? 0.f : v[i] * first * second;
         }
-        return d;
+        return r;
     }
 
-    __device__ __forceinline__ Triangle triangle(const Decays& d, v4f gram) const {
+    __device__ __forceinline__ Triangle triangle(Decays d, v4f gram) const {
         Triangle t;
-        t.nC = -(d.M * gram);
+        t.nC = decayed(d, -gram);
         // Inverse of the 4 x 4 unit triangle of this slot's group of four times: this lane's
         // entry is that of times min(g, f), max(g, f) of group c % 4, f = c / 4.
         const int grp = c & 3, f = c >> 2;

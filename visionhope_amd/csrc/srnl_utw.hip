@@ -1,88 +1,98 @@
-// SRNL chunk scan for head_dim 16 (bf16, fp16 or FP32 activations) when the lines are few (fewer than
-// the GPU's 1024 SIMDs: VisionHOPE-Base at 512^2 has 96 to 640 lines per launch, with chunks
-// of 128 down to 16 tokens).  It is the block form of srnl_ut.hip (same algebra, same
-// operand arithmetic) with the blocks of a chunk spread over the waves of a workgroup:
+// SRNL chunk scan for head_dim 16 (bf16, fp16 or FP32 activations) in 16-token blocks, one
+// workgroup per line, one wave per block of a chunk (W = the chunk's blocks rounded up to a
+// power of two, at most 8): every line count with chunks of one block, fewer than 2,048 lines
+// with longer ones (launch_scan in srnl.hip).
 //
-//   * one workgroup per line, W waves (W = the chunk's 16-slot blocks rounded up to a power
-//     of two, at most 8); wave w forms the affine map (X_w, Y_w) of block w of the current
-//     chunk -- token projections, gates, the triangle L, Z = (I + L)^-1 W K^T by back
-//     substitution, X_w = a_15 I - (K D_a) Z, Y_w = -Delta Z -- exactly as srnl_ut.hip forms
-//     one tile's map (reference recurrence: inference_recurrence.cuh:32-135, memory.cuh:
-//     219-233);
-//   * the maps compose in order on wave 0 (srnl_ut.hip's chain): wave 0 forms G^T =
-//     (X_0 + Y_0)^T in registers, the other waves hand X_w and Y_w^T over through LDS, and
-//     G^T <- X_w^T G^T + Y_w^T follows block by block -- one barrier, no transposes (a tree
-//     of log2 W levels measured 3,800 of 8,600 cycles per chunk at W = 8, against about
-//     1,200 for the chain);
-//   * the state S = [M_m; M_v; M_k; e; a; 0] (64 x 16 FP32) lives in LDS; the refresh
-//     S <- S G (the reference's M <- M G and e <- G^T e, a <- G^T a, :119-133) is split over
-//     the waves by 16-row blocks.
+// With Gamma the product of the gains of the chunks so far, the state is S_0 Gamma (reference
+// refresh inference_recurrence.cuh:119-133: M <- M G, e <- G^T e, a <- G^T a), so only the
+// 16 x 16 Gamma is carried: z = Gamma x, k~ = M_k z, v = M_v z and the gate pre-activations
+// e.z, a.z come from the initial memories, which stay in registers.  For a block of 16 slots
+// entered with gain G (D_a, D_e, L: srnl_blocks.h; K the keys, Delta = k - v):
+//   G' = a G - R D_e K^T,  R (I + L) = G K D_a + Delta;   as a map  G' = G X + Y,
+//   X = a I - K D_a S,  Y = -Delta S,  (I + L) S = D_e K^T.
+//   * several blocks per chunk: wave w forms X_w and (Gamma Y_w)^T = -S^T (Gamma Delta)^T;
+//     after one barrier wave 0 chains P <- X_w^T P + (Gamma Y_w)^T from P = Gamma^T, which
+//     ends as the next chunk's Gamma^T, and hands it out through LDS; the last wave stores
+//     the chunk-start content memory M_m Gamma meanwhile;
+//   * one block per chunk (W = 1): the right-hand side is multiplied by Gamma before the
+//     solve, (I + L^T) (Gamma R)^T = D_a K^T Gamma^T + (Gamma Delta)^T, so Gamma'^T =
+//     a Gamma^T - K D_e (Gamma R)^T needs no map.
+// Products run on bf16 operands split hi + lo (x exact when it is bf16), which leave the vector
+// pipe free while they run; the solves are FP32 (v_mfma_f32_16x16x4_f32), which hold it.
+// (Measured: a vector FMA of another wave waits for a 34-cycle FP32 product, not for a bf16
+// one; with FP32 products throughout, two waves on a SIMD did not overlap and 8 waves took
+// 389 us where the split ones take 296.)  Bound by the dependency chain of a chunk.
 //
-// Matrices pass between waves in LDS in the accumulator layout of lane 16 q + j (rows
-// 4q..4q+3 of column j), read back by the lane that wrote them: X_w is then the A operand of
-// X_w^T and Y_w^T the addend, one 16-byte load each.  Slots past the chunk act as the identity.
+// Per launch on MI355X, against the form that carried the whole 64 x 16 state and solved
+// (I + L) by columns on the vector unit: 96 lines of 16,384 tokens (chunks of 128) 370 -> 296
+// us, 64 lines of 600 (30, 20) 64 -> 44, 32 lines of 196 (14) 30 -> 18; against the packed form
+// (srnl_ut.hip): 1,024 lines of 3,136 (56) 202 -> 179, 4,096 of 196 (14) 52 -> 47, 8,192 of 49
+// (7) 48 -> 42.
+#include <algorithm>
+
 #include "srnl_block_form.h"
+#include "srnl_blocks.h"
 
 namespace vh {
-using namespace blockform;
+using namespace blocks;
+using blockform::XQuad;
 
 namespace {
 
-// The wave's own LDS writes become visible to its other lanes (wave-private tables).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// An FP32 tile as bf16 matrix-core operands, |v - hi - lo| <= 2^-16 |v|.
+struct Op {
+    v4s h, l;
+};
+__device__ __forceinline__ Op split(v4f v) {
+    Op o;
+    blockform::split4(v, o.h, o.l);
+    return o;
 }
+// acc + A^T B
+__device__ __forceinline__ v4f mm(const Op& a, const Op& b, v4f acc) { return blockform::mma3(a.h, a.l, b.h, b.l, acc); }
 
-__device__ __forceinline__ void st4(float* p, const v4f& v) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
+__device__ __forceinline__ v4f load4f(const float* p) { return *reinterpret_cast<const v4f*>(p); }
+
+template <int W>
+struct Shared {
+    Scratch scratch[W];
+    float gam[16][kTrStride];                          // Gamma, by rows
+    Op gamT[64];                                       // Gamma^T as a tile, split
+    Op X[W > 1 ? W : 1][W > 1 ? 64 : 1];               // X_w as a tile, split
+    v4f Y[W > 1 ? W : 1][W > 1 ? 64 : 1];              // (Gamma Y_w)^T as a tile
+};
 
 }  // namespace
 
 template <typename T, int W, bool SPATIAL>
-__global__ __launch_bounds__(64 * W) void srnl_scan16_utw_kernel(const ScanParams p) {
+__global__ __launch_bounds__(64 * W, 4) void srnl_scan16_utw_kernel(const ScanParams p) {
+    constexpr int D = 16;
     using XQ = XQuad<T>;
-    // Row strides are padded to 20 floats (keys, L, Z, state, G) so that the 16-byte loads of
-    // 16 lanes down a column of rows fall in different LDS banks; the hand-over maps are read
-    // back by the lane that wrote them, so they are stored lane-major.
-    constexpr int D = 16, DKS = 20, TS = 20, SD = 20;
-    __shared__ __align__(16) float kT[W][D * DKS];    // normalised keys [feature][slot]
-    __shared__ __align__(16) float ndT[W][D * DKS];   // v - k [feature][slot]
-    __shared__ __align__(16) float tk[W][64];         // per slot: rho, kappa, -a_{t-1}, w
-    __shared__ __align__(16) float Lc[W][16 * TS];    // L[s][t] at [t][s]
-    __shared__ __align__(16) float Zs[W][16 * TS];    // Z[s][f] at [f][s]
-    __shared__ __align__(16) float Xt[W][256];        // X_w, accumulator layout, lane-major
-    __shared__ __align__(16) float Yt[W][256];        // Y_w^T, accumulator layout, lane-major
-    __shared__ __align__(16) float St[64 * SD];       // state rows
-    __shared__ __align__(16) float Gr[16 * SD];       // chunk gain G, by rows
+    __shared__ Shared<W> sh;
+    const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const Block bl(sh.scratch[wv], static_cast<int>(threadIdx.x) & 63);
+    const int lane = bl.lane, g = bl.g, c = bl.c;
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
 
-    const int tid = static_cast<int>(threadIdx.x);
-    const int wv = tid >> 6, lane = tid & 63, i16 = lane & 15, q = lane >> 4;
     const int64_t lines = p.B * p.R * p.heads;
     const int64_t line = xcd_remap(blockIdx.x, lines);
     const int64_t head = line % p.heads;
     const int r = static_cast<int>((line / p.heads) % p.R);
     const int64_t b = line / (p.heads * p.R);
     const int64_t sidx = p.per_line_state ? line : r * p.heads + head;
-
-    // initial state: rows 0-15 M_m, 16-31 M_v, 32-47 M_k, 48 e, 49 a, 50-63 zero
-    for (int idx = tid; idx < 16 * D; idx += 64 * W) {
-        const int row = idx >> 2, c4 = (idx & 3) * 4;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row < 16) v = ld4(p.Mm + sidx * D * D + row * D + c4);
-        else if (row < 32) v = ld4(p.Mv + sidx * D * D + (row - 16) * D + c4);
-        else if (row < 48) v = ld4(p.Mk + sidx * D * D + (row - 32) * D + c4);
-        else if (row == 48) v = ld4(p.Me + sidx * D + c4);
-        else if (row == 49) v = ld4(p.Ma + sidx * D + c4);
-        *reinterpret_cast<float4*>(St + row * SD + c4) = v;
-    }
+    // rows c of the memories as tiles N(M^T); entries 4g.. of the gate vectors
+    const Op MkT = split(load4f(p.Mk + (sidx * D + c) * D + 4 * g)), MvT = split(load4f(p.Mv + (sidx * D + c) * D + 4 * g));
+    const v4f Mm_rows = load4f(p.Mm + (sidx * D + c) * D + 4 * g);
+    const Op MmT = split(Mm_rows);
+    // e and a as operand rows 4 j and 4 j + 1, so every lane's registers 0 and 1 end with e.z and a.z
+    const Op gates = split((c & 3) < 2 ? load4f(((c & 1) ? p.Ma : p.Me) + sidx * D + 4 * g) : zero);
 
     const int C = chunk_of(p.chunk, r);
     const int64_t nc = (p.L + C - 1) / C;
     const int nblk = (C + 15) / 16;
-    const T* xcol = static_cast<const T*>(p.x.ptr) + b * p.x.sb + r * p.x.sr + head * p.x.sh + 4 * q;
+    const int slot = 16 * wv + bl.tau;   // this lane's token of a chunk
+    const bool valid = slot < C;         // every chunk but the last is whole, and the last forms no gain
+    const T* xcol = static_cast<const T*>(p.x.ptr) + b * p.x.sb + r * p.x.sr + head * p.x.sh + 4 * g;
     int pa = 0, pb = 0, pc = 0, pst = 0;
     if constexpr (SPATIAL) {
         const int Wd = static_cast<int>(p.x.W), L = static_cast<int>(p.x.H * p.x.W);
@@ -91,212 +101,104 @@ __global__ __launch_bounds__(64 * W) void srnl_scan16_utw_kernel(const ScanParam
         pc = (r & 1) ? L - 1 : 0;
         pst = static_cast<int>(p.x.st);
     }
-    // x of token (chunk cc, slot 16 wv + i16), features 4q..4q+3, as raw bits; slots past the
-    // chunk read the line's first token and are zeroed when decoded
-    auto load_x = [&](int64_t cc, typename XQ::Raw& raw, bool& ok) {
-        const int slot = 16 * wv + i16;
-        const int64_t tok = cc * C + slot;
-        ok = slot < C && tok < p.L;
+    // x of this lane's token of chunk cc as raw bits; slots past the chunk read the line's
+    // first token and are zeroed when decoded
+    auto load_x = [&](int64_t cc) {
         int64_t off = 0;
-        if (ok) {
+        if (valid) {
             if (SPATIAL && p.aligned) off = static_cast<int64_t>(pa * static_cast<int>(cc) + pb * slot + pc) * pst;
-            else off = token_offset<SPATIAL>(p.x, r, tok);
+            else off = token_offset<SPATIAL>(p.x, r, cc * C + slot);
         }
-        raw = XQ::load(xcol + off);
+        return load_xraw<T, 16>(xcol + off);
     };
-    float* const kTw = kT[wv];
-    float* const ndTw = ndT[wv];
-    float* const tkw = tk[wv];
-    float* const Lcw = Lc[wv];
-    float* const Zsw = Zs[wv];
+    // The content memory M_m Gamma the readout of chunk cc uses (M_m itself, unrounded, for the
+    // first): (M_m Gamma)^T, row c and columns 4g.. of M_m Gamma.
+    auto store_content = [&](int64_t cc, v4f gam) {
+        const v4f m = cc == 0 ? Mm_rows : mm(split(gam), MmT, zero);
+        store_state4(p.states + (line * p.max_chunks + cc) * D * D + c * D + 4 * g,
+                     make_float4(m[0], m[1], m[2], m[3]), p.split_states);
+    };
+    auto gamma_rows = [&]() {   // N(Gamma) from its rows in LDS
+        v4f v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = sh.gam[4 * g + i][c];
+        return v;
+    };
 
-    typename XQ::Raw xr{};
-    bool xok = false, have = false;
-    __syncthreads();
-    for (int64_t c = 0; c < nc; ++c) {
-        if (wv == 0)   // chunk-start M_m for the readout
-            store_state4(p.states + (line * p.max_chunks + c) * D * D + i16 * D + 4 * q,
-                         ld4(St + i16 * SD + 4 * q), p.split_states);
-        if (c == nc - 1) break;
-
-        v4f gT = {0.f, 0.f, 0.f, 0.f};   // wave 0: G^T of the blocks composed so far
-        if (wv < nblk) {
-            if (!have) load_x(c, xr, xok);
-            const bool valid = 16 * wv + i16 < C;   // slot inside the chunk (every such token is < L here)
-            // ---- token phase: [M_k; M_v] x and (x.e, x.a) on the matrix cores ----
-            v4s akh, akl, avh, avl, gah, gal;
-            {
-                const float4 mk = ld4(St + (32 + i16) * SD + 4 * q);
-                const float4 mv = ld4(St + (16 + i16) * SD + 4 * q);
-                const float4 g4 = ld4(St + (48 + (i16 & 1)) * SD + 4 * q);
-                const bool on = (i16 & 3) < 2;   // operand rows 4q' + 0 / 4q' + 1: e / a, others zero
-                const float ak[4] = {mk.x, mk.y, mk.z, mk.w};
-                const float av[4] = {mv.x, mv.y, mv.z, mv.w};
-                const float ga[4] = {on ? g4.x : 0.f, on ? g4.y : 0.f, on ? g4.z : 0.f, on ? g4.w : 0.f};
-                split4(ak, akh, akl);
-                split4(av, avh, avl);
-                split4(ga, gah, gal);
-            }
+    v4f gamT = bl.diagonal(1.f), gam = gamT;
+    Op G = split(gamT);
+    XRaw<T, 16> xr{};
+    if (nc > 1 && wv < nblk) xr = load_x(0);
+    for (int64_t ch = 0; ch < nc - 1; ++ch) {
+        v4f K, Dl;
+        if (W == 1 || wv < nblk) {
             v4s xh, xl;
-            XQ::operands(xr, xok, xh, xl);
-            const v4f z4 = {0.f, 0.f, 0.f, 0.f};
-            const v4f kacc = XQ::mma(akh, akl, xh, xl, z4);
-            const v4f vacc = XQ::mma(avh, avl, xh, xl, z4);
-            const v4f gacc = XQ::mma(gah, gal, xh, xl, z4);
-            // the next computing chunk's x, in flight during the rest of this chunk
-            have = c + 1 < nc - 1;
-            if (have) load_x(c + 1, xr, xok);
-            float kn = kacc[0] * kacc[0] + kacc[1] * kacc[1] + kacc[2] * kacc[2] + kacc[3] * kacc[3];
-            kn = xor16_32_sum(kn);
+            XQ::operands(xr, valid, xh, xl);
+            const Op Z = split(XQ::mma(G.h, G.l, xh, xl, zero));
+            if (ch + 1 < nc - 1) xr = load_x(ch + 1);   // in flight during this chunk
+            K = mm(MkT, Z, zero);
+            const v4f V = mm(MvT, Z, zero), pre = mm(gates, Z, zero);
+            float dsq = 0.f;
+            const float kn = xor16_32_sum((K[0] * K[0] + K[1] * K[1]) + (K[2] * K[2] + K[3] * K[3]));
             // ||k||^2 of the normalised key is ||k~||^2 / (||k~||^2 + 1e-6)
             const float inv = rsqrtf(kn + 1e-6f);
-            const float ksq = kn * inv * inv;
-            float kn4[4], dsq = 0.f;
+            K *= inv;
+            Dl = K - V;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float kv = kacc[j] * inv, nd = vacc[j] - kv;
-                kn4[j] = kv;
-                dsq += nd * nd;
-                kTw[(4 * q + j) * DKS + i16] = kv;
-                ndTw[(4 * q + j) * DKS + i16] = nd;
-            }
+            for (int i = 0; i < 4; ++i) dsq += Dl[i] * Dl[i];
             dsq = xor16_32_sum(dsq);
             float alpha, eff;
-            token_gates_fast(p.k, gacc[0], gacc[1], dsq, ksq, alpha, eff);   // every lane: token i16
-            // Per-slot scalars (srnl_ut.hip): cl = inclusive prefix of log2 alpha over the
-            // 16-lane row, a_15 = 2^cl_15, and the triangle's ratio a_{t-1} / a_s split into
-            // rho_s = eta^_s 2^(m - cl_s) and kappa_t = 2^(clx_t - m) about m = cl_15 / 2.
-            const float la = valid ? __builtin_amdgcn_logf(alpha) : 0.f;
-            const float eh = valid ? eff : 0.f;
-            float cl = la;
-            cl += row_shr<1>(cl);
-            cl += row_shr<2>(cl);
-            cl += row_shr<4>(cl);
-            cl += row_shr<8>(cl);
-            const float tot = readlane_f(cl, 15);
-            const float decay = __builtin_amdgcn_exp2f(tot), mid = 0.5f * tot, clx = cl - la;
-            if (lane < 16) {
-                tkw[lane] = eh * __builtin_amdgcn_exp2f(mid - cl);        // rho
-                tkw[16 + lane] = __builtin_amdgcn_exp2f(clx - mid);       // kappa
-                tkw[32 + lane] = -__builtin_amdgcn_exp2f(clx);            // -a_{t-1}
-                tkw[48 + lane] = eh * __builtin_amdgcn_exp2f(tot - cl);   // w
+            token_gates_fast(p.k, pre[0], pre[1], dsq, kn * inv * inv, alpha, eff);
+            const Op k = split(K);
+            const v4f gram = mm(k, k, zero), KT = bl.transpose(K);
+            const v4f gd = mm(split(Dl), G, zero);   // (Gamma Delta)^T
+            const Decays dec = bl.decays(valid ? eff : 0.f, valid ? alpha : 1.f);
+            const Triangle tri = bl.triangle(dec, gram);
+            if constexpr (W == 1) {
+                v4f RT[1] = {mm(k, G, zero) * dec.Da_r() + gd};
+                bl.solve_lower(tri, RT);
+                store_content(ch, gam);
+                gamT = mm(split(-(KT * dec.De_r())), split(RT[0]), gamT * dec.a());
+                G = split(gamT);
+                gam = bl.transpose(gamT);
+            } else {
+                v4f S[1] = {KT * dec.De_r()};
+                bl.solve_upper(tri, S);
+                const Op s = split(-S[0]);
+                sh.X[wv][lane] = split(mm(split(KT * dec.Da_r()), s, bl.diagonal(dec.a())));
+                sh.Y[wv][lane] = mm(s, split(gd), zero);
             }
-            wave_sync();
-            // ---- L = diag(rho) K^T K diag(kappa), strict upper triangle, by columns (the
-            //      Gram tile from the keys split once, scaled after the product) ----
-            {
-                const float kap = tkw[16 + i16];
-                const float4 r4 = ld4(tkw + 4 * q);   // rho of rows 4q..4q+3
-                const float rr[4] = {r4.x, r4.y, r4.z, r4.w};
-                v4s kh, kl;
-                split4(kn4, kh, kl);
-                const v4f P = mma3(kh, kl, kh, kl, v4f{0.f, 0.f, 0.f, 0.f});
-                float lv[4];
+        }
+        if constexpr (W > 1) {
+            __syncthreads();
+            if (wv == 0) {
+                // the next map is in flight while a step runs (past the last block: read, unused)
+                Op X = sh.X[0][lane];
+                v4f Y = sh.Y[0][lane];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) lv[j] = (4 * q + j < i16) ? (P[j] * rr[j]) * kap : 0.f;
-                *reinterpret_cast<float4*>(Lcw + i16 * TS + 4 * q) = make_float4(lv[0], lv[1], lv[2], lv[3]);
-            }
-            wave_sync();
-            // ---- Z = (I + L)^-1 W K^T: lane f (of the first 16) solves column f from the last
-            //      row up, Z[s][f] = w_s k_s[f] - sum_{v > s} L[s][v] Z[v][f] ----
-            if (q == 0) {
-                float acc[16], zc[16];
-#pragma unroll
-                for (int s0 = 0; s0 < 16; s0 += 4) {
-                    const float4 k4 = ld4(kTw + i16 * DKS + s0);
-                    const float4 w4 = ld4(tkw + 48 + s0);
-                    acc[s0] = k4.x * w4.x; acc[s0 + 1] = k4.y * w4.y;
-                    acc[s0 + 2] = k4.z * w4.z; acc[s0 + 3] = k4.w * w4.w;
-                }
-                float lA[4][16], lB[4][16];
-                auto load_group = [&](int v0, float (&buf)[4][16]) {
-#pragma unroll
-                    for (int dv = 0; dv < 4; ++dv)
-#pragma unroll
-                        for (int s0 = 0; s0 < v0 + dv; s0 += 4) {
-                            const float4 l4 = ld4(Lcw + (v0 + dv) * TS + s0);
-                            buf[dv][s0] = l4.x; buf[dv][s0 + 1] = l4.y; buf[dv][s0 + 2] = l4.z; buf[dv][s0 + 3] = l4.w;
-                        }
-                };
-                auto solve_group = [&](int v0, const float (&buf)[4][16]) {
-#pragma unroll
-                    for (int dv = 3; dv >= 0; --dv) {
-                        const int v = v0 + dv;
-                        zc[v] = acc[v];
-#pragma unroll
-                        for (int s2 = 0; s2 < v; ++s2) acc[s2] -= buf[dv][s2] * zc[v];
+                for (int w = 0; w < W; ++w) {
+                    const Op x = X;
+                    const v4f y = Y;
+                    if (w + 1 < W) {
+                        X = sh.X[w + 1][lane];
+                        Y = sh.Y[w + 1][lane];
                     }
-                };
-                load_group(12, lA);
-                load_group(8, lB);
-                solve_group(12, lA);
-                load_group(4, lA);
-                solve_group(8, lB);
-                load_group(0, lB);
-                solve_group(4, lA);
-                solve_group(0, lB);
-#pragma unroll
-                for (int s = 0; s < 16; s += 4)
-                    *reinterpret_cast<float4*>(Zsw + i16 * TS + s) = make_float4(zc[s], zc[s + 1], zc[s + 2], zc[s + 3]);
-            }
-            wave_sync();
-            // ---- the block's map: X = a_15 I - (K D_a) Z, Y = -Delta Z; wave 0 (the first
-            //      block, entered with G = I) keeps (X_0 + Y_0)^T, the others hand over X_w
-            //      and Y_w^T (accumulator layouts) ----
-            {
-                const float4 z4f = ld4(Zsw + i16 * TS + 4 * q);
-                const float4 k4 = ld4(kTw + i16 * DKS + 4 * q);
-                const float4 d4 = ld4(ndTw + i16 * DKS + 4 * q);
-                const float4 a4 = ld4(tkw + 32 + 4 * q);
-                const float zv[4] = {z4f.x, z4f.y, z4f.z, z4f.w};
-                const float nka[4] = {k4.x * a4.x, k4.y * a4.y, k4.z * a4.z, k4.w * a4.w};
-                const float ndl[4] = {d4.x, d4.y, d4.z, d4.w};
-                v4s zh, zl, kah, kal, dlh, dll;
-                split4(zv, zh, zl);
-                if (wv == 0) {
-                    const float nb[4] = {nka[0] + ndl[0], nka[1] + ndl[1], nka[2] + ndl[2], nka[3] + ndl[3]};
-                    v4s nbh, nbl;
-                    split4(nb, nbh, nbl);
-                    gT = mma3(zh, zl, nbh, nbl, diag4(decay, q, i16));   // (X_0 + Y_0)^T
-                } else {
-                    split4(nka, kah, kal);
-                    split4(ndl, dlh, dll);
-                    st4(Xt[wv] + 4 * lane, mma3(kah, kal, zh, zl, diag4(decay, q, i16)));   // X_w
-                    st4(Yt[wv] + 4 * lane, mma3(zh, zl, dlh, dll, v4f{0.f, 0.f, 0.f, 0.f}));  // Y_w^T
+                    if (w < nblk) {
+                        gamT = mm(x, G, y);
+                        G = split(gamT);
+                    }
                 }
+                sh.gamT[lane] = G;
+                *reinterpret_cast<v4f*>(&sh.gam[c][4 * g]) = gamT;
+            } else if (wv == W - 1) {
+                store_content(ch, gam);
             }
+            __syncthreads();
+            if (wv != 0) G = sh.gamT[lane];
+            if (wv == W - 1) gam = gamma_rows();
         }
-        __syncthreads();
-        // ---- composition on wave 0: G^T <- X_w^T G^T + Y_w^T, then G row-major ----
-        if (wv == 0) {
-            for (int w = 1; w < nblk; ++w) {
-                const float4 x4 = ld4(Xt[w] + 4 * lane);   // A operand of X_w^T
-                const float4 y4 = ld4(Yt[w] + 4 * lane);   // Y_w^T
-                const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
-                v4s xh, xl, gh, gl;
-                split4(xv, xh, xl);
-                split4(gT, gh, gl);
-                gT = mma3(xh, xl, gh, gl, v4f{y4.x, y4.y, y4.z, y4.w});
-            }
-            st4(Gr + i16 * SD + 4 * q, gT);   // lane (j, q) holds G[j][4q..4q+3]
-        }
-        __syncthreads();
-        // ---- refresh: S <- S G, one 16-row block per wave ----
-        for (int R = wv; R < 4; R += W) {
-            const float4 s4 = ld4(St + (16 * R + i16) * SD + 4 * q);   // A operand: row 16R + i16
-            const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
-            float gv[4];                                              // B operand: column i16 of G
-#pragma unroll
-            for (int k = 0; k < 4; ++k) gv[k] = Gr[(4 * q + k) * SD + i16];
-            v4s sh, sl, gh, gl;
-            split4(sv, sh, sl);
-            split4(gv, gh, gl);
-            const v4f sn = mma3(sh, sl, gh, gl, v4f{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int k = 0; k < 4; ++k) St[(16 * R + 4 * q + k) * SD + i16] = sn[k];
-        }
-        __syncthreads();
     }
+    if (wv == W - 1) store_content(nc - 1, gam);
 }
 
 // Waves per line of the few-line block-form scan: the chunk's 16-slot blocks rounded up to
