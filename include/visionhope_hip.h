@@ -191,20 +191,34 @@ int vh_srnl_backward(
     float* dM_alpha, int64_t B, int64_t R, int64_t heads, int64_t N, int32_t head_dim, const int64_t* chunks,
     const vh_srnl_consts* consts, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Backward of vh_srnl_spatial_forward: x, q [B, H, W, C] (io_dtype), dout [B, H, W, C] fp32
- * the gradient of its output, the same memories (one state per direction and head), skip,
- * direction weights and chunks.  Outputs: dx, dq [B, H, W, C] in io_dtype (each direction's
- * part rounded to io_dtype, the four summed in fp32), and fp32 gradients of the memories,
- * of d_skip (its own layout) and of dir_weight [4, C].  head_dim 16 or 32, chunks in
- * [1, 256].  No counterpart in the reference's native code, which restores and fuses the
- * directions in separate passes (operator.py:88-145). */
+/* The scan of a training step on maps x [B, H, W, C] (io_dtype), FP32 products throughout:
+ * gains (vh_srnl_spatial_gains_bytes), the products of the chunk gains that
+ * vh_srnl_spatial_backward starts from, and in workspace (vh_srnl_workspace_bytes of the
+ * B * 4 * C / head_dim lines) the chunk-start memories that vh_srnl_spatial_readout reads,
+ * as vh_srnl_spatial_scan leaves them.  head_dim 16 or 32, chunks in [1, 256]. */
+size_t vh_srnl_spatial_gains_bytes(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim,
+                                   const int64_t* chunks);
+int vh_srnl_spatial_gains(
+    const void* x, int32_t io_dtype, const float* M_m, const float* M_v, const float* M_k, const float* M_eta,
+    const float* M_alpha, int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim, const int64_t chunks[4],
+    const vh_srnl_consts* consts, float* gains, size_t gains_bytes, void* workspace, size_t workspace_bytes,
+    void* stream);
+
+/* Backward of the spatial operator (vh_srnl_spatial_gains and vh_srnl_spatial_readout to
+ * fp32): x, q [B, H, W, C] (io_dtype), dout [B, H, W, C] fp32 the gradient of its output, the
+ * same memories (one state per direction and head), skip, direction weights and chunks, and
+ * the gains of the forward.  Outputs: dx, dq [B, H, W, C] in io_dtype (each direction's part
+ * rounded to io_dtype, the four summed in fp32), and fp32 gradients of the memories, of
+ * d_skip (its own layout) and of dir_weight [4, C].  head_dim 16 or 32, chunks in [1, 256].
+ * No counterpart in the reference's native code, which restores and fuses the directions
+ * in separate passes (operator.py:88-145). */
 size_t vh_srnl_spatial_backward_workspace_bytes(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim,
                                                 int32_t io_dtype, const int64_t* chunks);
 int vh_srnl_spatial_backward(
     const void* x, const void* q, int32_t io_dtype, const float* dout, const float* M_m, const float* M_v,
     const float* M_k, const float* M_eta, const float* M_alpha, const float* d_skip, int32_t skip_per_direction,
-    const float* dir_weight, void* dx, void* dq, float* dM_m, float* dM_v, float* dM_k, float* dM_eta,
-    float* dM_alpha, float* dd_skip, float* ddir_weight, int64_t B, int64_t H, int64_t W, int64_t C,
+    const float* dir_weight, const float* gains, void* dx, void* dq, float* dM_m, float* dM_v, float* dM_k,
+    float* dM_eta, float* dM_alpha, float* dd_skip, float* ddir_weight, int64_t B, int64_t H, int64_t W, int64_t C,
     int32_t head_dim, const int64_t chunks[4], const vh_srnl_consts* consts, void* workspace,
     size_t workspace_bytes, void* stream);
 

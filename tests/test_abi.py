@@ -326,7 +326,7 @@ def test_srnl_spatial_backward_validates(lib):
     def call(head_dim=16, chunk=4, C=32, H=4, dtype=hip.VH_DTYPE_F32, nbytes=None, x=p):
         arr, keep = hip.int64_array([chunk] * 4)
         size = lib.vh_srnl_spatial_backward_workspace_bytes(1, H, 4, C, head_dim, dtype, arr)
-        rc = lib.vh_srnl_spatial_backward(x, p, dtype, p, p, p, p, p, p, p, 0, p, p, p, p, p, p, p, p, p, p,
+        rc = lib.vh_srnl_spatial_backward(x, p, dtype, p, p, p, p, p, p, p, 0, p, p, p, p, p, p, p, p, p, p, p,
                                           1, H, 4, C, head_dim, arr, _consts(), p,
                                           size if nbytes is None else nbytes, None)
         return size, rc

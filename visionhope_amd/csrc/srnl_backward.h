@@ -20,6 +20,7 @@ struct BwdParams {
     float* dline;       // [lines, 3 D^2 + 2 D] per-line gradient of the initial state
     float* states;      // small head dims: [lines, nc, 3 D^2 + 2 D] chunk-start states;
                         // block form: [lines, nc, D^2] products of the chunk gains before each chunk
+                        // (from the first chunk on; written by the gains kernel)
     float* gtraj;       // small head dims: [lines, CMAX, D, D] gain trajectory of the current chunk;
                         // block form: [lines, waves, segments, D^2] segment-start gains (chunks of several segments)
     int64_t B, R, heads, N, nc;
@@ -31,10 +32,12 @@ struct BwdParams {
     // (x and q io dtype, dy the FP32 gradient of the fused output), R = 4 scan orders; dx and
     // dq become four planes of such maps in the io dtype, one per direction, and the M_m part
     // of dline the gradient for unit direction weights.
-    const float* scale;   // [4, heads * D] direction weights; null: packed lines
+    const float* scale;   // [4, heads * D] direction weights; null: packed lines (backward kernel)
     int64_t H, W;
     float inv_h;
     void *dx_planes, *dq_planes;
+    float* content;       // gains kernel: chunk-start M_m for the readout, or null
+    int content_split;    // stored as bf16 hi + lo pairs (store_state4)
 };
 
 // d(eta^)/d(cap) of eta^ = cap (1 - exp(-u)), u = eta / cap: (1 - e^-u) - u e^-u, by its
@@ -48,6 +51,7 @@ __device__ __forceinline__ float softcap_dcap(float u, float e_neg) {
 // of 16 * waves tokens that chunk takes.
 int bwd_block_waves(int head_dim, int64_t max_chunk);
 inline int bwd_block_segs(int waves, int64_t max_chunk) { return static_cast<int>((max_chunk + 16 * waves - 1) / (16 * waves)); }
+int launch_backward_gains(const BwdParams& p, bool spatial, int head_dim, int waves, int64_t lines, hipStream_t stream);
 int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream);
 
 }  // namespace vh

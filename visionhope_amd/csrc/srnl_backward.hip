@@ -659,11 +659,32 @@ SpatialBwdLayout spatial_bwd_layout(int64_t B, int64_t H, int64_t W, int64_t C, 
     l.blocks = std::max<int64_t>(1, std::min<int64_t>(1024, (pixels + 4 * rows - 1) / (4 * rows)));
     auto round = [](size_t v) { return (v + 255) / 256 * 256; };
     const size_t plane = round(static_cast<size_t>(4 * pixels * C) * (io_dtype == VH_DTYPE_F32 ? 4 : 2));
-    l.dx_planes = round(l.lines.total);
+    l.dx_planes = round((l.lines.traj + l.lines.dline) * sizeof(float));   // the gains are the caller's
     l.dq_planes = l.dx_planes + plane;
     l.parts = l.dq_planes + plane;
     l.total = l.parts + round(static_cast<size_t>(l.blocks * C) * sizeof(float));
     return l;
+}
+
+// Arguments of the spatial training entries.
+int check_spatial_args(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim, int32_t io_dtype,
+                       const int64_t* chunks, const vh_srnl_consts* consts) {
+    VH_REQUIRE(B > 0 && H > 0 && W > 0 && C > 0, VH_ERR_SHAPE, "spatial SRNL training needs nonempty [B, H, W, C]");
+    const int rc = check_srnl_consts(consts);
+    if (rc) return rc;
+    VH_REQUIRE(head_dim == 16 || head_dim == 32, VH_ERR_HEAD_DIM,
+               "spatial SRNL training supports head_dim 16 and 32; got %d", head_dim);
+    VH_REQUIRE(C % head_dim == 0, VH_ERR_SHAPE, "C=%lld is not a multiple of head_dim=%d", (long long)C, head_dim);
+    VH_REQUIRE(H * W < (int64_t(1) << 24), VH_ERR_SHAPE, "spatial SRNL supports H*W < 2^24 pixels, got %lld",
+               (long long)(H * W));
+    VH_REQUIRE(valid_dtype(io_dtype), VH_ERR_DTYPE, "unsupported io dtype code %d", io_dtype);
+    for (int r = 0; r < 4; ++r)
+        VH_REQUIRE(chunks[r] > 0 && chunks[r] <= kBwdLongChunk, VH_ERR_ARG,
+                   "SRNL backward chunk lengths must be in [1, %d], got %lld", kBwdLongChunk, (long long)chunks[r]);
+    const BwdLayout l = bwd_layout(B, 4, C / head_dim, H * W, head_dim, chunks);
+    VH_REQUIRE(l.lines * l.nc * l.sd < (int64_t(1) << 40) && l.lines < (int64_t(1) << 31), VH_ERR_SHAPE,
+               "SRNL backward problem too large");
+    return VH_OK;
 }
 
 int launch_backward_reduce(const float* dline, int64_t batch, int64_t S, int32_t head_dim, float* dM_m, float* dM_v,
@@ -767,6 +788,8 @@ int vh_srnl_backward(const void* x, const void* q, int32_t io_dtype, int32_t q_r
     };
     int rc;
     if (head_dim >= 16) {
+        rc = launch_backward_gains(bp, false, head_dim, lay.waves, lay.lines, s);
+        if (rc) return rc;
         rc = launch_backward_blocks(bp, head_dim, lay.waves, lay.lines, s);
     } else {
         if (head_dim == 4) by_type(std::integral_constant<int, 4>{});
@@ -779,6 +802,41 @@ int vh_srnl_backward(const void* x, const void* q, int32_t io_dtype, int32_t q_r
     return launch_backward_reduce(bp.dline, batch, S, head_dim, dM_m, dM_v, dM_k, dM_eta, dM_alpha, s);
 }
 
+size_t vh_srnl_spatial_gains_bytes(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim,
+                                   const int64_t* chunks) {
+    return spatial_bwd_layout(B, H, W, C, head_dim, VH_DTYPE_F32, chunks).lines.states * sizeof(float);
+}
+
+int vh_srnl_spatial_gains(const void* x, int32_t io_dtype, const float* M_m, const float* M_v, const float* M_k,
+                          const float* M_eta, const float* M_alpha, int64_t B, int64_t H, int64_t W, int64_t C,
+                          int32_t head_dim, const int64_t chunks[4], const vh_srnl_consts* consts, float* gains,
+                          size_t gains_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    VH_REQUIRE(x && M_m && M_v && M_k && M_eta && M_alpha && chunks && consts && gains && workspace, VH_ERR_ARG,
+               "spatial SRNL gains pointers must not be null");
+    {
+        const int rc = check_spatial_args(B, H, W, C, head_dim, io_dtype, chunks, consts);
+        if (rc) return rc;
+    }
+    const SpatialBwdLayout lay = spatial_bwd_layout(B, H, W, C, head_dim, io_dtype, chunks);
+    const size_t content = static_cast<size_t>(lay.lines.lines * lay.lines.nc) * head_dim * head_dim * sizeof(float);
+    VH_REQUIRE(gains_bytes >= lay.lines.states * sizeof(float) && workspace_bytes >= content, VH_ERR_WORKSPACE,
+               "spatial SRNL gains need %zu and %zu bytes, got %zu and %zu", lay.lines.states * sizeof(float), content,
+               gains_bytes, workspace_bytes);
+    BwdParams bp{};
+    bp.x = x;
+    bp.m0[0] = M_m; bp.m0[1] = M_v; bp.m0[2] = M_k; bp.m0[3] = M_eta; bp.m0[4] = M_alpha;
+    bp.states = gains;
+    bp.content = static_cast<float*>(workspace);
+    bp.content_split = io_dtype == VH_DTYPE_BF16 ? 1 : 0;   // the readout's format (state_split_bf16)
+    bp.B = B; bp.R = 4; bp.heads = C / head_dim; bp.N = H * W; bp.nc = lay.lines.nc;
+    bp.segs = lay.lines.segs;
+    bp.io_dtype = io_dtype; bp.q_raw = 1;
+    for (int r = 0; r < 4; ++r) bp.chunk[r] = static_cast<int>(chunks[r]);
+    bp.k = *consts;
+    bp.H = H; bp.W = W; bp.inv_h = 1.0f / static_cast<float>(H);
+    return launch_backward_gains(bp, true, head_dim, lay.lines.waves, lay.lines.lines, static_cast<hipStream_t>(stream));
+}
+
 size_t vh_srnl_spatial_backward_workspace_bytes(int64_t B, int64_t H, int64_t W, int64_t C, int32_t head_dim,
                                                 int32_t io_dtype, const int64_t* chunks) {
     if (!valid_dtype(io_dtype)) return 0;
@@ -787,41 +845,29 @@ size_t vh_srnl_spatial_backward_workspace_bytes(int64_t B, int64_t H, int64_t W,
 
 int vh_srnl_spatial_backward(const void* x, const void* q, int32_t io_dtype, const float* dout, const float* M_m,
                              const float* M_v, const float* M_k, const float* M_eta, const float* M_alpha,
-                             const float* d_skip, int32_t skip_per_direction, const float* dir_weight, void* dx,
-                             void* dq, float* dM_m, float* dM_v, float* dM_k, float* dM_eta, float* dM_alpha,
+                             const float* d_skip, int32_t skip_per_direction, const float* dir_weight,
+                             const float* gains, void* dx, void* dq, float* dM_m, float* dM_v, float* dM_k, float* dM_eta, float* dM_alpha,
                              float* dd_skip, float* ddir_weight, int64_t B, int64_t H, int64_t W, int64_t C,
                              int32_t head_dim, const int64_t chunks[4], const vh_srnl_consts* consts, void* workspace,
                              size_t workspace_bytes, void* stream) {
-    VH_REQUIRE(x && q && dout && M_m && M_v && M_k && M_eta && M_alpha && d_skip && dir_weight && dx && dq && dM_m &&
+    VH_REQUIRE(x && q && dout && M_m && M_v && M_k && M_eta && M_alpha && d_skip && dir_weight && gains && dx && dq && dM_m &&
                    dM_v && dM_k && dM_eta && dM_alpha && dd_skip && ddir_weight && chunks && consts,
                VH_ERR_ARG, "spatial SRNL backward pointers must not be null");
-    VH_REQUIRE(B > 0 && H > 0 && W > 0 && C > 0, VH_ERR_SHAPE, "spatial SRNL backward needs nonempty [B, H, W, C]");
     {
-        const int rc = check_srnl_consts(consts);
+        const int rc = check_spatial_args(B, H, W, C, head_dim, io_dtype, chunks, consts);
         if (rc) return rc;
     }
-    VH_REQUIRE(head_dim == 16 || head_dim == 32, VH_ERR_HEAD_DIM,
-               "spatial SRNL backward supports head_dim 16 and 32; got %d", head_dim);
-    VH_REQUIRE(C % head_dim == 0, VH_ERR_SHAPE, "C=%lld is not a multiple of head_dim=%d", (long long)C, head_dim);
-    VH_REQUIRE(H * W < (int64_t(1) << 24), VH_ERR_SHAPE, "spatial SRNL supports H*W < 2^24 pixels, got %lld",
-               (long long)(H * W));
-    VH_REQUIRE(valid_dtype(io_dtype), VH_ERR_DTYPE, "unsupported io dtype code %d", io_dtype);
-    for (int r = 0; r < 4; ++r)
-        VH_REQUIRE(chunks[r] > 0 && chunks[r] <= kBwdLongChunk, VH_ERR_ARG,
-                   "SRNL backward chunk lengths must be in [1, %d], got %lld", kBwdLongChunk, (long long)chunks[r]);
     const SpatialBwdLayout lay = spatial_bwd_layout(B, H, W, C, head_dim, io_dtype, chunks);
     VH_REQUIRE(workspace && workspace_bytes >= lay.total, VH_ERR_WORKSPACE,
                "spatial SRNL backward workspace needs %zu bytes, got %zu", lay.total,
                workspace ? workspace_bytes : (size_t)0);
-    VH_REQUIRE(lay.lines.lines * lay.lines.nc * lay.lines.sd < (int64_t(1) << 40) && lay.lines.lines < (int64_t(1) << 31),
-               VH_ERR_SHAPE, "SRNL backward problem too large");
     char* const ws = static_cast<char*>(workspace);
     BwdParams bp{};
     bp.x = x; bp.q = q; bp.dy = dout;
     bp.m0[0] = M_m; bp.m0[1] = M_v; bp.m0[2] = M_k; bp.m0[3] = M_eta; bp.m0[4] = M_alpha;
-    bp.states = reinterpret_cast<float*>(ws);
-    bp.gtraj = bp.states + lay.lines.states;
-    bp.dline = bp.states + lay.lines.states + lay.lines.traj;
+    bp.states = const_cast<float*>(gains);
+    bp.gtraj = reinterpret_cast<float*>(ws);
+    bp.dline = bp.gtraj + lay.lines.traj;
     bp.dx_planes = ws + lay.dx_planes;
     bp.dq_planes = ws + lay.dq_planes;
     bp.B = B; bp.R = 4; bp.heads = C / head_dim; bp.N = H * W; bp.nc = lay.lines.nc;

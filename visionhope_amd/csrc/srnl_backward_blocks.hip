@@ -26,13 +26,18 @@
 // segment of a chunk (W = 1, 2, 4 or 8 waves; longer chunks take several segments).  Tiles,
 // slot order and solves: srnl_blocks.h.
 //
-// Bound: the dependency chain.  A chunk is one serial chain of solves and products per line,
-// and the chunks of a line follow one another; the compulsory matrix work and the bytes take
-// well under a tenth of the time.  Times on MI355X against the token-by-token kernel (which
-// head_dim 4 and 8 still run): 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 305 us;
-// 512 lines of 3,136 tokens, d = 16, chunks of 56: 24,500 -> 802 us; 48 lines of 960 tokens,
-// d = 32, chunks of 40 and 24: 11,800 -> 769 us; 4 lines of 196 tokens, d = 32, chunks of 64:
-// 1,690 -> 77 us.
+// Two kernels: the gains kernel runs the forward and leaves Gamma before every chunk (a training
+// step on maps runs it as its forward, so its backward starts there; packed lines run it ahead of
+// the backward), the backward kernel takes the chunks in reverse.
+//
+// Bound: the dependency chain of a chunk, and within it the issue of the FP32 products, which
+// hold the vector pipe (34 cycles each, srnl_utw.hip); the bytes take under a tenth of the time.
+// Times on MI355X against the token-by-token kernel (which head_dim 4 and 8 still run), gains +
+// backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 80 + 192 us; 512 lines of
+// 3,136 tokens, d = 16, chunks of 56: 24,500 -> 183 + 536 us; 48 lines of 960 tokens, d = 32,
+// chunks of 40 and 24: 11,800 -> 174 + 558 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
+// -> 19 + 57 us.  With the forward repeated inside the backward kernel the first three took 249,
+// 710 and 745 us after a separate forward scan of 54, 125 and 130 us.
 #include <algorithm>
 #include <cmath>
 
@@ -105,16 +110,17 @@ struct Tokens {
     float dn, inv_denom, cap, deff_deta, deff_dcap, deff_dalpha, deff_dksq, s_eta, s_alpha;
 };
 
-template <int D, int W>
+template <int D, typename SharedT>
 struct Line {
     static constexpr int ND = D / 16;
-    Shared<D, W>& sh;
+    SharedT& sh;
     const int w;
     const Block bl;
     const vh_srnl_consts& k;
 
     // Keys, values and gates of the block from x (channel rows; zero in slots past the
     // chunk) and Gamma^T.  Slots past the chunk act as the identity.
+    template <bool DELTA_T = true>
     __device__ __forceinline__ void tokens(const v4f (&X)[ND], bool valid, const v4f (&GamT)[ND][ND],
                                            Tokens<ND>& t) const {
         const v4f zero = {0.f, 0.f, 0.f, 0.f};
@@ -205,12 +211,11 @@ struct Line {
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
             t.KT[i] = bl.transpose(t.K[i]);
-            t.DlT[i] = bl.transpose(t.Dl[i]);
+            if constexpr (DELTA_T) t.DlT[i] = bl.transpose(t.Dl[i]);
         }
     }
 
-    // The block's maps into slot w of the segment's table: X, Y^T, and X^T for the adjoint.
-    template <bool ADJOINT>
+    // The block's maps into slot w of the segment's table: X, X^T for the adjoint, Y^T.
     __device__ __forceinline__ void store_maps(const Tokens<ND>& t) const {
         const v4f zero = {0.f, 0.f, 0.f, 0.f};
         v4f S[ND], KD[ND];
@@ -226,7 +231,7 @@ struct Line {
             for (int j = 0; j < ND; ++j) {
                 const v4f start = i == j ? bl.diagonal(t.d.a()) : zero;
                 sh.maps[w][0][i * ND + j][bl.lane] = mm(KD[i], S[j], start);
-                if constexpr (ADJOINT) sh.maps[w][1][i * ND + j][bl.lane] = mm(S[i], KD[j], start);
+                sh.maps[w][1][i * ND + j][bl.lane] = mm(S[i], KD[j], start);
                 sh.maps[w][2][i * ND + j][bl.lane] = mm(-S[i], t.DlT[j], zero);
             }
     }
@@ -273,6 +278,232 @@ struct Line {
     }
 };
 
+// Token addresses of one line: element offsets of this lane's first channel in x (and dy, dx)
+// and in q (and dq).
+template <int D, bool SPATIAL>
+struct LineAddress {
+    static constexpr int ND = D / 16;
+    using Index = std::conditional_t<SPATIAL, int, int64_t>;   // a map has fewer than 2^24 pixels
+    const Index N;
+    int64_t xbase, qbase, qstride;
+    int r_dir;
+    uint32_t height, width, channels;
+    float inv_h;
+
+    __device__ __forceinline__ LineAddress(const BwdParams& p, int64_t ln, int g) : N(static_cast<Index>(p.N)) {
+        const int64_t b = ln / (p.R * p.heads), head = ln % p.heads, all = p.heads * D;
+        r_dir = static_cast<int>((ln / p.heads) % p.R);
+        xbase = (SPATIAL ? b * N * all + head * D : ln * N * D) + 4 * g;
+        qbase = SPATIAL ? xbase : p.q_raw ? (b * p.R + r_dir) * N * all + head * D + 4 * g : xbase;
+        qstride = p.q_raw ? all : D;
+        height = static_cast<uint32_t>(p.H);
+        width = static_cast<uint32_t>(p.W);
+        channels = static_cast<uint32_t>(all);
+        inv_h = p.inv_h;
+    }
+    // Pixel of scan index t (scan_to_pixel in 32 bits).
+    __device__ __forceinline__ uint32_t pixel(int t) const {
+        const uint32_t orig = static_cast<uint32_t>((r_dir & 1) ? static_cast<int>(N) - 1 - t : t);
+        if (r_dir < 2) return orig;
+        uint32_t col, row;
+        divmod24(orig, height, inv_h, col, row);
+        return row * width + col;
+    }
+    __device__ __forceinline__ int64_t x(Index t) const {
+        if constexpr (SPATIAL) return xbase + static_cast<int64_t>(pixel(t)) * channels;
+        else return xbase + t * D;
+    }
+    __device__ __forceinline__ int64_t q(Index t, int64_t x_offset) const {
+        if constexpr (SPATIAL) return x_offset;
+        else return qbase + t * qstride;
+    }
+    // x of token slot tl of the chunk starting at token `start`, zero past the chunk.
+    __device__ __forceinline__ bool load_tokens(const BwdParams& p, Index start, int tl, int C, v4f (&X)[ND]) const {
+        const Index t = start + tl;
+        const bool valid = tl < C && t < N;
+        const int64_t at = x(valid ? t : 0);
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            X[i] = v4f{0.f, 0.f, 0.f, 0.f};
+            if (valid) X[i] = load_io4(p.x, at + 16 * i, p.io_dtype);
+        }
+        return valid;
+    }
+};
+
+template <int D, int W>
+struct GainShared {
+    static constexpr int ND = D / 16, NT = ND * ND;
+    v4f mem[3][NT][64];                // N(M^T) of M_k, M_v, M_m
+    float ev[2][D];
+    float gam[D][D + 4];               // Gamma, by rows
+    Scratch scratch[W];
+    v4f maps[W > 1 ? W : 1][W > 1 ? 2 : 1][NT][64];   // X and (Gamma Y)^T of the segment's blocks
+};
+
+// The forward of the training path: Gamma before every chunk (for the backward) and the
+// chunk-start content memories M_m Gamma (for the readout), in FP32 products throughout.
+// Waves hold the blocks of a chunk; the first D / 16 waves chain the maps, one column tile of
+// Gamma^T each: P <- X^T P + (Gamma Y)^T from P = Gamma^T (srnl_utw.hip).
+template <int D, int W, bool SPATIAL>
+__global__ __launch_bounds__(64 * W, (D == 16 ? 4 : 1)) void srnl_backward_gains_kernel(const BwdParams p) {
+    constexpr int ND = D / 16, NT = ND * ND, DD = D * D;
+    __shared__ GainShared<D, W> sh;
+    const int w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const Line<D, GainShared<D, W>> L{sh, w, Block(sh.scratch[w], static_cast<int>(threadIdx.x) & 63), p.k};
+    const Block& bl = L.bl;
+    const int lane = bl.lane, g = bl.g, c = bl.c, tau = bl.tau;
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+
+    const int64_t ln = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t RH = p.R * p.heads, s = p.per_line ? ln : ln % RH;
+    const LineAddress<D, SPATIAL> at(p, ln, g);
+    using Index = typename LineAddress<D, SPATIAL>::Index;
+    const int C = chunk_of(p.chunk, at.r_dir);
+    const Index nc = (at.N + C - 1) / C;
+    const int nb = (C + 15) / 16, nseg = (nb + W - 1) / W;
+    float* const my_gam = p.states + ln * p.nc * DD;
+    float* const my_content = p.content ? p.content + ln * p.nc * DD : nullptr;
+
+    for (int t = w; t < 3 * NT; t += W) {
+        const int m = t / NT, i = (t % NT) / ND, j = t % ND;
+        sh.mem[m][t % NT][lane] =
+            *reinterpret_cast<const v4f_any*>(p.m0[2 - m] + s * DD + (16 * j + c) * D + 16 * i + 4 * g);
+    }
+    if (threadIdx.x < 2 * D)
+        sh.ev[threadIdx.x / D][threadIdx.x % D] = p.m0[3 + threadIdx.x / D][s * D + threadIdx.x % D];
+    __syncthreads();
+
+    v4f GamT[ND][ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+        for (int j = 0; j < ND; ++j) GamT[i][j] = i == j ? bl.diagonal(1.f) : zero;
+    // Tiles of (M_m Gamma)^T, spread over the waves from the last: row 16 j + c, columns
+    // 16 i + 4 g.. of M_m Gamma (M_m itself for the first chunk).
+    auto store_content = [&](Index ch) {
+        if (my_content == nullptr) return;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+                if (W - 1 - (i * ND + j) % W == w) {
+                    v4f m = zero;
+                    if (ch == 0) m = sh.mem[2][i * ND + j][lane];
+                    else
+#pragma unroll
+                        for (int k = 0; k < ND; ++k) {
+                            v4f gam;
+                            if constexpr (W == 1) gam = bl.transpose(GamT[i][k]);
+                            else
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) gam[r] = sh.gam[16 * k + 4 * g + r][16 * i + c];
+                            m = mm(gam, sh.mem[2][k * ND + j][lane], m);
+                        }
+                    store_state4(my_content + static_cast<int64_t>(ch) * DD + (16 * j + c) * D + 16 * i + 4 * g,
+                                 make_float4(m[0], m[1], m[2], m[3]), p.content_split != 0);
+                }
+    };
+    for (Index ch = 0; ch < nc - 1; ++ch) {
+        store_content(ch);
+        float* const out = my_gam + static_cast<int64_t>(ch + 1) * DD;
+        if constexpr (W == 1) {
+            v4f X[ND], RT[ND], next[ND][ND];
+            Tokens<ND> t;
+            const bool valid = at.load_tokens(p, ch * C, tau, C, X);
+            L.tokens(X, valid, GamT, t);
+#pragma unroll
+            for (int j = 0; j < ND; ++j) RT[j] = t.d.Da_r() * t.KT[j] + t.DlT[j];
+            bl.solve_lower(t.tri, RT);
+            // Gamma^T <- G^T Gamma^T, G = a I - R D_e K^T
+            v4f G[ND][ND];
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j)
+                    G[i][j] = mm(-RT[i], t.d.De_r() * t.KT[j], i == j ? bl.diagonal(t.d.a()) : zero);
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) {
+                    next[i][j] = zero;
+#pragma unroll
+                    for (int m = 0; m < ND; ++m) next[i][j] = mm(G[m][i], GamT[m][j], next[i][j]);
+                }
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j) {
+                    GamT[i][j] = next[i][j];
+                    *reinterpret_cast<v4f_any*>(out + (16 * j + c) * D + 16 * i + 4 * g) = next[i][j];
+                }
+        } else {
+            v4f P[ND];   // waves below ND: column tile w of the chained Gamma^T
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+                if (w == j)
+#pragma unroll
+                    for (int i = 0; i < ND; ++i) P[i] = GamT[i][j];
+            for (int seg = 0; seg < nseg; ++seg) {
+                const int nbs = min(W, nb - seg * W);
+                if (seg > 0) __syncthreads();   // the previous segment's maps are read
+                if (w < nbs) {
+                    v4f X[ND], S[ND], KD[ND], gd[ND];
+                    Tokens<ND> t;
+                    const bool valid = at.load_tokens(p, ch * C, 16 * (seg * W + w) + tau, C, X);
+                    L.template tokens<false>(X, valid, GamT, t);
+#pragma unroll
+                    for (int j = 0; j < ND; ++j) {
+                        S[j] = t.d.De_r() * t.KT[j];
+                        KD[j] = -(t.d.Da_r() * t.KT[j]);
+                        gd[j] = zero;   // (Gamma Delta)^T
+#pragma unroll
+                        for (int i = 0; i < ND; ++i) gd[j] = mm(t.Dl[i], GamT[i][j], gd[j]);
+                    }
+                    bl.solve_upper(t.tri, S);
+#pragma unroll
+                    for (int i = 0; i < ND; ++i)
+#pragma unroll
+                        for (int j = 0; j < ND; ++j) {
+                            sh.maps[w][0][i * ND + j][lane] = mm(KD[i], S[j], i == j ? bl.diagonal(t.d.a()) : zero);
+                            sh.maps[w][1][i * ND + j][lane] = mm(-S[i], gd[j], zero);
+                        }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < ND; ++j)
+                    if (w == j)
+                        for (int blk = 0; blk < nbs; ++blk) {
+                            v4f next[ND];
+#pragma unroll
+                            for (int i = 0; i < ND; ++i) {
+                                next[i] = sh.maps[blk][1][i * ND + j][lane];
+#pragma unroll
+                                for (int m = 0; m < ND; ++m) next[i] = mm(sh.maps[blk][0][m * ND + i][lane], P[m], next[i]);
+                            }
+#pragma unroll
+                            for (int i = 0; i < ND; ++i) P[i] = next[i];
+                        }
+            }
+#pragma unroll
+            for (int j = 0; j < ND; ++j)
+                if (w == j)
+#pragma unroll
+                    for (int i = 0; i < ND; ++i) {
+                        *reinterpret_cast<v4f*>(&sh.gam[16 * j + c][16 * i + 4 * g]) = P[i];
+                        *reinterpret_cast<v4f_any*>(out + (16 * j + c) * D + 16 * i + 4 * g) = P[i];
+                    }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int j = 0; j < ND; ++j)
+                    GamT[i][j] = *reinterpret_cast<const v4f*>(&sh.gam[16 * j + c][16 * i + 4 * g]);
+        }
+    }
+    store_content(nc - 1);
+}
+
 template <int ND>
 __device__ __forceinline__ void copy_tiles(const v4f (&from)[ND][ND], v4f (&to)[ND][ND]) {
 #pragma unroll
@@ -291,7 +522,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
     using Tok = Tokens<ND>;
     __shared__ Shared<D, W> sh;
     const int w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const Line<D, W> L{sh, w, Block(sh.scratch[w], static_cast<int>(threadIdx.x) & 63), p.k};
+    const Line<D, Shared<D, W>> L{sh, w, Block(sh.scratch[w], static_cast<int>(threadIdx.x) & 63), p.k};
     const Block& bl = L.bl;
     const int lane = bl.lane, g = bl.g, c = bl.c, tau = bl.tau;
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
@@ -299,34 +530,18 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
     const int64_t ln = blockIdx.x;
     const int64_t RH = p.R * p.heads, s = p.per_line ? ln : ln % RH;
     const int r_dir = static_cast<int>((ln / p.heads) % p.R);
-    const int64_t b = ln / RH, head = ln % p.heads;
+    const int64_t head = ln % p.heads;
     const int C = chunk_of(p.chunk, r_dir);
-    using Index = std::conditional_t<SPATIAL, int, int64_t>;   // a map has fewer than 2^24 pixels
-    const Index N = static_cast<Index>(p.N), nc = (N + C - 1) / C;
+    const LineAddress<D, SPATIAL> at_(p, ln, g);
+    using Index = typename LineAddress<D, SPATIAL>::Index;
+    const Index N = at_.N, nc = (N + C - 1) / C;
     const int nb = (C + 15) / 16, nseg = (nb + W - 1) / W;
-    // Element offsets of token t (this lane's first channel): of x, dy and dx, and of q and dq.
     const bool q_raw = SPATIAL || p.q_raw;
     const int64_t C_all = p.heads * D;
-    const int64_t xbase = (SPATIAL ? b * N * C_all + head * D : ln * N * D) + 4 * g;
-    const int64_t qbase = SPATIAL ? xbase : p.q_raw ? (b * p.R + r_dir) * N * C_all + head * D + 4 * g : xbase;
-    // Pixel of scan index t (scan_to_pixel in 32 bits).
-    auto pixel_of = [&](int t) {
-        const uint32_t orig = static_cast<uint32_t>((r_dir & 1) ? static_cast<int>(p.N) - 1 - t : t);
-        if (r_dir < 2) return orig;
-        uint32_t col, row;
-        divmod24(orig, static_cast<uint32_t>(p.H), p.inv_h, col, row);
-        return row * static_cast<uint32_t>(p.W) + col;
-    };
-    auto x_at = [&](Index t) {
-        if constexpr (SPATIAL) return xbase + static_cast<int64_t>(pixel_of(t)) * static_cast<uint32_t>(C_all);
-        else return xbase + t * D;
-    };
-    auto q_at = [&](Index t, int64_t x_off) {
-        if constexpr (SPATIAL) return x_off;
-        else return qbase + t * (p.q_raw ? C_all : D);
-    };
+    auto x_at = [&](Index t) { return at_.x(t); };
+    auto q_at = [&](Index t, int64_t x_off) { return at_.q(t, x_off); };
     const int64_t plane = SPATIAL ? r_dir * p.B * N * C_all : 0;
-    float* const my_gam = p.states + ln * p.nc * DD;
+    const float* const my_gam = p.states + ln * p.nc * DD;
     float* const my_seg = p.gtraj + (ln * W + w) * static_cast<int64_t>(p.segs) * DD;
 
     // ---- memories into LDS -------------------------------------------------------------
@@ -347,15 +562,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
     __syncthreads();
 
     auto load_x = [&](Index ch, int blk, bool& valid, v4f (&X)[ND]) {
-        const int tl = 16 * blk + tau;
-        const Index t = ch * C + tl;
-        valid = tl < C && t < N;
-        const int64_t at = x_at(valid ? t : 0);
-#pragma unroll
-        for (int i = 0; i < ND; ++i) {
-            X[i] = zero;
-            if (valid) X[i] = load_io4(p.x, at + 16 * i, p.io_dtype);
-        }
+        valid = at_.load_tokens(p, ch * C, 16 * blk + tau, C, X);
     };
     auto store_dx = [&](int64_t at, v4f v) {
         if constexpr (SPATIAL) store_io4(p.dx_planes, plane + at, p.io_dtype, v);
@@ -374,69 +581,9 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
         bl.solve_lower(t.tri, RT);
     };
 
-    // ---- 1. forward: Gamma before every chunk ------------------------------------------
     v4f GamT[ND][ND];
-    identity(GamT);
-    for (Index ch = 0; ch < nc - 1; ++ch) {
-        v4f G[ND][ND];
-        if constexpr (W == 1) {
-            v4f X[ND], RT[ND];
-            bool valid;
-            Tok t;
-            load_x(ch, 0, valid, X);
-            L.tokens(X, valid, GamT, t);
-            solve_r(t, t.KT, RT);
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-#pragma unroll
-                for (int j = 0; j < ND; ++j)
-                    G[i][j] = mm(-RT[i], t.d.De_r() * t.KT[j], i == j ? bl.diagonal(t.d.a()) : zero);
-        } else {
-            v4f GT[ND][ND];
-            identity(GT);
-            for (int seg = 0; seg < nseg; ++seg) {
-                const int nbs = min(W, nb - seg * W);
-                if (w < nbs) {
-                    v4f X[ND];
-                    bool valid;
-                    Tok t;
-                    load_x(ch, seg * W + w, valid, X);
-                    L.tokens(X, valid, GamT, t);
-                    L.template store_maps<false>(t);
-                }
-                __syncthreads();
-                for (int blk = 0; blk < nbs; ++blk) L.apply_map(blk, GT);
-                __syncthreads();
-            }
-#pragma unroll
-            for (int i = 0; i < ND; ++i)
-#pragma unroll
-                for (int j = 0; j < ND; ++j) G[i][j] = bl.transpose(GT[j][i]);
-        }
-        // Gamma^T <- G^T Gamma^T
-        v4f next[ND][ND];
-#pragma unroll
-        for (int i = 0; i < ND; ++i)
-#pragma unroll
-            for (int j = 0; j < ND; ++j) {
-                next[i][j] = zero;
-#pragma unroll
-                for (int m = 0; m < ND; ++m) next[i][j] = mm(G[m][i], GamT[m][j], next[i][j]);
-            }
-#pragma unroll
-        for (int i = 0; i < ND; ++i)
-#pragma unroll
-            for (int j = 0; j < ND; ++j) {
-                GamT[i][j] = next[i][j];
-                // row 16 j + c of Gamma, columns 16 i + 4 g ..
-                if ((i * ND + j) % W == w)
-                    *reinterpret_cast<v4f_any*>(my_gam + static_cast<int64_t>(ch + 1) * DD + (16 * j + c) * D + 16 * i +
-                                            4 * g) = next[i][j];
-            }
-    }
-    __syncthreads();   // Gamma of every chunk is written (each wave reads all of it below)
 
-    // ---- 2. chunks in reverse ----------------------------------------------------------
+    // ---- chunks in reverse -------------------------------------------------------------
     v4f dMm[ND][ND], dMv[ND][ND], dMk[ND][ND], dEv[ND], dAv[ND];
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -607,7 +754,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                     if (w < nbs) {
                         load_x(ch, seg * W + w, valid, X);
                         L.tokens(X, valid, GamT, t);
-                        L.template store_maps<true>(t);
+                        L.store_maps(t);
                     }
                     __syncthreads();
                     for (int blk = 0; blk < nbs; ++blk) {
@@ -649,7 +796,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                         if (w < nbs) {
                             load_x(ch, seg * W + w, valid, X);
                             L.tokens(X, valid, GamT, t);
-                            L.template store_maps<true>(t);
+                            L.store_maps(t);
                         }
                         __syncthreads();
                         for (int blk = 0; blk < w; ++blk) L.apply_map(blk, GTb);   // a segment with a successor is full
@@ -767,7 +914,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
         __syncthreads();
     }
 
-    // ---- 3. the line's gradient of its initial memories ----------------------------------
+    // ---- the line's gradient of its initial memories -------------------------------------
     float* const dst = p.dline + ln * SD;
     auto store_matrix = [&](int m, const v4f (&M)[ND][ND]) {
         if constexpr (W > 1) {
@@ -819,26 +966,43 @@ int bwd_block_waves(int head_dim, int64_t max_chunk) {
     return w;
 }
 
-int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream) {
-    auto go = [&](auto d, auto w) {
-        constexpr int D = decltype(d)::value, W = decltype(w)::value;
-        const dim3 grid(static_cast<unsigned>(lines)), block(64 * W);
-        if (p.scale) hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, false>), grid, block, 0, stream, p);
-    };
+namespace {
+
+template <typename F>
+void by_shape(int head_dim, int waves, F&& go) {
     auto by_waves = [&](auto d) {
-        constexpr int D = decltype(d)::value;
         switch (waves) {
             case 1: go(d, std::integral_constant<int, 1>{}); break;
             case 2: go(d, std::integral_constant<int, 2>{}); break;
             case 4: go(d, std::integral_constant<int, 4>{}); break;
             default:
-                if constexpr (D == 16) go(d, std::integral_constant<int, 8>{});
+                if constexpr (decltype(d)::value == 16) go(d, std::integral_constant<int, 8>{});
                 break;
         }
     };
     if (head_dim == 16) by_waves(std::integral_constant<int, 16>{});
     else by_waves(std::integral_constant<int, 32>{});
+}
+
+}  // namespace
+
+int launch_backward_gains(const BwdParams& p, bool spatial, int head_dim, int waves, int64_t lines, hipStream_t stream) {
+    by_shape(head_dim, waves, [&](auto d, auto w) {
+        constexpr int D = decltype(d)::value, W = decltype(w)::value;
+        const dim3 grid(static_cast<unsigned>(lines)), block(64 * W);
+        if (spatial) hipLaunchKernelGGL((srnl_backward_gains_kernel<D, W, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((srnl_backward_gains_kernel<D, W, false>), grid, block, 0, stream, p);
+    });
+    return check_launch("srnl_backward_gains_kernel");
+}
+
+int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream) {
+    by_shape(head_dim, waves, [&](auto d, auto w) {
+        constexpr int D = decltype(d)::value, W = decltype(w)::value;
+        const dim3 grid(static_cast<unsigned>(lines)), block(64 * W);
+        if (p.scale) hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((srnl_backward_blocks_kernel<D, W, false>), grid, block, 0, stream, p);
+    });
     return check_launch("srnl_backward_blocks_kernel");
 }
 

@@ -1,10 +1,10 @@
 """The four-direction operator on channels-last maps, with autograd.
 
 ``srnl_spatial`` is what a training step of the operator runs where the spatial kernels
-apply: the forward is the inference scan and fused readout (``vh_srnl_spatial_forward``),
-which read x and the queries at their pixels, and the backward
-(``vh_srnl_spatial_backward``) writes the gradients at their pixels and sums the four
-directions in one pass.  The packed path it replaces serialises x and the queries into
+apply: a scan in FP32 products that keeps the chunk gains (``vh_srnl_spatial_gains``), the
+fused readout of the inference path, and a backward (``vh_srnl_spatial_backward``) that
+starts from those gains, all reading and writing maps at their pixels; the four directions'
+gradients are summed in one pass.  The packed path it replaces serialises x and the queries into
 four scan orders, scans, reads out, restores and fuses in separate passes (reference
 ``operator.py:88-145``), each with its transposed pass in the backward.
 """
@@ -12,7 +12,7 @@ four scan orders, scans, reads out, restores and fuses in separate passes (refer
 import torch
 
 from .chunk import BACKWARD_MAX_CHUNK, _float_memories, srnl_consts
-from .fused import srnl_spatial_inference
+from .fused import srnl_spatial_inference, srnl_spatial_readout, srnl_spatial_workspace
 from ...utils import hip
 from ...utils.cuda import on_tensor_device
 
@@ -37,20 +37,41 @@ class SpatialSRNLFunction(torch.autograd.Function):
         if torch.jit.is_tracing():
             raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
         memories = (M_m_0, M_v_0, M_k_0, M_eta_0, M_alpha_0)
-        ctx.save_for_backward(*memories, x, q, d_skip, weights)
+        out, gains = srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks)
+        ctx.save_for_backward(*memories, x, q, d_skip, weights, gains)
         ctx.chunks = chunks
-        return srnl_spatial_inference(memories, x, q, d_skip, weights, chunks)
+        return out
 
     @staticmethod
     def backward(ctx, dout):
-        *memories, x, q, d_skip, weights = ctx.saved_tensors
-        return (*srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, dout), None)
+        *memories, x, q, d_skip, weights, gains = ctx.saved_tensors
+        return (*srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, gains, dout), None)
 
 
 @on_tensor_device
-def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, dout):
-    """Gradients of ``SpatialSRNLFunction`` for the output gradient ``dout [B, H, W, C]``:
-    the five memories, x, q, d_skip and the weights, each shaped and typed like its input."""
+def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
+    """The operator's output ``[B, H, W, C]`` FP32 and the gains its backward starts from."""
+    batch, height, width, channels = x.shape
+    head_dim = memories[0].shape[-1]
+    heads = channels // head_dim
+    states, _ = _float_memories(memories, 4, heads, head_dim, batch * 4 * heads)
+    x_c = x.contiguous()
+    lib = hip.load_library()
+    chunk_ptr, _keep = hip.int64_array(chunks)
+    gains = hip.workspace(lib.vh_srnl_spatial_gains_bytes(batch, height, width, channels, head_dim, chunk_ptr), x.device)
+    ws = srnl_spatial_workspace(x_c, head_dim, chunks)
+    hip.check(lib.vh_srnl_spatial_gains(
+        hip.ptr(x_c), hip.dtype_code(x.dtype), *[hip.ptr(m) for m in states], batch, height, width, channels, head_dim,
+        chunk_ptr, srnl_consts(), hip.ptr(gains), gains.numel() * 4, hip.ptr(ws), ws.numel() * 4,
+        hip.stream_of(x_c)), "vh_srnl_spatial_gains")
+    return srnl_spatial_readout(ws, x_c, q, d_skip, weights, chunks, head_dim), gains
+
+
+@on_tensor_device
+def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
+    """Gradients of ``SpatialSRNLFunction`` for the output gradient ``dout [B, H, W, C]`` and
+    the ``gains`` of its forward: the five memories, x, q, d_skip and the weights, each
+    shaped and typed like its input."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
     heads = channels // head_dim
@@ -71,7 +92,7 @@ def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, dout):
     ws = hip.workspace(nbytes, x.device)
     hip.check(lib.vh_srnl_spatial_backward(
         hip.ptr(x_c), hip.ptr(q_c), io, hip.ptr(g), *[hip.ptr(m) for m in states], hip.ptr(skip),
-        int(skip.numel() == 4 * channels), hip.ptr(wts), hip.ptr(dx), hip.ptr(dq), *[hip.ptr(m) for m in dmem],
+        int(skip.numel() == 4 * channels), hip.ptr(wts), hip.ptr(gains), hip.ptr(dx), hip.ptr(dq), *[hip.ptr(m) for m in dmem],
         hip.ptr(dskip), hip.ptr(dweights), batch, height, width, channels, head_dim, chunk_ptr, srnl_consts(),
         hip.ptr(ws), ws.numel() * 4, hip.stream_of(x_c)), "vh_srnl_spatial_backward")
     grads = [d.view(m.shape).to(m.dtype) for d, m in zip(dmem, memories)]
@@ -82,4 +103,9 @@ def srnl_spatial(memories, x_nhwc, q_nhwc, d_skip, weights, chunks):
     """Differentiable spatial operator (``spatial_training_supported``)."""
     if weights.shape != (4, x_nhwc.shape[-1]) or d_skip.numel() not in (weights.numel(), x_nhwc.shape[-1]):
         raise RuntimeError("d_skip must contain C or 4*C values and the direction weights 4*C")
+    if not (torch.is_grad_enabled() and any(t.requires_grad for t in (*memories, x_nhwc, q_nhwc, d_skip, weights))):
+        # nothing to differentiate: the inference scan, which keeps nothing
+        if torch.jit.is_tracing():
+            raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
+        return srnl_spatial_inference(memories, x_nhwc, q_nhwc, d_skip, weights, chunks)
     return SpatialSRNLFunction.apply(*memories, x_nhwc, q_nhwc, d_skip, weights, tuple(int(c) for c in chunks))

@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "vh_dwconv2d_nhwc_forward", "vh_dwconv2d_add_layernorm2d_forward", "vh_grn_scale_forward", "vh_pointwise_add_layernorm_nhwc_forward", "vh_pointwise_chain_nhwc_forward", "vh_pointwise_conv_nhwc_forward",
     "vh_bias_act_nhwc_forward", "vh_dwconv2d_gelu_grn_workspace_bytes", "vh_dwconv2d_gelu_grn_forward",
     "vh_conv3x3_nhwc_forward", "vh_srnl_backward_workspace_bytes", "vh_srnl_backward",
+    "vh_srnl_spatial_gains_bytes", "vh_srnl_spatial_gains",
     "vh_srnl_spatial_backward_workspace_bytes", "vh_srnl_spatial_backward",
     "vh_postprocess_scale_backward_workspace_bytes", "vh_postprocess_scale_backward",
     "vh_grn_backward_workspace_bytes", "vh_grn_backward", "vh_layernorm2d_backward_workspace_bytes",
@@ -88,9 +89,12 @@ _SIGNATURES = {
     "vh_srnl_backward": (ctypes.c_int, [
         _vp, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
         _i64, _i64, _i64, _i64, _i32, _I64P, _CP, _vp, _sz, _vp]),
+    "vh_srnl_spatial_gains_bytes": (_sz, [_i64, _i64, _i64, _i64, _i32, _I64P]),
+    "vh_srnl_spatial_gains": (ctypes.c_int, [
+        _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _I64P, _CP, _vp, _sz, _vp, _sz, _vp]),
     "vh_srnl_spatial_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i32, _i32, _I64P]),
     "vh_srnl_spatial_backward": (ctypes.c_int, [
-        _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+        _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
         _i64, _i64, _i64, _i64, _i32, _I64P, _CP, _vp, _sz, _vp]),
     "vh_postprocess_scale_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i32, _i32]),
     "vh_postprocess_scale_backward": (ctypes.c_int, [
