@@ -222,6 +222,19 @@ int vh_srnl_spatial_backward(
     int32_t head_dim, const int64_t chunks[4], const vh_srnl_consts* consts, void* workspace,
     size_t workspace_bytes, void* stream);
 
+/* A linear layer out = x weight^T + bias in training, on the rows of channels-last maps
+ * (nn.Linear under autocast: operator.py:77, no native counterpart in the reference).
+ * vh_linear_operands casts weight [N, K] and bias [N] (dtype) to what its bf16 products take:
+ * w16 [N, K] and wt16 [K, N] bf16, b32 [N] FP32 holding bf16-rounded values.  The products are
+ * vh_pointwise_conv_nhwc_forward with w16, b32 (out) and with wt16 (dx).
+ * vh_linear_weight_grad: dw [N, K] = dy^T x and db [N] = sum dy in FP32 from bf16 dy [M, N],
+ * x [M, K]; N, K multiples of 16. */
+int vh_linear_operands(const void* weight, const void* bias, int32_t dtype, int64_t N, int64_t K, void* w16,
+                       void* wt16, float* b32, void* stream);
+size_t vh_linear_weight_grad_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int vh_linear_weight_grad(const void* dy, const void* x, int64_t M, int64_t N, int64_t K, float* dw, float* db,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* The reference's fused spatial entry with its own argument layout: X and
  * Q_raw are the serialized stacks [B, 4, H*W, C]; Out is [B, H, W, C] fp32;
  * chunks are (W, W, H, H).  Replaces srnl_line_forward_seq_noatomic

@@ -22,7 +22,8 @@ from torch.nn import functional as F
 from torch.nn.init import trunc_normal_
 
 from .srnl import SRNL
-from .srnl_core.spatial import spatial_training_supported, srnl_spatial
+from .srnl_core.spatial import (projected_training_supported, spatial_training_supported, srnl_spatial,
+                                srnl_spatial_projected)
 from ..utils.cached_params import linear_weights
 from ..utils.cuda import on_tensor_device
 from ..utils.direction_fusion import visionhope_postprocess_scale
@@ -168,22 +169,29 @@ class VisionHOPEOperator(nn.Module):
         """Packed scan of the serialized orders, then the native restoring fusion.  With
         ``memories`` (the inference sequence path) the scan is the gradient-free entry."""
         batch, _, height, width = x.shape
-        seq_hw = x.flatten(2).transpose(1, 2)
+        seq_hw = None
         if memories is None and self._spatial_training_ok():
-            q_hw = self.W_q(seq_hw)
             chunks = self.srnl._chunk_lengths((height, width))
-            if spatial_training_supported(x, q_hw, self.head_dim, chunks):
-                states = self.srnl._validate_memories(x.device)
-                x_nhwc = x.permute(0, 2, 3, 1).contiguous()
-                if x_nhwc.data_ptr() == x.data_ptr() and not self.W_q.weight.requires_grad:
-                    x_nhwc = x_nhwc.clone()   # nothing else keeps x for the backward: the caller may overwrite it
-                out = srnl_spatial(states, x_nhwc,
-                                   q_hw.reshape(batch, height, width, self.dim), self.d_skip.float(),
-                                   self.direction_weights().float(), chunks).permute(0, 3, 1, 2)
-                return out.contiguous(memory_format=torch.channels_last if channels_last
-                                      else torch.contiguous_format)
+            x_nhwc, out = x.permute(0, 2, 3, 1), None
+            if self._projection_fused(x, x_nhwc, chunks):
+                out = srnl_spatial_projected(self.srnl._validate_memories(x.device), x_nhwc.contiguous(), self.W_q,
+                                             self.d_skip.float(), self.direction_weights().float(), chunks)
+            else:
+                seq_hw = x.flatten(2).transpose(1, 2)
+                q_hw = self.W_q(seq_hw)
+                if spatial_training_supported(x, q_hw, self.head_dim, chunks):
+                    states = self.srnl._validate_memories(x.device)
+                    x_nhwc = x_nhwc.contiguous()
+                    if x_nhwc.data_ptr() == x.data_ptr() and not self.W_q.weight.requires_grad:
+                        x_nhwc = x_nhwc.clone()   # nothing else keeps x for the backward: the caller may overwrite it
+                    out = srnl_spatial(states, x_nhwc, q_hw.reshape(batch, height, width, self.dim),
+                                       self.d_skip.float(), self.direction_weights().float(), chunks)
+            if out is not None:
+                return out.permute(0, 3, 1, 2).contiguous(
+                    memory_format=torch.channels_last if channels_last else torch.contiguous_format)
             queries = scan_orders(q_hw, height, width)
         else:
+            seq_hw = x.flatten(2).transpose(1, 2)
             queries = self.project_queries(seq_hw, height, width)
         lines = scan_orders(seq_hw, height, width)
         lines = lines.reshape(batch, 4, height * width, self.num_heads, self.head_dim).transpose(2, 3).contiguous()
@@ -204,6 +212,15 @@ class VisionHOPEOperator(nn.Module):
         return (type(self.srnl) is SRNL and type(self).project_queries is VisionHOPEOperator.project_queries
                 and "project_queries" not in self.__dict__ and "forward" not in self.srnl.__dict__
                 and not _observed(self.srnl))
+
+    def _projection_fused(self, x, x_nhwc, chunks):
+        """Whether a training step runs ``W_q`` inside the spatial Function: a plain Linear
+        whose calls nothing watches, with everything differentiable in the usual case (its
+        weight trained, so that autograd's own linear would keep x as it is, too)."""
+        return (torch.is_grad_enabled() and type(self.W_q) is nn.Linear and "forward" not in self.W_q.__dict__
+                and not _observed(self.W_q) and self.W_q.bias is not None and self.W_q.weight.requires_grad
+                and spatial_training_supported(x, x, self.head_dim, chunks)
+                and projected_training_supported(x_nhwc, self.W_q))
 
     def _merge_weights(self):
         """FP32 merge weights for the inference kernels (no autograd)."""

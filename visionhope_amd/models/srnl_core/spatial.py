@@ -11,10 +11,11 @@ four scan orders, scans, reads out, restores and fuses in separate passes (refer
 
 import torch
 
-from .chunk import BACKWARD_MAX_CHUNK, _float_memories, srnl_consts
+from .chunk import BACKWARD_MAX_CHUNK, srnl_consts
 from .fused import srnl_spatial_inference, srnl_spatial_readout, srnl_spatial_workspace
 from ...utils import hip
 from ...utils.cuda import on_tensor_device
+from ...utils.pointwise import EPI_ADD, EPI_BIAS
 
 # Head dims of the block-form backward.
 SPATIAL_BACKWARD_HEAD_DIMS = (16, 32)
@@ -48,21 +49,25 @@ class SpatialSRNLFunction(torch.autograd.Function):
         return (*srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, gains, dout), None)
 
 
+def _fp32(t):
+    """``t`` as contiguous FP32, itself where it is."""
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().float().contiguous()
+
+
 @on_tensor_device
 def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
     """The operator's output ``[B, H, W, C]`` FP32 and the gains its backward starts from."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
-    heads = channels // head_dim
-    states, _ = _float_memories(memories, 4, heads, head_dim, batch * 4 * heads)
+    states = [_fp32(m) for m in memories]
     x_c = x.contiguous()
     lib = hip.load_library()
     chunk_ptr, _keep = hip.int64_array(chunks)
     gains = hip.workspace(lib.vh_srnl_spatial_gains_bytes(batch, height, width, channels, head_dim, chunk_ptr), x.device)
     ws = srnl_spatial_workspace(x_c, head_dim, chunks)
     hip.check(lib.vh_srnl_spatial_gains(
-        hip.ptr(x_c), hip.dtype_code(x.dtype), *[hip.ptr(m) for m in states], batch, height, width, channels, head_dim,
-        chunk_ptr, srnl_consts(), hip.ptr(gains), gains.numel() * 4, hip.ptr(ws), ws.numel() * 4,
+        x_c.data_ptr(), hip.dtype_code(x.dtype), *[m.data_ptr() for m in states], batch, height, width, channels,
+        head_dim, chunk_ptr, srnl_consts(), gains.data_ptr(), gains.numel() * 4, ws.data_ptr(), ws.numel() * 4,
         hip.stream_of(x_c)), "vh_srnl_spatial_gains")
     return srnl_spatial_readout(ws, x_c, q, d_skip, weights, chunks, head_dim), gains
 
@@ -74,15 +79,11 @@ def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
     shaped and typed like its input."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
-    heads = channels // head_dim
-    states, _ = _float_memories(memories, 4, heads, head_dim, batch * 4 * heads)
-    x_c, q_c = x.contiguous(), q.contiguous()
-    g = dout.float().contiguous()
-    skip = d_skip.detach().float().contiguous()
-    wts = weights.detach().float().contiguous()
+    states = [_fp32(m) for m in memories]
+    x_c, q_c, g = x.contiguous(), q.contiguous(), _fp32(dout)
+    skip, wts = _fp32(d_skip), _fp32(weights)
     dx, dq = torch.empty_like(x_c), torch.empty_like(q_c)
-    dmem = [torch.empty_like(m) for m in states]
-    dskip, dweights = torch.empty_like(skip), torch.empty_like(wts)
+    grads = [torch.empty_like(t) for t in (*states, skip, wts)]
     lib = hip.load_library()
     chunk_ptr, _keep = hip.int64_array(chunks)
     io = hip.dtype_code(x.dtype)
@@ -91,21 +92,110 @@ def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
         raise ValueError(f"spatial SRNL backward does not cover head_dim={head_dim} with chunks {tuple(chunks)}")
     ws = hip.workspace(nbytes, x.device)
     hip.check(lib.vh_srnl_spatial_backward(
-        hip.ptr(x_c), hip.ptr(q_c), io, hip.ptr(g), *[hip.ptr(m) for m in states], hip.ptr(skip),
-        int(skip.numel() == 4 * channels), hip.ptr(wts), hip.ptr(gains), hip.ptr(dx), hip.ptr(dq), *[hip.ptr(m) for m in dmem],
-        hip.ptr(dskip), hip.ptr(dweights), batch, height, width, channels, head_dim, chunk_ptr, srnl_consts(),
-        hip.ptr(ws), ws.numel() * 4, hip.stream_of(x_c)), "vh_srnl_spatial_backward")
-    grads = [d.view(m.shape).to(m.dtype) for d, m in zip(dmem, memories)]
-    return (*grads, dx, dq, dskip.view(d_skip.shape).to(d_skip.dtype), dweights.view(weights.shape).to(weights.dtype))
+        x_c.data_ptr(), q_c.data_ptr(), io, g.data_ptr(), *[m.data_ptr() for m in states], skip.data_ptr(),
+        int(skip.numel() == 4 * channels), wts.data_ptr(), gains.data_ptr(), dx.data_ptr(), dq.data_ptr(),
+        *[d.data_ptr() for d in grads], batch, height, width, channels, head_dim, chunk_ptr, srnl_consts(),
+        ws.data_ptr(), ws.numel() * 4, hip.stream_of(x_c)), "vh_srnl_spatial_backward")
+    grads = [d.view(t.shape).to(t.dtype) for d, t in zip(grads, (*memories, d_skip, weights))]
+    return (*grads[:5], dx, dq, *grads[5:])
+
+
+def projected_training_supported(x_nhwc, linear):
+    """Whether ``srnl_spatial_projected`` takes x and the query projection ``linear``: what
+    bf16 autocast makes of an FP32 Linear, at the widths of the 1x1 convolution kernel."""
+    w, b = linear.weight, linear.bias
+    return (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and x_nhwc.dtype == torch.bfloat16 and (x_nhwc.data_ptr() % 16 == 0 or not x_nhwc.is_contiguous())
+            and type(w) is torch.nn.Parameter and type(b) is torch.nn.Parameter
+            and w.dtype == b.dtype == torch.float32 and w.device == b.device == x_nhwc.device
+            and w.shape == (x_nhwc.shape[-1],) * 2 and b.shape == w.shape[:1] and x_nhwc.shape[-1] % 32 == 0)
+
+
+class ProjectedSpatialSRNLFunction(torch.autograd.Function):
+    """``SpatialSRNLFunction`` of q = x W^T + b under bf16 autocast, x ``[B, H, W, C]``
+    contiguous bf16 (``projected_training_supported``), with the projection's own gradients:
+    dx gains dq W in the product's epilogue, dW and db come from one pass over the maps.
+
+    Autocast's linear rounds W, b and q to bf16, and so does this; its weight gradients are
+    FP32 sums rounded to bf16 on the way, these are not."""
+
+    @staticmethod
+    def forward(ctx, M_m_0, M_v_0, M_k_0, M_eta_0, M_alpha_0, x, w, b, d_skip, weights, chunks):
+        if torch.jit.is_tracing():
+            raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
+        memories = (M_m_0, M_v_0, M_k_0, M_eta_0, M_alpha_0)
+        operands, q = project_queries(x, w, b)
+        out, gains = srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks)
+        ctx.save_for_backward(*memories, x, q, operands, d_skip, weights, gains)
+        ctx.chunks = chunks
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        *memories, x, q, operands, d_skip, weights, gains = ctx.saved_tensors
+        *dmem, dx, dq, dskip, dweights = srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, gains, dout)
+        needs = ctx.needs_input_grad
+        dx, dw, db = project_queries_backward(x, operands, dx, dq, needs[5], needs[6] or needs[7])
+        return (*dmem, dx, dw, db, dskip, dweights, None)
+
+
+@on_tensor_device
+def project_queries(x, w, b):
+    """The projection's bf16 operands (W, W^T and b, in one buffer) and the queries."""
+    channels = x.shape[-1]
+    w, b = _fp32(w), _fp32(b)
+    operands = torch.empty((2 * channels + 2, channels), device=x.device, dtype=torch.bfloat16)
+    q = torch.empty_like(x)
+    lib, base, half = hip.load_library(), operands.data_ptr(), 2 * channels * channels
+    stream = hip.stream_of(x)
+    hip.check(lib.vh_linear_operands(w.data_ptr(), b.data_ptr(), hip.VH_DTYPE_F32, channels, channels, base, base + half,
+                                     base + 2 * half, stream), "vh_linear_operands")
+    hip.check(lib.vh_pointwise_conv_nhwc_forward(
+        x.data_ptr(), hip.VH_DTYPE_BF16, base, base + 2 * half, EPI_BIAS, None, None, None, 0, q.data_ptr(),
+        x.numel() // channels, channels, channels, stream), "vh_pointwise_conv_nhwc_forward")
+    return operands, q
+
+
+@on_tensor_device
+def project_queries_backward(x, operands, dx, dq, need_dx, need_params):
+    """dx + dq W (or None), dW and db (or None) of ``project_queries``."""
+    channels = x.shape[-1]
+    tokens, lib, stream = x.numel() // channels, hip.load_library(), hip.stream_of(x)
+    total = dw = db = None
+    if need_dx:
+        total = torch.empty_like(x)
+        hip.check(lib.vh_pointwise_conv_nhwc_forward(
+            dq.data_ptr(), hip.VH_DTYPE_BF16, operands.data_ptr() + 2 * channels * channels, None, EPI_ADD,
+            dx.data_ptr(), None, None, 0, total.data_ptr(), tokens, channels, channels, stream),
+            "vh_pointwise_conv_nhwc_forward")
+    if need_params:
+        dw = torch.empty((channels, channels), device=x.device, dtype=torch.float32)
+        db = torch.empty(channels, device=x.device, dtype=torch.float32)
+        ws = hip.workspace(lib.vh_linear_weight_grad_workspace_bytes(tokens, channels, channels), x.device)
+        hip.check(lib.vh_linear_weight_grad(dq.data_ptr(), x.data_ptr(), tokens, channels, channels, dw.data_ptr(),
+                                            db.data_ptr(), ws.data_ptr(), ws.numel() * 4, stream),
+                  "vh_linear_weight_grad")
+    return total, dw, db
+
+
+def _check_merge(x_nhwc, d_skip, weights):
+    if weights.shape != (4, x_nhwc.shape[-1]) or d_skip.numel() not in (weights.numel(), x_nhwc.shape[-1]):
+        raise RuntimeError("d_skip must contain C or 4*C values and the direction weights 4*C")
 
 
 def srnl_spatial(memories, x_nhwc, q_nhwc, d_skip, weights, chunks):
     """Differentiable spatial operator (``spatial_training_supported``)."""
-    if weights.shape != (4, x_nhwc.shape[-1]) or d_skip.numel() not in (weights.numel(), x_nhwc.shape[-1]):
-        raise RuntimeError("d_skip must contain C or 4*C values and the direction weights 4*C")
+    _check_merge(x_nhwc, d_skip, weights)
     if not (torch.is_grad_enabled() and any(t.requires_grad for t in (*memories, x_nhwc, q_nhwc, d_skip, weights))):
         # nothing to differentiate: the inference scan, which keeps nothing
         if torch.jit.is_tracing():
             raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
         return srnl_spatial_inference(memories, x_nhwc, q_nhwc, d_skip, weights, chunks)
     return SpatialSRNLFunction.apply(*memories, x_nhwc, q_nhwc, d_skip, weights, tuple(int(c) for c in chunks))
+
+
+def srnl_spatial_projected(memories, x_nhwc, linear, d_skip, weights, chunks):
+    """``srnl_spatial`` of the queries ``linear(x_nhwc)`` (``projected_training_supported``)."""
+    _check_merge(x_nhwc, d_skip, weights)
+    return ProjectedSpatialSRNLFunction.apply(*memories, x_nhwc, linear.weight, linear.bias, d_skip, weights,
+                                              tuple(int(c) for c in chunks))

@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "vh_conv3x3_nhwc_forward", "vh_srnl_backward_workspace_bytes", "vh_srnl_backward",
     "vh_srnl_spatial_gains_bytes", "vh_srnl_spatial_gains",
     "vh_srnl_spatial_backward_workspace_bytes", "vh_srnl_spatial_backward",
+    "vh_linear_operands", "vh_linear_weight_grad_workspace_bytes", "vh_linear_weight_grad",
     "vh_postprocess_scale_backward_workspace_bytes", "vh_postprocess_scale_backward",
     "vh_grn_backward_workspace_bytes", "vh_grn_backward", "vh_layernorm2d_backward_workspace_bytes",
     "vh_layernorm2d_backward", "vh_qnorm_backward", "vh_residual_add_backward_workspace_bytes",
@@ -96,6 +97,9 @@ _SIGNATURES = {
     "vh_srnl_spatial_backward": (ctypes.c_int, [
         _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
         _i64, _i64, _i64, _i64, _i32, _I64P, _CP, _vp, _sz, _vp]),
+    "vh_linear_operands": (ctypes.c_int, [_vp, _vp, _i32, _i64, _i64, _vp, _vp, _vp, _vp]),
+    "vh_linear_weight_grad_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "vh_linear_weight_grad": (ctypes.c_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _sz, _vp]),
     "vh_postprocess_scale_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i32, _i32]),
     "vh_postprocess_scale_backward": (ctypes.c_int, [
         _vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp, _sz, _vp]),
