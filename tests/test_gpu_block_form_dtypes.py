@@ -125,3 +125,24 @@ def test_line_per_workgroup_scan_edges(oracle, device, batch, height, width, hea
     expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 16)
     r, m = rel_err(got, expected), max_rel_err(got, expected)
     assert r <= BLOCK_TOL and m <= BLOCK_TOL, f"{dtype} {height}x{width}: normwise {r:.3e}, elementwise {m:.3e}"
+
+
+@pytest.mark.parametrize("batch,height,width,heads", [
+    (2, 1, 16, 1), (1, 17, 1, 2), (2, 16, 17, 1), (1, 31, 32, 2), (1, 33, 48, 1), (2, 49, 15, 1), (1, 64, 65, 1),
+    (1, 5, 127, 2), (1, 128, 3, 1), (64, 16, 16, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_line_per_workgroup_scan_edges_wide_heads(oracle, device, batch, height, width, heads, dtype):
+    """The same at head_dim 32: 1 to 8 blocks per chunk, full, ragged and single-token, rows and
+    columns with different wave counts."""
+    from visionhope_amd.models.srnl_core.fused import srnl_spatial_inference
+
+    channels = 32 * heads
+    seed = 1000 * height + width
+    mems = memories(4, heads, 32, kind="strong", seed=seed)
+    x, q = (randn(batch, height, width, channels, seed=seed + i).to(dtype) for i in (1, 2))
+    skip, wts = randn(channels, seed=seed + 3, scale=0.1), 1 + randn(4, channels, seed=seed + 4, scale=0.1)
+    got = srnl_spatial_inference(tuple(torch.from_numpy(m).to(device) for m in mems), x.to(device), q.to(device),
+                                 skip.to(device), wts.to(device), (width, width, height, height)).cpu().numpy()
+    expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 32)
+    r, m = rel_err(got, expected), max_rel_err(got, expected)
+    assert r <= BLOCK_TOL and m <= BLOCK_TOL, f"{dtype} {height}x{width}: normwise {r:.3e}, elementwise {m:.3e}"

@@ -417,8 +417,7 @@ def test_spatial_few_lines_block_form(oracle, device, height, width, heads, kind
 @pytest.mark.parametrize("kind", ["perturbed", "strong"])
 def test_spatial_head_dim32_block_form(oracle, device, height, width, heads, kind):
     """head_dim 32, bf16: the block form with one workgroup per line and the chunk's blocks
-    over 1, 2 or 4 waves (chunks of up to 64 tokens; the 65-row map sends its column scans'
-    launch to the wide scan)."""
+    over 1, 2, 4 or, for the 65-row map, 8 waves."""
     channels = heads * 32
     mems = memories(4, heads, 32, kind=kind, seed=height * 5 + width)
     x = randn(2, height, width, channels, seed=height + 111).bfloat16()
@@ -433,7 +432,7 @@ def test_spatial_head_dim32_block_form(oracle, device, height, width, heads, kin
 @pytest.mark.parametrize("chunks", [(5, 16, 64, 3), (64, 33, 17, 48), (65, 7, 30, 12)])
 def test_sequence_head_dim32_block_form(oracle, device, chunks):
     """Packed bf16 sequences with head_dim 32 (157 tokens, ragged last chunks) through the
-    block form; a chunk of 65 tokens sends the launch to the wide scan."""
+    block form; a chunk of 65 tokens takes 8 waves."""
     from visionhope_amd.models.srnl_core.chunk import srnl_packed_forward
 
     batch, directions, heads, length = 2, 4, 2, 157

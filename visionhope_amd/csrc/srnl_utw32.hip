@@ -1,95 +1,119 @@
-// SRNL chunk scan for head_dim 32 (bf16, fp16 or FP32 activations) in the block form: the algebra of
-// srnl_ut.hip (same operand arithmetic) with the 32-wide matrices cut into 2 x 2 tiles of
-// 16 x 16 matrix-core products, and the layout of srnl_utw.hip (one workgroup per line, the
-// chunk's 16-token blocks spread over its waves).  Reference recurrence:
-// models/srnl_core/csrc/inference_recurrence.cuh:32-135, memory.cuh:219-233.
+// SRNL chunk scan for head_dim 32 (bf16, fp16 or FP32 activations): the form of
+// srnl_utw.hip (one workgroup per line, one wave per 16-token block of a chunk, W waves, the
+// product Gamma of the chunk gains carried) with 32-wide matrices as 2 x 2 tiles.  Reference
+// recurrence: models/srnl_core/csrc/inference_recurrence.cuh:32-135, memory.cuh:219-233.
 //
-//   * one workgroup per line, W waves (the chunk's 16-slot blocks rounded up to a power of
-//     two, at most 4: chunks of up to 64 tokens); wave w forms the affine map (X_w, Y_w) of
-//     block w: k_t = normalise(M_k x_t), v_t = M_v x_t and the gate pre-activations as two
-//     16-feature steps of bf16 products, the triangle L = diag(rho) K^T K diag(kappa) over
-//     the 32 features, Z = (I + L)^-1 W K^T by back substitution (32 columns, one lane
-//     each), then the four 16 x 16 tiles of X_w = a_15 I - (K D_a) Z and of Y_w^T = -(Delta Z)^T;
-//   * the maps compose in order, G^T <- X_w^T G^T + Y_w^T, with tile (I, J) =
-//     sum_K (X_w^T)[I][K] (G^T)[K][J] + (Y_w^T)[I][J] on wave 2I + J (mod W), one barrier per
-//     block;
-//   * the state S = [M_m; M_v; M_k; e; a; 0] (98 rows padded to 112, 32 columns, FP32) lives
-//     in LDS; the refresh S <- S G (reference :119-133) runs by 16-row blocks over the waves.
+//   * products over the 32 features run as one 16x16x32 step of bf16 hi + lo operands (a lane's
+//     quads of the two tiles as eight consecutive k), those over 16 tokens as 16x16x16; the
+//     solves are FP32 with both feature tiles as right-hand sides;
+//   * several blocks per chunk: the column tiles of P <- X_w^T P + (Gamma Y_w)^T do not meet, so
+//     waves 0 and 1 chain one each without a barrier, while the last two waves store the
+//     chunk-start content memory M_m Gamma, half of its columns each;
+//   * one block per chunk (W = 1): Gamma'^T = a Gamma^T - K D_e (Gamma R)^T, no map.
 //
-// Tiles pass between waves in the accumulator layout (lane 16 q + j: rows 4q..4q+3 of column
-// j), which the receiving lane reads back as it was written.  The accumulator layout of a
-// tile C is the A-operand layout of C^T and the B-operand layout of C, so X_w's tile (K, I)
-// is the A operand of (X_w^T)[I][K].  Slots past the chunk act as the identity.  The
-// chunk-start M_m goes to the workspace for the readout, split into bf16 hi + lo pairs for
-// spatial maps (p.split_states).
+// Bound by the dependency chain of a chunk.  Per launch on MI355X, against the form that
+// carried the whole 112 x 32 state, solved (I + L) by columns on the vector unit and met at
+// a barrier for every block of a chunk: 384 lines of 3,136 tokens (chunks of 56) 274 -> 204 us,
+// 128 lines 215 -> 149, 1,024 lines of 784 (28) 222 -> 110, 4,096 of 196 (14) 212 -> 102, 8 of
+// 196 (14) 50 -> 33; with chunks of more than 64 tokens (8 waves, one workgroup per CU; it was
+// the wide scan) 1,024 lines of 6,400 (80) 1,692 -> 1,157, 384 of 16,384 (128) 1,699 -> 1,018.
+#include <algorithm>
+
 #include "srnl_block_form.h"
+#include "srnl_blocks.h"
 
 namespace vh {
-using namespace blockform;
+using namespace blocks;
+using blockform::XQuad;
 
 namespace {
 
-// The wave's own LDS writes become visible to its other lanes (wave-private tables).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// A column of two FP32 tiles (32 rows) as bf16 matrix-core operands, |v - hi - lo| <= 2^-16 |v|.
+struct Col {
+    v4s h[2], l[2];
+};
+__device__ __forceinline__ Col split(v4f t0, v4f t1) {
+    Col o;
+    blockform::split4(t0, o.h[0], o.l[0]);
+    blockform::split4(t1, o.h[1], o.l[1]);
+    return o;
+}
+// acc + A^T B over 32 rows
+__device__ __forceinline__ v4f mm(const Col& a, const Col& b, v4f acc) { return blockform::mma3k2(a.h, a.l, b.h, b.l, acc); }
+// acc + A^T B over 16 rows, tile i of a and j of b
+__device__ __forceinline__ v4f mm16(const Col& a, int i, const Col& b, int j, v4f acc) {
+    return blockform::mma3(a.h[i], a.l[i], b.h[j], b.l[j], acc);
 }
 
-__device__ __forceinline__ void st4(float* p, const v4f& v) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
+__device__ __forceinline__ v4f load4f(const float* p) { return *reinterpret_cast<const v4f*>(p); }
 
-__device__ __forceinline__ void split4(const float4& v, v4s& hi, v4s& lo) {
-    const float a[4] = {v.x, v.y, v.z, v.w};
-    blockform::split4(a, hi, lo);
-}
+// A column in LDS: hi and lo halves apart, so that a wave's 16-byte accesses meet no conflict.
+struct ColStore {
+    uint4 h[64], l[64];
+    __device__ __forceinline__ void put(int lane, const Col& v) {
+        const uint2 a = __builtin_bit_cast(uint2, v.h[0]), b = __builtin_bit_cast(uint2, v.h[1]);
+        const uint2 c = __builtin_bit_cast(uint2, v.l[0]), d = __builtin_bit_cast(uint2, v.l[1]);
+        h[lane] = make_uint4(a.x, a.y, b.x, b.y);
+        l[lane] = make_uint4(c.x, c.y, d.x, d.y);
+    }
+    __device__ __forceinline__ Col get(int lane) const {
+        const uint4 a = h[lane], b = l[lane];
+        Col v;
+        v.h[0] = __builtin_bit_cast(v4s, make_uint2(a.x, a.y));
+        v.h[1] = __builtin_bit_cast(v4s, make_uint2(a.z, a.w));
+        v.l[0] = __builtin_bit_cast(v4s, make_uint2(b.x, b.y));
+        v.l[1] = __builtin_bit_cast(v4s, make_uint2(b.z, b.w));
+        return v;
+    }
+};
+
+constexpr int kGamStride = 36;   // floats per row of Gamma: 16-byte aligned, rows in different banks
+
+template <int W>
+struct Shared {
+    Scratch scratch[W];
+    float tr[W][16 * kTrStride];           // second transpose scratch
+    float gam[W > 1 ? 32 : 1][kGamStride]; // Gamma, by rows
+    ColStore G[2];                         // Gamma^T by columns of tiles
+    ColStore X[W > 1 ? W : 1][2];          // X_w by columns of tiles
+    v4f Y[W > 1 ? W : 1][2][2][W > 1 ? 64 : 1];   // (Gamma Y_w)^T: column tile, row tile
+};
 
 }  // namespace
 
 template <typename T, int W, bool SPATIAL>
-__global__ __launch_bounds__(64 * W) void srnl_scan32_utw_kernel(const ScanParams p) {
+__global__ __launch_bounds__(64 * W, 2) void srnl_scan32_utw_kernel(const ScanParams p) {
+    constexpr int D = 32;
     using XQ = XQuad<T>;
-    // Row strides are padded (keys 20, L and Z 20, state and G 36 floats) so that the 16-byte
-    // loads of 16 lanes down a column of rows fall in different LDS banks; the hand-over
-    // tiles are read back by the lane that wrote them, so they are stored lane-major.
-    constexpr int D = 32, DKS = 20, TS = 20, SD = 36;
-    constexpr int SR = 112;           // state rows: M_m 0-31, M_v 32-63, M_k 64-95, e 96, a 97, zero
-    constexpr int XW = W > 1 ? W - 1 : 1;
-    __shared__ __align__(16) float kT[W][D * DKS];    // normalised keys [feature][slot]
-    __shared__ __align__(16) float ndT[W][D * DKS];   // v - k [feature][slot]
-    __shared__ __align__(16) float tk[W][64];         // per slot: rho, kappa, -a_{t-1}, w
-    __shared__ __align__(16) float LZ[W][D * TS];     // L[s][t] at [t][s], then Z[s][f] at [f][s]
-    __shared__ __align__(16) float Xt[XW][4 * 256];   // waves 1..: X_w tile (K, I) at [2K + I], lane-major
-    __shared__ __align__(16) float Yt[XW][4 * 256];   // waves 1..: Y_w^T tile (I, J) at [2I + J], lane-major
-    __shared__ __align__(16) float St[SR * SD];       // state rows
-    __shared__ __align__(16) float Gr[D * SD];        // chunk gain G, by rows
-    __shared__ __align__(16) float G0[4 * 256];       // wave 0: (X_0 + Y_0)^T tile (I, J) at [2I + J], lane-major
+    __shared__ Shared<W> sh;
+    const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const Block bl(sh.scratch[wv], static_cast<int>(threadIdx.x) & 63);
+    const int lane = bl.lane, g = bl.g, c = bl.c;
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
 
-    const int tid = static_cast<int>(threadIdx.x);
-    const int wv = tid >> 6, lane = tid & 63, i16 = lane & 15, q = lane >> 4;
     const int64_t lines = p.B * p.R * p.heads;
     const int64_t line = xcd_remap(blockIdx.x, lines);
     const int64_t head = line % p.heads;
     const int r = static_cast<int>((line / p.heads) % p.R);
     const int64_t b = line / (p.heads * p.R);
     const int64_t sidx = p.per_line_state ? line : r * p.heads + head;
-
-    for (int idx = tid; idx < SR * D / 4; idx += 64 * W) {
-        const int row = idx >> 3, c4 = (idx & 7) * 4;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row < 32) v = ld4(p.Mm + sidx * D * D + row * D + c4);
-        else if (row < 64) v = ld4(p.Mv + sidx * D * D + (row - 32) * D + c4);
-        else if (row < 96) v = ld4(p.Mk + sidx * D * D + (row - 64) * D + c4);
-        else if (row == 96) v = ld4(p.Me + sidx * D + c4);
-        else if (row == 97) v = ld4(p.Ma + sidx * D + c4);
-        *reinterpret_cast<float4*>(St + row * SD + c4) = v;
-    }
+    // columns i of the transposed memories: rows 16 i + c, entries 4g.. and 16 + 4g..
+    auto column = [&](const float* m, int i) {
+        const float* row = m + (sidx * D + 16 * i + c) * D + 4 * g;
+        return split(load4f(row), load4f(row + 16));
+    };
+    const Col MkT[2] = {column(p.Mk, 0), column(p.Mk, 1)}, MvT[2] = {column(p.Mv, 0), column(p.Mv, 1)};
+    const Col MmT[2] = {column(p.Mm, 0), column(p.Mm, 1)};
+    // e and a as operand rows 4 j and 4 j + 1, so every lane's registers 0 and 1 end with e.z and a.z
+    const float* gate_row = ((c & 1) ? p.Ma : p.Me) + sidx * D + 4 * g;
+    const Col gates = (c & 3) < 2 ? split(load4f(gate_row), load4f(gate_row + 16)) : split(zero, zero);
 
     const int C = chunk_of(p.chunk, r);
     const int64_t nc = (p.L + C - 1) / C;
     const int nblk = (C + 15) / 16;
-    const T* xcol = static_cast<const T*>(p.x.ptr) + b * p.x.sb + r * p.x.sr + head * p.x.sh + 4 * q;
+    const int slot = 16 * wv + bl.tau;   // this lane's token of a chunk
+    const bool valid = slot < C;         // every chunk but the last is whole, and the last forms no gain
+    const T* xcol = static_cast<const T*>(p.x.ptr) + b * p.x.sb + r * p.x.sr + head * p.x.sh + 4 * g;
     int pa = 0, pb = 0, pc = 0, pst = 0;
     if constexpr (SPATIAL) {
         const int Wd = static_cast<int>(p.x.W), L = static_cast<int>(p.x.H * p.x.W);
@@ -98,301 +122,172 @@ __global__ __launch_bounds__(64 * W) void srnl_scan32_utw_kernel(const ScanParam
         pc = (r & 1) ? L - 1 : 0;
         pst = static_cast<int>(p.x.st);
     }
-    // x of token (chunk cc, slot 16 wv + i16), features 4q..4q+3 and 16+4q..16+4q+3, as raw
-    // bits; slots past the chunk read the line's first token and are zeroed when decoded
-    auto load_x = [&](int64_t cc, typename XQ::Raw (&raw)[2], bool& ok) {
-        const int slot = 16 * wv + i16;
-        const int64_t tok = cc * C + slot;
-        ok = slot < C && tok < p.L;
+    // x of this lane's token of chunk cc as raw bits; slots past the chunk read the line's
+    // first token and are zeroed when decoded
+    XRaw<T, 16> xr[2] = {};
+    auto load_x = [&](int64_t cc) {
         int64_t off = 0;
-        if (ok) {
+        if (valid) {
             if (SPATIAL && p.aligned) off = static_cast<int64_t>(pa * static_cast<int>(cc) + pb * slot + pc) * pst;
-            else off = token_offset<SPATIAL>(p.x, r, tok);
+            else off = token_offset<SPATIAL>(p.x, r, cc * C + slot);
         }
-        raw[0] = XQ::load(xcol + off);
-        raw[1] = XQ::load(xcol + off + 16);
+        xr[0] = XQ::load(xcol + off);
+        xr[1] = XQ::load(xcol + off + 16);
     };
-    float* const kTw = kT[wv];
-    float* const ndTw = ndT[wv];
-    float* const tkw = tk[wv];
-    float* const LZw = LZ[wv];
-
-    // x is always loaded one computing chunk ahead, so the only loads in flight when a chunk
-    // starts are its own x, issued before the chunk-start store: the wait for them leaves
-    // that store outstanding.
-    typename XQ::Raw xr[2] = {};
-    bool xok = false;
-    if (wv < nblk && nc > 1) load_x(0, xr, xok);
-    __syncthreads();
-    for (int64_t c = 0; c < nc; ++c) {
-        // chunk-start M_m for the readout (FP32 or split, p.split_states), a fixed number of
-        // stores per thread
+    // Columns 16 i + 4g.. of the content memory M_m Gamma the readout of chunk cc uses (M_m
+    // itself, unrounded, for the first), from column i of Gamma's tiles.
+    auto store_content = [&](int64_t cc, int i, const Col& gam) {
 #pragma unroll
-        for (int k = 0; k < D * D / 4 / (64 * W); ++k) {
-            const int idx = tid + 64 * W * k;
-            store_state4(p.states + (line * p.max_chunks + c) * D * D + idx * 4, ld4(St + (idx >> 3) * SD + (idx & 7) * 4),
+        for (int j = 0; j < 2; ++j) {
+            const int at = (16 * j + c) * D + 16 * i + 4 * g;
+            const v4f m = cc == 0 ? load4f(p.Mm + sidx * D * D + at) : mm(gam, MmT[j], zero);
+            store_state4(p.states + (line * p.max_chunks + cc) * D * D + at, make_float4(m[0], m[1], m[2], m[3]),
                          p.split_states);
         }
-        if (c == nc - 1) break;
+    };
+    // W > 1: the waves that store the content, and the column of Gamma each holds for it
+    constexpr int kFirstStore = W > 2 ? W - 2 : 0;
+    const int part = wv - kFirstStore;
+    auto gamma_column = [&]() {
+        v4f t[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[k][i] = sh.gam[W > 1 ? 16 * k + 4 * g + i : 0][16 * part + c];
+        return split(t[0], t[1]);
+    };
 
-        if (wv < nblk) {
-            const bool valid = 16 * wv + i16 < C;   // slot inside the chunk (every such token is < L here)
-            // ---- token phase: [M_k; M_v] x and (x.e, x.a), two 16-feature steps each ----
+    v4f gamT[2][2] = {{bl.diagonal(1.f), zero}, {zero, bl.diagonal(1.f)}};   // [column][row]
+    Col G[2] = {split(gamT[0][0], gamT[0][1]), split(gamT[1][0], gamT[1][1])};
+    Col gam[2] = {G[0], G[1]};   // columns of Gamma; W > 1: [0], column `part`
+    if (W > 1) gam[0] = part == 1 ? G[1] : G[0];
+    if (nc > 1 && wv < nblk) load_x(0);
+    for (int64_t ch = 0; ch < nc - 1; ++ch) {
+        if (W == 1 || wv < nblk) {
             v4s xh[2], xl[2];
-            XQ::operands(xr[0], xok, xh[0], xl[0]);
-            XQ::operands(xr[1], xok, xh[1], xl[1]);
-            // (both 16-feature steps in one 16x16x32 product: the lane's two quads as 8 k)
-            v4f kacc[2], vacc[2], gacc;
-            const bool on = (i16 & 3) < 2;   // operand rows 4q' + 0 / 4q' + 1: e / a, others zero
-            const v4f z4 = {0.f, 0.f, 0.f, 0.f};
+            XQ::operands(xr[0], valid, xh[0], xl[0]);
+            XQ::operands(xr[1], valid, xh[1], xl[1]);
+            const Col Z = split(XQ::mma_k2(G[0].h, G[0].l, xh, xl, zero), XQ::mma_k2(G[1].h, G[1].l, xh, xl, zero));
+            if (ch + 1 < nc - 1) load_x(ch + 1);   // in flight during this chunk
+            v4f K[2] = {mm(MkT[0], Z, zero), mm(MkT[1], Z, zero)}, Dl[2];
+            const v4f V[2] = {mm(MvT[0], Z, zero), mm(MvT[1], Z, zero)}, pre = mm(gates, Z, zero);
+            float kn = 0.f, dsq = 0.f;
 #pragma unroll
-            for (int RB = 0; RB < 2; ++RB) {
-                v4s h[2], l[2];
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) split4(ld4(St + (64 + 16 * RB + i16) * SD + 16 * kk + 4 * q), h[kk], l[kk]);
-                kacc[RB] = XQ::mma_k2(h, l, xh, xl, z4);
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) split4(ld4(St + (32 + 16 * RB + i16) * SD + 16 * kk + 4 * q), h[kk], l[kk]);
-                vacc[RB] = XQ::mma_k2(h, l, xh, xl, z4);
-            }
-            {
-                v4s h[2], l[2];
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    float4 g4 = ld4(St + (96 + (i16 & 1)) * SD + 16 * kk + 4 * q);
-                    if (!on) g4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                    split4(g4, h[kk], l[kk]);
-                }
-                gacc = XQ::mma_k2(h, l, xh, xl, z4);
-            }
-            // the next computing chunk's x, in flight during the rest of this chunk
-            if (c + 1 < nc - 1) load_x(c + 1, xr, xok);
-            float kn = 0.f;
-#pragma unroll
-            for (int RB = 0; RB < 2; ++RB)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) kn += kacc[RB][j] * kacc[RB][j];
+            for (int i = 0; i < 4; ++i) kn += K[0][i] * K[0][i] + K[1][i] * K[1][i];
             kn = xor16_32_sum(kn);
             // ||k||^2 of the normalised key is ||k~||^2 / (||k~||^2 + 1e-6)
             const float inv = rsqrtf(kn + 1e-6f);
-            const float ksq = kn * inv * inv;
-            float kn4[2][4], dsq = 0.f;
 #pragma unroll
-            for (int RB = 0; RB < 2; ++RB)
+            for (int t = 0; t < 2; ++t) {
+                K[t] *= inv;
+                Dl[t] = K[t] - V[t];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float kv = kacc[RB][j] * inv, nd = vacc[RB][j] - kv;
-                    kn4[RB][j] = kv;
-                    dsq += nd * nd;
-                    kTw[(16 * RB + 4 * q + j) * DKS + i16] = kv;
-                    ndTw[(16 * RB + 4 * q + j) * DKS + i16] = nd;
-                }
+                for (int i = 0; i < 4; ++i) dsq += Dl[t][i] * Dl[t][i];
+            }
             dsq = xor16_32_sum(dsq);
             float alpha, eff;
-            token_gates_fast(p.k, gacc[0], gacc[1], dsq, ksq, alpha, eff);   // every lane: token i16
-            // Per-slot scalars (srnl_ut.hip): cl = inclusive prefix of log2 alpha over the
-            // 16-lane row, a_15 = 2^cl_15, and the triangle's ratio a_{t-1} / a_s split into
-            // rho_s = eta^_s 2^(m - cl_s) and kappa_t = 2^(clx_t - m) about m = cl_15 / 2.
-            const float la = valid ? __builtin_amdgcn_logf(alpha) : 0.f;
-            const float eh = valid ? eff : 0.f;
-            float cl = la;
-            cl += row_shr<1>(cl);
-            cl += row_shr<2>(cl);
-            cl += row_shr<4>(cl);
-            cl += row_shr<8>(cl);
-            const float tot = readlane_f(cl, 15);
-            const float decay = __builtin_amdgcn_exp2f(tot), mid = 0.5f * tot, clx = cl - la;
-            if (lane < 16) {
-                tkw[lane] = eh * __builtin_amdgcn_exp2f(mid - cl);        // rho
-                tkw[16 + lane] = __builtin_amdgcn_exp2f(clx - mid);       // kappa
-                tkw[32 + lane] = -__builtin_amdgcn_exp2f(clx);            // -a_{t-1}
-                tkw[48 + lane] = eh * __builtin_amdgcn_exp2f(tot - cl);   // w
+            token_gates_fast(p.k, pre[0], pre[1], dsq, kn * inv * inv, alpha, eff);
+            const Col k = split(K[0], K[1]), dl = split(Dl[0], Dl[1]);
+            const v4f gram = mm(k, k, zero);
+            const v4f gd[2] = {mm(dl, G[0], zero), mm(dl, G[1], zero)};   // (Gamma Delta)^T
+            // K^T by two transposes in one pass through LDS
+            v4f KT[2];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bl.s.tr[(4 * g + i) * kTrStride + c] = K[0][i];
+                sh.tr[wv][(4 * g + i) * kTrStride + c] = K[1][i];
             }
-            wave_sync();
-            // ---- L = diag(rho) K^T K diag(kappa) over 32 features, strict upper triangle,
-            //      by columns ----
-            {
-                // the Gram tile from the keys split once, scaled after the product
-                const float kap = tkw[16 + i16];
-                const float4 r4 = ld4(tkw + 4 * q);   // rho of rows 4q..4q+3
-                const float rr[4] = {r4.x, r4.y, r4.z, r4.w};
-                v4s kh[2], kl[2];
+            __builtin_amdgcn_wave_barrier();
+            KT[0] = load4f(&bl.s.tr[c * kTrStride + 4 * g]);
+            KT[1] = load4f(&sh.tr[wv][c * kTrStride + 4 * g]);
+            __builtin_amdgcn_wave_barrier();
+            const Decays dec = bl.decays(valid ? eff : 0.f, valid ? alpha : 1.f);
+            const Triangle tri = bl.triangle(dec, gram);
+            if constexpr (W == 1) {
+                v4f RT[2];
 #pragma unroll
-                for (int kk = 0; kk < 2; ++kk) blockform::split4(kn4[kk], kh[kk], kl[kk]);
-                const v4f P = mma3k2(kh, kl, kh, kl, v4f{0.f, 0.f, 0.f, 0.f});
-                float lv[4];
+                for (int j = 0; j < 2; ++j) RT[j] = mm(k, G[j], zero) * dec.Da_r() + gd[j];
+                bl.solve_lower(tri, RT);
+                store_content(ch, 0, gam[0]);
+                store_content(ch, 1, gam[1]);
+                const Col kd = split(-(KT[0] * dec.De_r()), -(KT[1] * dec.De_r())), rt = split(RT[0], RT[1]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) lv[j] = (4 * q + j < i16) ? (P[j] * rr[j]) * kap : 0.f;
-                *reinterpret_cast<float4*>(LZw + i16 * TS + 4 * q) = make_float4(lv[0], lv[1], lv[2], lv[3]);
-            }
-            wave_sync();
-            // ---- Z = (I + L)^-1 W K^T: lane 16 q + i (q < 2) solves column f = 16 q + i from
-            //      the last row up, Z[s][f] = w_s k_s[f] - sum_{v > s} L[s][v] Z[v][f]; Z
-            //      overwrites L once every lane has read it (one wave, program order) ----
-            if (q < 2) {
-                const int f = 16 * q + i16;
-                float acc[16], zc[16];
+                for (int j = 0; j < 2; ++j) {
 #pragma unroll
-                for (int s0 = 0; s0 < 16; s0 += 4) {
-                    const float4 k4 = ld4(kTw + f * DKS + s0);
-                    const float4 w4 = ld4(tkw + 48 + s0);
-                    acc[s0] = k4.x * w4.x; acc[s0 + 1] = k4.y * w4.y;
-                    acc[s0 + 2] = k4.z * w4.z; acc[s0 + 3] = k4.w * w4.w;
+                    for (int i = 0; i < 2; ++i) gamT[j][i] = mm16(kd, i, rt, j, gamT[j][i] * dec.a());
+                    G[j] = split(gamT[j][0], gamT[j][1]);
                 }
-                float lA[4][16], lB[4][16];
-                auto load_group = [&](int v0, float (&buf)[4][16]) {
 #pragma unroll
-                    for (int dv = 0; dv < 4; ++dv)
+                for (int i = 0; i < 2; ++i) gam[i] = split(bl.transpose(gamT[0][i]), bl.transpose(gamT[1][i]));
+            } else {
+                v4f S[2] = {KT[0] * dec.De_r(), KT[1] * dec.De_r()};
+                bl.solve_upper(tri, S);
+                const Col s = split(-S[0], -S[1]), ka = split(KT[0] * dec.Da_r(), KT[1] * dec.Da_r());
+                const Col d = split(gd[0], gd[1]);
+                const v4f aI = bl.diagonal(dec.a());
 #pragma unroll
-                        for (int s0 = 0; s0 < v0 + dv; s0 += 4) {
-                            const float4 l4 = ld4(LZw + (v0 + dv) * TS + s0);
-                            buf[dv][s0] = l4.x; buf[dv][s0 + 1] = l4.y; buf[dv][s0 + 2] = l4.z; buf[dv][s0 + 3] = l4.w;
-                        }
-                };
-                auto solve_group = [&](int v0, const float (&buf)[4][16]) {
+                for (int j = 0; j < 2; ++j) {
+                    sh.X[wv][j].put(lane, split(mm16(ka, 0, s, j, j == 0 ? aI : zero), mm16(ka, 1, s, j, j == 1 ? aI : zero)));
 #pragma unroll
-                    for (int dv = 3; dv >= 0; --dv) {
-                        const int v = v0 + dv;
-                        zc[v] = acc[v];
-#pragma unroll
-                        for (int s2 = 0; s2 < v; ++s2) acc[s2] -= buf[dv][s2] * zc[v];
-                    }
-                };
-                load_group(12, lA);
-                load_group(8, lB);
-                solve_group(12, lA);
-                load_group(4, lA);
-                solve_group(8, lB);
-                load_group(0, lB);
-                solve_group(4, lA);
-                solve_group(0, lB);
-#pragma unroll
-                for (int s = 0; s < 16; s += 4)
-                    *reinterpret_cast<float4*>(LZw + f * TS + s) = make_float4(zc[s], zc[s + 1], zc[s + 2], zc[s + 3]);
-            }
-            wave_sync();
-            // ---- the block's map, tile by tile: X = a_15 I - (K D_a) Z, Y = -Delta Z; wave 0
-            //      (the first block, entered with G = I) keeps (X_0 + Y_0)^T, the others hand
-            //      over X_w and Y_w^T ----
-            {
-                const float4 a4 = ld4(tkw + 32 + 4 * q);
-                v4s zh[2], zl[2];
-                float nka[2][4], ndl[2][4];
-#pragma unroll
-                for (int F = 0; F < 2; ++F) {
-                    split4(ld4(LZw + (16 * F + i16) * TS + 4 * q), zh[F], zl[F]);   // Z[4q + j][16F + i16]
-                    const float4 k4 = ld4(kTw + (16 * F + i16) * DKS + 4 * q);
-                    const float4 d4 = ld4(ndTw + (16 * F + i16) * DKS + 4 * q);
-                    nka[F][0] = k4.x * a4.x; nka[F][1] = k4.y * a4.y; nka[F][2] = k4.z * a4.z; nka[F][3] = k4.w * a4.w;
-                    ndl[F][0] = d4.x; ndl[F][1] = d4.y; ndl[F][2] = d4.z; ndl[F][3] = d4.w;
-                }
-                const v4f dI = diag4(decay, q, i16), z0 = {0.f, 0.f, 0.f, 0.f};
-                if (wv == 0) {
-                    v4s nbh[2], nbl[2];
-#pragma unroll
-                    for (int F = 0; F < 2; ++F) {
-                        const float nb[4] = {nka[F][0] + ndl[F][0], nka[F][1] + ndl[F][1], nka[F][2] + ndl[F][2],
-                                             nka[F][3] + ndl[F][3]};
-                        blockform::split4(nb, nbh[F], nbl[F]);
-                    }
-#pragma unroll
-                    for (int I = 0; I < 2; ++I)
-#pragma unroll
-                        for (int J = 0; J < 2; ++J) {
-                            const v4f gT = mma3(zh[I], zl[I], nbh[J], nbl[J], I == J ? dI : z0);   // (X_0 + Y_0)^T
-                            // one block: G itself (lane (j, q) of tile (I, J) holds
-                            // G[16J + j][16I + 4q..16I + 4q + 3]); else the composition's start
-                            if (nblk == 1) st4(Gr + (16 * J + i16) * SD + 16 * I + 4 * q, gT);
-                            else st4(G0 + (2 * I + J) * 256 + 4 * lane, gT);
-                        }
-                } else {
-                    v4s kah[2], kal[2], dlh[2], dll[2];
-#pragma unroll
-                    for (int F = 0; F < 2; ++F) {
-                        blockform::split4(nka[F], kah[F], kal[F]);
-                        blockform::split4(ndl[F], dlh[F], dll[F]);
-                    }
-                    float* const xt = Xt[wv - 1];
-                    float* const yt = Yt[wv - 1];
-#pragma unroll
-                    for (int A = 0; A < 2; ++A)
-#pragma unroll
-                        for (int B = 0; B < 2; ++B) {
-                            // X_w tile (A, B); Y_w^T tile (A, B)
-                            st4(xt + (2 * A + B) * 256 + 4 * lane, mma3(kah[A], kal[A], zh[B], zl[B], A == B ? dI : z0));
-                            st4(yt + (2 * A + B) * 256 + 4 * lane, mma3(zh[A], zl[A], dlh[B], dll[B], z0));
-                        }
+                    for (int i = 0; i < 2; ++i) sh.Y[wv][j][i][lane] = mm16(s, i, d, j, zero);
                 }
             }
         }
-        __syncthreads();
-        // ---- composition, tile (I, J) of G^T on wave 2I + J (mod W):
-        //      (G^T)[I][J] <- sum_K (X_w^T)[I][K] (G^T)[K][J] + (Y_w^T)[I][J], one barrier per
-        //      block.  Step w writes its tiles over Y_w's (each read only by the wave that
-        //      owns the tile); the last step writes G by rows. ----
-        {
-            const float* gprev = G0;
-            for (int w = 1; w < nblk; ++w) {
-                if (w > 1) __syncthreads();   // step w - 1's tiles written
-                float* const ynext = Yt[w - 1];
-                for (int t = wv; t < 4; t += W) {
-                    const int I = t >> 1, J = t & 1;
-                    v4s gh[2], gl[2], xh[2], xl[2];
+        if constexpr (W > 1) {
+            if (W == 2) store_content(ch, part, gam[0]);
+            __syncthreads();
+            if (wv < 2) {
+                Col P = G[0];
+                if (wv == 1) P = G[1];
+                v4f t[2];
+                // the next map is in flight while a step runs (past the last block: read, unused)
+                Col X[2] = {sh.X[0][0].get(lane), sh.X[0][1].get(lane)};
+                v4f Y[2] = {sh.Y[0][wv][0][lane], sh.Y[0][wv][1][lane]};
 #pragma unroll
-                    for (int K = 0; K < 2; ++K) {
-                        split4(ld4(gprev + (2 * K + J) * 256 + 4 * lane), gh[K], gl[K]);
-                        // (X_w^T)[I][K] is the transpose of X_w's tile (K, I)
-                        split4(ld4(Xt[w - 1] + (2 * K + I) * 256 + 4 * lane), xh[K], xl[K]);
+                for (int w = 0; w < W; ++w) {
+                    const Col x[2] = {X[0], X[1]};
+                    const v4f y[2] = {Y[0], Y[1]};
+                    if (w + 1 < W) {
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            X[i] = sh.X[w + 1][i].get(lane);
+                            Y[i] = sh.Y[w + 1][wv][i][lane];
+                        }
                     }
-                    const float4 y4 = ld4(ynext + t * 256 + 4 * lane);
-                    const v4f gT = mma3k2(xh, xl, gh, gl, v4f{y4.x, y4.y, y4.z, y4.w});
-                    if (w == nblk - 1) st4(Gr + (16 * J + i16) * SD + 16 * I + 4 * q, gT);
-                    else st4(ynext + t * 256 + 4 * lane, gT);
+                    if (w < nblk) {
+                        t[0] = mm(x[0], P, y[0]);
+                        t[1] = mm(x[1], P, y[1]);
+                        P = split(t[0], t[1]);
+                    }
                 }
-                gprev = ynext;
+                sh.G[wv].put(lane, P);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) *reinterpret_cast<v4f*>(&sh.gam[W > 1 ? 16 * wv + c : 0][16 * i + 4 * g]) = t[i];
+            } else if (W > 2 && part >= 0) {
+                store_content(ch, part, gam[0]);
             }
+            __syncthreads();
+            G[0] = sh.G[0].get(lane);
+            G[1] = sh.G[1].get(lane);
+            if (part >= 0) gam[0] = gamma_column();
         }
-        __syncthreads();
-        // ---- refresh: S <- S G, 16-row blocks over the waves (A: S rows; B: G columns) ----
-        {
-            v4s gh[2][2], gl[2][2];   // [K][FC]: G[16K + 4q + k][16FC + i16]
-#pragma unroll
-            for (int K = 0; K < 2; ++K)
-#pragma unroll
-                for (int FC = 0; FC < 2; ++FC) {
-                    float gv[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) gv[k] = Gr[(16 * K + 4 * q + k) * SD + 16 * FC + i16];
-                    blockform::split4(gv, gh[K][FC], gl[K][FC]);
-                }
-            for (int R = wv; R < SR / 16; R += W) {
-                v4s sh[2], sl[2];
-#pragma unroll
-                for (int K = 0; K < 2; ++K) split4(ld4(St + (16 * R + i16) * SD + 16 * K + 4 * q), sh[K], sl[K]);
-                v4f sn[2];
-#pragma unroll
-                for (int FC = 0; FC < 2; ++FC) {
-                    const v4s bh[2] = {gh[0][FC], gh[1][FC]}, bl[2] = {gl[0][FC], gl[1][FC]};
-                    sn[FC] = mma3k2(sh, sl, bh, bl, v4f{0.f, 0.f, 0.f, 0.f});
-                }
-#pragma unroll
-                for (int FC = 0; FC < 2; ++FC)
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) St[(16 * R + 4 * q + k) * SD + 16 * FC + i16] = sn[FC][k];
-            }
-        }
-        __syncthreads();
+    }
+    if (W == 1) {
+        store_content(nc - 1, 0, gam[0]);
+        store_content(nc - 1, 1, gam[1]);
+    } else if (part >= 0) {
+        store_content(nc - 1, part, gam[0]);
     }
 }
 
 // Waves per line of the head_dim-32 block-form scan: the chunk's 16-slot blocks rounded up to
-// a power of two; 0 when a chunk exceeds 4 blocks (64 tokens) or the input rows are not
+// a power of two; 0 when a chunk exceeds 8 blocks (128 tokens) or the input rows are not
 // aligned for vector loads.
 int scan32_utw_waves(const ScanParams& sp) {
     int max_chunk = 0;
     for (int r = 0; r < sp.R; ++r) max_chunk = std::max(max_chunk, sp.chunk[r]);
     const int blocks = (max_chunk + 15) / 16;
-    if (blocks > 4 || !sp.x_vec) return 0;
+    if (blocks > 8 || !sp.x_vec) return 0;
     int w = 1;
     while (w < blocks) w *= 2;
     return w;
@@ -412,7 +307,8 @@ bool launch_scan32_utw(const ScanParams& sp, hipStream_t stream) {
         switch (waves) {
             case 1: go(std::integral_constant<int, 1>{}, spc); break;
             case 2: go(std::integral_constant<int, 2>{}, spc); break;
-            default: go(std::integral_constant<int, 4>{}, spc); break;
+            case 4: go(std::integral_constant<int, 4>{}, spc); break;
+            default: go(std::integral_constant<int, 8>{}, spc); break;
         }
     };
     if (sp.x.spatial) pick(std::true_type{});
