@@ -83,3 +83,37 @@ def test_projected_step_matches_module_call(device, shape, head_dim, frozen, lay
     for g, w, leaf in zip((y, *got), (y_ref, *want), (y_ref, *leaves)):
         assert g.dtype == w.dtype == leaf.dtype and g.shape == w.shape
         assert rel_err(g.detach().float().cpu().numpy(), w.detach().float().cpu().numpy()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("dim,head_dim,layout", [(32, 16, "channels_last"), (96, 32, "nchw"), (48, 16, "nchw"),
+                                                 (128, 16, "offset")])
+@pytest.mark.parametrize("bias", [True, False])
+def test_inference_projection(device, dim, head_dim, layout, bias):
+    """The operator's queries in inference under bf16 autocast against float64: one rounding
+    of W and b (2^-9 each of their terms) and one of q."""
+    from visionhope_amd.models import VisionHOPEOperator
+    from visionhope_amd.models.srnl_core import fused
+
+    op = VisionHOPEOperator(dim, head_dim=head_dim, fast_inference=True).to(device).eval()
+    with torch.no_grad():
+        op.W_q.weight.copy_(randn(dim, dim, seed=5, scale=dim ** -0.5))
+        op.W_q.bias.copy_(randn(dim, seed=4, scale=0.1))
+    if not bias:
+        op.W_q.bias = None
+    x = randn(2, 5, 7, dim, seed=7).to(torch.bfloat16).to(device)
+    if layout == "offset":
+        x = torch.empty(x.numel() + 1, dtype=x.dtype, device=device)[1:].view(x.shape).copy_(x)
+    x = x.permute(0, 3, 1, 2)
+    x = x.contiguous() if layout == "nchw" else x
+    seen, real = [], fused.srnl_spatial_inference
+    fused.srnl_spatial_inference = lambda m, xs, q, *rest: seen.append(q) or real(m, xs, q, *rest)
+    try:
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            op(x)
+    finally:
+        fused.srnl_spatial_inference = real
+    q, = seen
+    x64, w64 = x.permute(0, 2, 3, 1).double(), op.W_q.weight.detach().double()
+    b64 = op.W_q.bias.detach().double() if bias else torch.zeros(dim, device=device, dtype=torch.float64)
+    bound = 2.0 ** -8 * (x64.abs() @ w64.abs().T + b64.abs())
+    assert q.dtype == torch.bfloat16 and ((q.double() - (x64 @ w64.T + b64)).abs() <= bound).all()
