@@ -87,16 +87,21 @@ class SRNL(nn.Module):
     def _inference_path(self, x, query_dtype):
         """("sequence", None) when the inference entry point applies, else ("ordinary",
         the first reason it does not)."""
-        blockers = (
-            (not self.fast_inference, "Fast inference is disabled"),
-            (self.training, "The module is in training mode"),
-            (torch.is_grad_enabled(), "Gradients are enabled"),
-            (not x.is_cuda, "SRNL requires CUDA inputs"),
-            (x.dtype not in _IO_DTYPES, "SRNL requires FP16, BF16, or FP32 inputs"),
-            (query_dtype != x.dtype, "Fast inference requires matching input and query dtypes"),
-        )
-        reason = next((why for blocked, why in blockers if blocked), None)
-        return ("ordinary", reason) if reason else ("sequence", None)
+        if not self.fast_inference:
+            reason = "Fast inference is disabled"
+        elif self.training:
+            reason = "The module is in training mode"
+        elif torch.is_grad_enabled():
+            reason = "Gradients are enabled"
+        elif not x.is_cuda:
+            reason = "SRNL requires CUDA inputs"
+        elif x.dtype not in _IO_DTYPES:
+            reason = "SRNL requires FP16, BF16, or FP32 inputs"
+        elif query_dtype != x.dtype:
+            reason = "Fast inference requires matching input and query dtypes"
+        else:
+            return "sequence", None
+        return "ordinary", reason
 
     def inference_status(self, x, queries=None):
         """Report path selection for valid inputs in the current eval/grad context."""
@@ -105,11 +110,11 @@ class SRNL(nn.Module):
 
     def _validate_memories(self, device):
         """The five memories, checked for shape, floating dtype and device."""
-        shapes = [(self.directions, self.num_heads, self.head_dim, self.head_dim)] * 3
-        shapes += [(self.directions, self.num_heads, self.head_dim)] * 2
+        matrix = (self.directions, self.num_heads, self.head_dim, self.head_dim)
         states = self.initial_memories
-        for i, (state, shape) in enumerate(zip(states, shapes)):
-            if (not isinstance(state, torch.Tensor) or tuple(state.shape) != shape
+        for i, state in enumerate(states):
+            shape = matrix if i < 3 else matrix[:3]
+            if (not isinstance(state, torch.Tensor) or state.shape != shape
                     or not state.is_floating_point() or state.device != device):
                 raise ValueError(f"SRNL memory {i} must be floating point, shape {shape}, on {device}")
         return states
@@ -175,7 +180,7 @@ class SRNL(nn.Module):
         batch, length, _ = x.shape
         lines = x.reshape(batch, 1, length, self.num_heads, self.head_dim).transpose(2, 3).contiguous()
         y = self._packed_forward(lines, queries.unsqueeze(1), spatial_shape)
-        return y[:, 0].transpose(1, 2).reshape(batch, length, self.dim)
+        return y.squeeze(1).transpose(1, 2).reshape(batch, length, self.dim)
 
     def extra_repr(self):
         return (f"dim={self.dim}, head_dim={self.head_dim}, directions={self.directions}, "

@@ -62,11 +62,14 @@ def _float_memories(memories, directions, heads, head_dim, n_flat):
         state_count, per_line = n_flat, 1
     else:
         raise AssertionError(f"Expected memory tensors with 4 or 5 dims, got shape {tuple(m_m.shape)}.")
-    mats = [m.detach().contiguous().view(state_count, head_dim, head_dim).float().contiguous()
-            for m in memories[:3]]
-    vecs = [m.detach().contiguous().view(state_count, head_dim).float().contiguous()
-            for m in memories[3:]]
-    return (*mats, *vecs), per_line
+    mats, vecs = (state_count, head_dim, head_dim), (state_count, head_dim)
+    return tuple(_float_memory(m, mats if i < 3 else vecs) for i, m in enumerate(memories)), per_line
+
+
+def _float_memory(m, shape):
+    if m.dtype == torch.float32 and m.is_contiguous() and m.numel() == math.prod(shape):
+        return m   # the kernels take it by pointer
+    return m.detach().contiguous().view(shape).float().contiguous()
 
 
 @on_tensor_device
@@ -85,22 +88,22 @@ def srnl_packed_forward(memories, x, q, chunk_sizes, *, q_raw):
     q_c = q.contiguous() if q_raw else q.float().contiguous()
     out = torch.empty_like(x_c)
     lib = hip.load_library()
-    max_chunks = max(math.ceil(length / c) for c in chunks)
+    max_chunks = -(-length // min(chunks))
     ws = hip.workspace(lib.vh_srnl_workspace_bytes(n_flat, max_chunks, head_dim), x.device)
     chunk_ptr, _keep = hip.int64_array(chunks)
     consts = srnl_consts()
-    mem_ptrs = [hip.ptr(m) for m in states]
+    mem_ptrs = [m.data_ptr() for m in states]
     if q_raw:
         rc = lib.vh_srnl_sequence_forward(
-            hip.ptr(x_c), hip.ptr(q_c), hip.dtype_code(x_c.dtype), *mem_ptrs, per_line,
-            hip.ptr(out), batch, directions, heads, length, head_dim, chunk_ptr,
-            consts, hip.ptr(ws), ws.numel() * 4, hip.stream_of(x_c))
+            x_c.data_ptr(), q_c.data_ptr(), hip.dtype_code(x_c.dtype), *mem_ptrs, per_line,
+            out.data_ptr(), batch, directions, heads, length, head_dim, chunk_ptr,
+            consts, ws.data_ptr(), ws.numel() * 4, hip.stream_of(x_c))
         hip.check(rc, "vh_srnl_sequence_forward")
     else:
         rc = lib.vh_srnl_forward(
-            hip.ptr(x_c), hip.dtype_code(x_c.dtype), hip.ptr(q_c), *mem_ptrs, per_line,
-            hip.ptr(out), batch, directions, heads, length, head_dim, chunk_ptr,
-            consts, hip.ptr(ws), ws.numel() * 4, hip.stream_of(x_c))
+            x_c.data_ptr(), hip.dtype_code(x_c.dtype), q_c.data_ptr(), *mem_ptrs, per_line,
+            out.data_ptr(), batch, directions, heads, length, head_dim, chunk_ptr,
+            consts, ws.data_ptr(), ws.numel() * 4, hip.stream_of(x_c))
         hip.check(rc, "vh_srnl_forward")
     return out
 
@@ -123,7 +126,7 @@ def srnl_packed_backward(memories, x, q, chunk_sizes, dy, *, q_raw):
     dy_c = dy.float().contiguous()
     dx = torch.empty(x_c.shape, device=x.device, dtype=torch.float32)
     dq = torch.empty(q_c.shape, device=x.device, dtype=torch.float32)
-    dmem = [torch.empty_like(m) for m in states]
+    dmem = [torch.empty(m.shape, device=x.device, dtype=torch.float32) for m in memories]
     lib = hip.load_library()
     chunk_ptr, _keep = hip.int64_array(chunks)
     nbytes = lib.vh_srnl_backward_workspace_bytes(batch, directions, heads, length, head_dim, chunk_ptr)
@@ -131,11 +134,11 @@ def srnl_packed_backward(memories, x, q, chunk_sizes, dy, *, q_raw):
         raise ValueError(f"SRNL backward does not cover head_dim={head_dim} with chunks {chunks}")
     ws = hip.workspace(nbytes, x.device)
     hip.check(lib.vh_srnl_backward(
-        hip.ptr(x_c), hip.ptr(q_c), hip.dtype_code(x_c.dtype), int(bool(q_raw)), hip.ptr(dy_c),
-        *[hip.ptr(m) for m in states], per_line, hip.ptr(dx), hip.ptr(dq), *[hip.ptr(m) for m in dmem],
-        batch, directions, heads, length, head_dim, chunk_ptr, srnl_consts(), hip.ptr(ws), ws.numel() * 4,
+        x_c.data_ptr(), q_c.data_ptr(), hip.dtype_code(x_c.dtype), int(bool(q_raw)), dy_c.data_ptr(),
+        *[m.data_ptr() for m in states], per_line, dx.data_ptr(), dq.data_ptr(), *[m.data_ptr() for m in dmem],
+        batch, directions, heads, length, head_dim, chunk_ptr, srnl_consts(), ws.data_ptr(), ws.numel() * 4,
         hip.stream_of(x_c)), "vh_srnl_backward")
-    grads = [g.view(m.shape).to(m.dtype) for g, m in zip(dmem, memories)]
+    grads = [g.to(m.dtype) for g, m in zip(dmem, memories)]
     return (*grads, dx.to(x.dtype), dq.to(q.dtype))
 
 

@@ -9,13 +9,11 @@ channels-last activation and query maps directly (no serialized copies).
 
 from __future__ import annotations
 
-import math
-
 import torch
 
 from .chunk import srnl_consts, srnl_packed_forward
 from ...utils import hip
-from ...utils.cached_params import contiguous_fp32
+from ...utils.cached_params import as_fp32, contiguous_fp32
 from ...utils.cuda import on_tensor_device
 
 _IO_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
@@ -39,23 +37,19 @@ def srnl_spatial_inference(states, x_nhwc, q_nhwc, d_skip, weights, chunks):
     if q_nhwc.shape != x_nhwc.shape or q_nhwc.dtype != x_nhwc.dtype:
         raise ValueError("Spatial SRNL expects x and queries with the same [B, H, W, C] shape and dtype")
     mems = _fp32_states(states)
-    skip = d_skip.detach().float().contiguous()
-    wts = weights.detach().float().contiguous()
+    skip, wts = as_fp32(d_skip), as_fp32(weights)
     if skip.numel() not in (channels, 4 * channels):
         raise RuntimeError("d_skip must contain C or 4*C values")
     x_c = x_nhwc.contiguous()
     q_c = q_nhwc.contiguous()
     out = torch.empty((batch, height, width, channels), device=x_nhwc.device, dtype=torch.float32)
     lib = hip.load_library()
-    length = height * width
-    max_chunks = max(math.ceil(length / int(c)) for c in chunks)
-    ws = hip.workspace(lib.vh_srnl_workspace_bytes(batch * 4 * (channels // head_dim), max_chunks,
-                                                   head_dim), x_nhwc.device)
+    ws = srnl_spatial_workspace(x_c, head_dim, chunks)
     chunk_ptr, _keep = hip.int64_array(chunks)
     hip.check(lib.vh_srnl_spatial_forward(
-        hip.ptr(x_c), hip.ptr(q_c), hip.dtype_code(x_c.dtype), *[hip.ptr(m) for m in mems],
-        hip.ptr(skip), int(skip.numel() == 4 * channels), hip.ptr(wts), hip.ptr(out),
-        batch, height, width, channels, head_dim, chunk_ptr, srnl_consts(), hip.ptr(ws),
+        x_c.data_ptr(), q_c.data_ptr(), hip.dtype_code(x_c.dtype), *[m.data_ptr() for m in mems],
+        skip.data_ptr(), int(skip.numel() == 4 * channels), wts.data_ptr(), out.data_ptr(),
+        batch, height, width, channels, head_dim, chunk_ptr, srnl_consts(), ws.data_ptr(),
         ws.numel() * 4, hip.stream_of(x_c)), "vh_srnl_spatial_forward")
     return out
 
@@ -67,7 +61,7 @@ def _chunk_array(chunks):
 def srnl_spatial_workspace(x_nhwc, head_dim, chunks):
     """An uninitialised workspace for ``srnl_spatial_scan`` of x_nhwc ``[B, H, W, C]``."""
     batch, height, width, channels = x_nhwc.shape
-    max_chunks = max(math.ceil(height * width / int(c)) for c in chunks)
+    max_chunks = -(-height * width // min(int(c) for c in chunks))
     lib = hip.load_library()
     return hip.workspace(lib.vh_srnl_workspace_bytes(batch * 4 * (channels // head_dim), max_chunks, head_dim),
                          x_nhwc.device)
@@ -106,8 +100,7 @@ def srnl_spatial_readout(workspace, x_nhwc, q_nhwc, d_skip, weights, chunks, hea
         raise ValueError("Spatial SRNL expects x and queries with the same [B, H, W, C] shape and dtype")
     if aux is not None and (aux.shape != x_nhwc.shape or aux.dtype != x_nhwc.dtype):
         raise ValueError("The readout addend must match x's shape and dtype")
-    skip = d_skip.detach().float().contiguous()
-    wts = weights.detach().float().contiguous()
+    skip, wts = as_fp32(d_skip), as_fp32(weights)
     x_c, q_c = x_nhwc.contiguous(), q_nhwc.contiguous()
     if lepe is not None:
         taps, bias = lepe
@@ -122,9 +115,9 @@ def srnl_spatial_readout(workspace, x_nhwc, q_nhwc, d_skip, weights, chunks, hea
         lib = hip.load_library()
         chunk_ptr, _keep = _chunk_array(chunks)
         hip.check(lib.vh_srnl_spatial_readout_lepe(
-            hip.ptr(x_c), hip.ptr(q_c), hip.dtype_code(x_c.dtype), hip.ptr(skip), int(skip.numel() == 4 * channels),
-            hip.ptr(wts), hip.ptr(taps_c), hip.ptr(bias_c), hip.ptr(out), batch, height, width, channels, head_dim,
-            chunk_ptr, hip.ptr(workspace), workspace.numel() * 4, hip.stream_of(x_c)),
+            x_c.data_ptr(), q_c.data_ptr(), hip.dtype_code(x_c.dtype), skip.data_ptr(), int(skip.numel() == 4 * channels),
+            wts.data_ptr(), taps_c.data_ptr(), hip.ptr(bias_c), out.data_ptr(), batch, height, width, channels, head_dim,
+            chunk_ptr, workspace.data_ptr(), workspace.numel() * 4, hip.stream_of(x_c)),
             "vh_srnl_spatial_readout_lepe")
         return out
     aux_c = None if aux is None else aux.contiguous()
@@ -132,9 +125,9 @@ def srnl_spatial_readout(workspace, x_nhwc, q_nhwc, d_skip, weights, chunks, hea
     lib = hip.load_library()
     chunk_ptr, _keep = _chunk_array(chunks)
     hip.check(lib.vh_srnl_spatial_readout(
-        hip.ptr(x_c), hip.ptr(q_c), hip.dtype_code(x_c.dtype), hip.ptr(skip), int(skip.numel() == 4 * channels),
-        hip.ptr(wts), hip.ptr(aux_c), hip.ptr(out), hip.dtype_code(out_dtype), batch, height, width, channels,
-        head_dim, chunk_ptr, hip.ptr(workspace), workspace.numel() * 4, hip.stream_of(x_c)),
+        x_c.data_ptr(), q_c.data_ptr(), hip.dtype_code(x_c.dtype), skip.data_ptr(), int(skip.numel() == 4 * channels),
+        wts.data_ptr(), hip.ptr(aux_c), out.data_ptr(), hip.dtype_code(out_dtype), batch, height, width, channels,
+        head_dim, chunk_ptr, workspace.data_ptr(), workspace.numel() * 4, hip.stream_of(x_c)),
         "vh_srnl_spatial_readout")
     return out
 

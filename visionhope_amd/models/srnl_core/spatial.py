@@ -14,6 +14,7 @@ import torch
 from .chunk import BACKWARD_MAX_CHUNK, srnl_consts
 from .fused import srnl_spatial_inference, srnl_spatial_readout, srnl_spatial_workspace
 from ...utils import hip
+from ...utils.cached_params import as_fp32
 from ...utils.cuda import on_tensor_device
 from ...utils.pointwise import EPI_ADD, EPI_BIAS
 
@@ -49,17 +50,12 @@ class SpatialSRNLFunction(torch.autograd.Function):
         return (*srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, gains, dout), None)
 
 
-def _fp32(t):
-    """``t`` as contiguous FP32, itself where it is."""
-    return t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().float().contiguous()
-
-
 @on_tensor_device
 def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
     """The operator's output ``[B, H, W, C]`` FP32 and the gains its backward starts from."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
-    states = [_fp32(m) for m in memories]
+    states = [as_fp32(m) for m in memories]
     x_c = x.contiguous()
     lib = hip.load_library()
     chunk_ptr, _keep = hip.int64_array(chunks)
@@ -79,9 +75,9 @@ def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
     shaped and typed like its input."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
-    states = [_fp32(m) for m in memories]
-    x_c, q_c, g = x.contiguous(), q.contiguous(), _fp32(dout)
-    skip, wts = _fp32(d_skip), _fp32(weights)
+    states = [as_fp32(m) for m in memories]
+    x_c, q_c, g = x.contiguous(), q.contiguous(), as_fp32(dout)
+    skip, wts = as_fp32(d_skip), as_fp32(weights)
     dx, dq = torch.empty_like(x_c), torch.empty_like(q_c)
     grads = [torch.empty_like(t) for t in (*states, skip, wts)]
     lib = hip.load_library()
@@ -143,7 +139,7 @@ class ProjectedSpatialSRNLFunction(torch.autograd.Function):
 def project_queries(x, w, b):
     """The projection's bf16 operands (W, W^T and b, in one buffer) and the queries."""
     channels = x.shape[-1]
-    w, b = _fp32(w), _fp32(b)
+    w, b = as_fp32(w), as_fp32(b)
     operands = torch.empty((2 * channels + 2, channels), device=x.device, dtype=torch.bfloat16)
     q = torch.empty_like(x)
     lib, base, half = hip.load_library(), operands.data_ptr(), 2 * channels * channels

@@ -16,13 +16,19 @@ def contiguous_fp32(t):
     """``t`` as a contiguous FP32 tensor, cached while ``t`` is unchanged.  Covers SRNL
     memories that ``Module.to(memory_format=torch.channels_last)`` relaid out."""
     if t.dtype == torch.float32 and t.is_contiguous():
-        return t.detach()
+        return t
     cached = getattr(t, "_vh_contiguous_fp32", None)
     key = _key(t)
     if cached is None or cached[0] != key:
         cached = (key, t.detach().float().contiguous())
         t._vh_contiguous_fp32 = cached
     return cached[1]
+
+
+def as_fp32(t):
+    """``t`` as contiguous FP32, itself where it is: for operands that kernels read by
+    pointer."""
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().float().contiguous()
 
 
 def linear_weights(module, dtype):

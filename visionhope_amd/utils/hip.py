@@ -188,8 +188,8 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_of(tensor: torch.Tensor):
-    """Current HIP stream of the tensor's device, as a void*."""
-    return ctypes.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
+    """The raw current stream of the tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
 
 
 def ptr(tensor):
@@ -206,7 +206,7 @@ def check(rc: int, what: str):
 
 def int64_array(values):
     arr = (ctypes.c_int64 * len(values))(*[int(v) for v in values])
-    return ctypes.cast(arr, _I64P), arr
+    return arr, arr   # an array argument passes as the pointer
 
 
 def make_consts(step_scale, min_retention, retention_bias, injection_margin, spectral_clamp,
