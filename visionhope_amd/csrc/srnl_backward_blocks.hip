@@ -33,11 +33,13 @@
 // Bound: the dependency chain of a chunk, and within it the issue of the FP32 products, which
 // hold the vector pipe (34 cycles each, srnl_utw.hip); the bytes take under a tenth of the time.
 // Times on MI355X against the token-by-token kernel (which head_dim 4 and 8 still run), gains +
-// backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 80 + 192 us; 512 lines of
-// 3,136 tokens, d = 16, chunks of 56: 24,500 -> 183 + 536 us; 48 lines of 960 tokens, d = 32,
-// chunks of 40 and 24: 11,800 -> 174 + 558 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
-// -> 19 + 57 us.  With the forward repeated inside the backward kernel the first three took 249,
-// 710 and 745 us after a separate forward scan of 54, 125 and 130 us.
+// backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 78 + 186 us; 512 lines of
+// 3,136 tokens, d = 16, chunks of 56: 24,500 -> 185 + 501 us; 48 lines of 960 tokens, d = 32,
+// chunks of 40 and 24: 11,800 -> 174 + 512 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
+// -> 19 + 52 us.  With the forward repeated inside the backward kernel the first three took 249,
+// 710 and 745 us after a separate forward scan of 54, 125 and 130 us; with every wave walking all
+// of a chunk's maps and forming all of H, and transposes as products: 193, 540, 558 and 57 us.
+// Fetching the next chunk's operands ahead changed these by under 3% either way.
 #include <algorithm>
 #include <cmath>
 
@@ -97,6 +99,7 @@ struct Shared {
     Scratch scratch[W];
     // Block maps X, X^T, Y^T of the segment (W > 1); also the waves' partial sums.
     v4f maps[W > 1 ? W : 1][W > 1 ? 3 : 1][NT][64];
+    v4f HT[W > 1 ? NT : 1][W > 1 ? 64 : 1];   // H^T at the chunk's exit
 };
 
 // Everything the recurrence needs from the 16 tokens of one block.
@@ -229,9 +232,9 @@ struct Line {
         for (int i = 0; i < ND; ++i)
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
-                const v4f start = i == j ? bl.diagonal(t.d.a()) : zero;
-                sh.maps[w][0][i * ND + j][bl.lane] = mm(KD[i], S[j], start);
-                sh.maps[w][1][i * ND + j][bl.lane] = mm(S[i], KD[j], start);
+                const v4f x = mm(KD[i], S[j], i == j ? bl.diagonal(t.d.a()) : zero);
+                sh.maps[w][0][i * ND + j][bl.lane] = x;
+                sh.maps[w][1][j * ND + i][bl.lane] = bl.transpose(x);
                 sh.maps[w][2][i * ND + j][bl.lane] = mm(-S[i], t.DlT[j], zero);
             }
     }
@@ -607,11 +610,11 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                     for (int r = 0; r < 4; ++r) Gam[i][j][r] = src[(16 * i + 4 * g + r) * D + 16 * j + c];
                 }
         }
-        v4f Ep[ND][ND], EG[ND][ND];   // this wave's part of dGamma_c; its tiles of dGamma_{c+1} G_C^T
+        v4f Ep[ND][ND];   // this wave's part of dGamma_c; dGamma_{c+1} G_C^T is in the last wave's
 #pragma unroll
         for (int i = 0; i < ND; ++i)
 #pragma unroll
-            for (int j = 0; j < ND; ++j) Ep[i][j] = EG[i][j] = zero;
+            for (int j = 0; j < ND; ++j) Ep[i][j] = zero;
 
         // Gradients of this wave's block (chunk block blk) from the adjoint H of its exit
         // gain; GTb: the transposed gain at its start (the identity when W is 1).
@@ -661,12 +664,10 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
             const float d_apre = valid ? d_alpha * t.s_alpha : 0.f;
             const float d_epre = d_eff * t.deff_deta * t.s_eta;
             const float cdn = -d_cap * t.cap * t.inv_denom * rcp1(t.dn), cks = 2.f * d_eff * t.deff_dksq;
-            v4f P = zero, PT = zero, Ws;
+            v4f P = zero, Ws;
 #pragma unroll
-            for (int i = 0; i < ND; ++i) {
-                P = mm(R[i], Rb[i], P);
-                PT = mm(Rb[i], R[i], PT);
-            }
+            for (int i = 0; i < ND; ++i) P = mm(R[i], Rb[i], P);
+            const v4f PT = bl.transpose(P);
 #pragma unroll
             for (int r = 0; r < 4; ++r) Ws[r] = bl.row_time(r) < tau ? P[r] : PT[r];
             Ws = bl.decayed(t.d, Ws);
@@ -729,6 +730,12 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
         };
 
         if (ch < nc - 1) {
+            auto e_rows = [&](int m, int i) {   // tile (m, i) of dGamma_{c+1}
+                v4f e;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e[r] = sh.E[16 * m + 4 * g + r][16 * i + c];
+                return e;
+            };
             Tok t;
             v4f X[ND], RT[ND], GT[ND][ND], HT[ND][ND], H[ND][ND];
             v4f GTb[ND][ND];   // G^T at the start of this wave's block of the segment
@@ -743,6 +750,17 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                     for (int j = 0; j < ND; ++j)
                         GT[i][j] = mm(t.d.De_r() * t.KT[i], -RT[j], i == j ? bl.diagonal(t.d.a()) : zero);
             } else {
+                // H^T at the chunk's exit, Gamma^T dGamma_{c+1}: a tile per wave, shared
+#pragma unroll
+                for (int i = 0; i < ND; ++i)
+#pragma unroll
+                    for (int j = 0; j < ND; ++j)
+                        if (W - 1 - (i * ND + j) % W == w) {
+                            v4f h = zero;
+#pragma unroll
+                            for (int m = 0; m < ND; ++m) h = mm(e_rows(m, i), Gam[m][j], h);
+                            sh.HT[i * ND + j][lane] = h;
+                        }
                 identity(GT);
                 for (int seg = 0; seg < nseg; ++seg) {
                     const int nbs = min(W, nb - seg * W);
@@ -757,31 +775,34 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
                         L.store_maps(t);
                     }
                     __syncthreads();
-                    for (int blk = 0; blk < nbs; ++blk) {
+                    // Up to this wave's block; the whole product for a following segment and, on
+                    // the last wave, for dGamma_{c+1} G_C^T.  (The adjoint below is the other way
+                    // round, so no wave walks the chunk twice.)
+                    const int upto = w == W - 1 || seg + 1 < nseg ? nbs : w < nbs ? w : 0;
+                    for (int blk = 0; blk < upto; ++blk) {
                         if (blk == w) copy_tiles(GT, GTb);
                         L.apply_map(blk, GT);
                     }
+                    if (upto == w) copy_tiles(GT, GTb);
                 }
             }
             // dGamma_{c+1} G_C^T and the adjoint of the chunk gain, dG_C = Gamma^T dGamma_{c+1}
 #pragma unroll
             for (int i = 0; i < ND; ++i)
 #pragma unroll
-                for (int j = 0; j < ND; ++j) HT[i][j] = H[i][j] = zero;
+                for (int j = 0; j < ND; ++j) {
+                    if constexpr (W == 1) {
+                        HT[i][j] = zero;
 #pragma unroll
-            for (int m = 0; m < ND; ++m)
-#pragma unroll
-                for (int i = 0; i < ND; ++i) {
-                    v4f e;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) e[r] = sh.E[16 * m + 4 * g + r][16 * i + c];
-                    const v4f et = *reinterpret_cast<const v4f*>(&sh.E[16 * i + c][16 * m + 4 * g]);
-#pragma unroll
-                    for (int j = 0; j < ND; ++j) {
-                        HT[i][j] = mm(e, Gam[m][j], HT[i][j]);
-                        if constexpr (W == 1) H[j][i] = mm(Gam[m][j], e, H[j][i]);
-                        if ((i * ND + j) % W == w) EG[i][j] = mm(et, GT[m][j], EG[i][j]);
+                        for (int m = 0; m < ND; ++m) HT[i][j] = mm(e_rows(m, i), Gam[m][j], HT[i][j]);
+                        H[j][i] = bl.transpose(HT[i][j]);
+                    } else {
+                        HT[i][j] = sh.HT[i * ND + j][lane];
                     }
+                    if (W == 1 || w == W - 1)
+#pragma unroll
+                        for (int m = 0; m < ND; ++m)
+                            Ep[i][j] = mm(*reinterpret_cast<const v4f*>(&sh.E[16 * i + c][16 * m + 4 * g]), GT[m][j], Ep[i][j]);
                 }
             if constexpr (W == 1) {
                 block_gradients(0, t, X, valid, RT, t.KT, GT, HT, H);
@@ -892,7 +913,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
             }
         }
 
-        // dGamma_c: the waves' parts and dGamma_{c+1} G_C^T, in wave order.
+        // dGamma_c: the waves' parts, in wave order.
         if constexpr (W > 1) {
             __syncthreads();   // every wave has read the maps and dGamma_{c+1}
 #pragma unroll
@@ -904,8 +925,8 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
 #pragma unroll
             for (int j = 0; j < ND; ++j)
                 if ((i * ND + j) % W == w) {
-                    v4f e = EG[i][j];
-                    if constexpr (W == 1) e += Ep[i][j];
+                    v4f e = zero;
+                    if constexpr (W == 1) e = Ep[i][j];
                     else
                         for (int v = 0; v < W; ++v) e += sh.maps[v][0][i * ND + j][lane];
 #pragma unroll
