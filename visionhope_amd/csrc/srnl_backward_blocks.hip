@@ -35,10 +35,12 @@
 // Times on MI355X against the token-by-token kernel (which head_dim 4 and 8 still run), gains +
 // backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 78 + 186 us; 512 lines of
 // 3,136 tokens, d = 16, chunks of 56: 24,500 -> 185 + 501 us; 48 lines of 960 tokens, d = 32,
-// chunks of 40 and 24: 11,800 -> 174 + 512 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
+// chunks of 40 and 24: 11,800 -> 174 + 424 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
 // -> 19 + 52 us.  With the forward repeated inside the backward kernel the first three took 249,
 // 710 and 745 us after a separate forward scan of 54, 125 and 130 us; with every wave walking all
 // of a chunk's maps and forming all of H, and transposes as products: 193, 540, 558 and 57 us.
+// The third also has waves without a block of their own, which take the readout's gradients
+// while the others form theirs (512 us with each wave doing its own block's afterwards).
 // Fetching the next chunk's operands ahead changed these by under 3% either way.
 #include <algorithm>
 #include <cmath>
@@ -850,7 +852,10 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
         }
 
         // Readout: y = M_m Gamma q^ of every token of the chunk.
-        for (int blk = w; blk < nb; blk += W) {
+        // Waves without a block of the chunk take it, while the others are in their gradients.
+        const int idle = ch < nc - 1 ? W - nb : 0;
+        const int first = idle <= 0 ? w : w >= nb ? w - nb : nb;
+        for (int blk = first; blk < nb; blk += idle > 0 ? idle : W) {
             const int tl = 16 * blk + tau;
             const Index tok = ch * C + tl;
             const bool valid = tl < C && tok < N;
