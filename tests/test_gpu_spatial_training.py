@@ -34,7 +34,9 @@ def _oracle(x, q, mems, skip, weights, chunks, dout, head_dim):
 @pytest.mark.parametrize("shape,head_dim,chunks,per_direction,offset", [
     ((2, 5, 7, 32), 16, None, False, 0), ((1, 16, 17, 48), 16, None, True, 1), ((1, 3, 33, 96), 32, None, True, 0),
     ((2, 1, 9, 16), 16, None, False, 3), ((1, 6, 6, 32), 32, (7, 7, 7, 7), False, 0),
-    ((1, 2, 70, 16), 16, None, False, 0)])
+    ((1, 2, 70, 16), 16, None, False, 0),
+    ((32, 2, 35, 32), 16, None, False, 0), ((33, 2, 35, 32), 16, None, False, 0),        # 256 lines: spare waves; 264
+    ((64, 17, 3, 32), 32, None, False, 0), ((65, 17, 3, 32), 32, None, False, 0)])
 def test_spatial_backward_matches_oracle(device, shape, head_dim, chunks, per_direction, offset, dtype):
     """Odd and single-row maps, several blocks per row, explicit chunk lengths, both skip
     layouts, tensors that start at an odd element.  FP32: the roundings of at most one

@@ -49,7 +49,7 @@ __device__ __forceinline__ float softcap_dcap(float u, float e_neg) {
 
 // Block form (head_dim 16 and 32): waves per line for the longest chunk, and the segments
 // of 16 * waves tokens that chunk takes.
-int bwd_block_waves(int head_dim, int64_t max_chunk);
+int bwd_block_waves(int head_dim, int64_t max_chunk, int64_t lines);
 inline int bwd_block_segs(int waves, int64_t max_chunk) { return static_cast<int>((max_chunk + 16 * waves - 1) / (16 * waves)); }
 int launch_backward_gains(const BwdParams& p, bool spatial, int head_dim, int waves, int64_t lines, hipStream_t stream);
 int launch_backward_blocks(const BwdParams& p, int head_dim, int waves, int64_t lines, hipStream_t stream);

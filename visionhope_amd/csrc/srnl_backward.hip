@@ -623,7 +623,7 @@ BwdLayout bwd_layout(int64_t B, int64_t R, int64_t heads, int64_t N, int d, cons
     int64_t cmax = 0;
     for (int64_t r = 0; r < R; ++r) cmax = std::max<int64_t>(cmax, chunks[r]);
     if (d >= 16) {
-        l.waves = bwd_block_waves(d, cmax);
+        l.waves = bwd_block_waves(d, cmax, l.lines);
         l.segs = bwd_block_segs(l.waves, cmax);
         l.states = round(static_cast<size_t>(l.lines * l.nc * d * d));
         l.traj = l.segs > 1 ? round(static_cast<size_t>(l.lines * l.waves * l.segs * d * d)) : 0;
