@@ -2,10 +2,10 @@
 activations, through the spatial operator (``vh_srnl_spatial_forward``, FP32 output) and
 the sequence entry, against the C oracle on the same inputs.
 
-Each shape selects one kernel of the library's own dispatch: the one-wave block form with
-its 2 x 2 and 1 x 4 packings (4096 and 1024 lines, head_dim 16), the few-line form with a
-chunk's blocks over 1 or 2 waves (head_dim 16, fewer than 1024 lines) and the head_dim-32
-form with chunks of 14 and 56 tokens (1 and 4 waves).  fp16 values are exact as bf16 hi + lo
+Each shape runs the library's own dispatch: one workgroup per line with a chunk's blocks over
+1 or 2 waves (head_dim 16: chunks of one block, or few lines), the packed one-wave form (2,048
+lines with longer chunks, in the edge cases) and the head_dim-32 form with chunks of 14 and 56
+tokens (1 and 4 waves).  fp16 values are exact as bf16 hi + lo
 operands and FP32 values enter within 2^-16 of their value, so both are held to the bound of
 the bf16 block form, 2e-5 (about one hi + lo rounding of the output, five times inside the
 FP32 contract of 1e-4; observed on MI355X: 5e-8 normwise with default-scale memories, up to
@@ -25,8 +25,8 @@ FP16_OUT_TOL = 2e-3  # fp16 output of the sequence entry: one fp16 rounding (2^-
 
 # (batch, H = W, heads, head_dim): kernel chosen by the default dispatch
 SHAPES = [
-    (64, 14, 16, 16),   # 4096 lines: one-wave block form, 2 x 2 packing
-    (32, 14, 8, 16),    # 1024 lines: one-wave block form, 1 x 4 packing
+    (64, 14, 16, 16),   # 4096 lines, one block per chunk
+    (32, 14, 8, 16),    # 1024 lines, one block per chunk
     (4, 28, 4, 16),     # 64 lines, chunks of 28: few-line form, 2 waves per line
     (8, 14, 4, 32),     # head_dim 32, chunks of 14: one wave per line
     (2, 56, 2, 32),     # head_dim 32, chunks of 56: four waves per line
