@@ -12,7 +12,7 @@ four scan orders, scans, reads out, restores and fuses in separate passes (refer
 import torch
 
 from .chunk import BACKWARD_MAX_CHUNK, srnl_consts
-from .fused import srnl_spatial_inference, srnl_spatial_readout, srnl_spatial_workspace
+from .fused import srnl_spatial_readout, srnl_spatial_workspace
 from ...utils import hip
 from ...utils.cached_params import as_fp32
 from ...utils.cuda import on_tensor_device
@@ -180,13 +180,10 @@ def _check_merge(x_nhwc, d_skip, weights):
 
 
 def srnl_spatial(memories, x_nhwc, q_nhwc, d_skip, weights, chunks):
-    """Differentiable spatial operator (``spatial_training_supported``)."""
+    """Differentiable spatial operator (``spatial_training_supported``).  The Function runs
+    without gradients too: it is what refuses tracing and forward-mode derivatives, and a
+    checkpointed step repeats its forward with the same kernels."""
     _check_merge(x_nhwc, d_skip, weights)
-    if not (torch.is_grad_enabled() and any(t.requires_grad for t in (*memories, x_nhwc, q_nhwc, d_skip, weights))):
-        # nothing to differentiate: the inference scan, which keeps nothing
-        if torch.jit.is_tracing():
-            raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
-        return srnl_spatial_inference(memories, x_nhwc, q_nhwc, d_skip, weights, chunks)
     return SpatialSRNLFunction.apply(*memories, x_nhwc, q_nhwc, d_skip, weights, tuple(int(c) for c in chunks))
 
 
