@@ -6,6 +6,7 @@ import pytest
 import torch
 from torch.autograd import forward_ad
 
+from visionhope_amd.models import VisionHOPEOperator, operator as operator_module
 from visionhope_amd.models.srnl_core import spatial
 
 HEADS, HEAD_DIM = 2, 16
@@ -62,3 +63,34 @@ def test_one_forward_with_and_without_gradients(calls):
             assert not spatial.srnl_spatial(*args).requires_grad
         assert spatial.srnl_spatial(*args).requires_grad == requires_grad
     assert calls == ["training"] * 4
+
+
+@pytest.fixture
+def operator(monkeypatch):
+    """An operator whose spatial training entries return x and record their map and queries."""
+    seen = []
+    monkeypatch.setattr(operator_module, "spatial_training_supported", lambda *_: True)
+    monkeypatch.setattr(operator_module, "projected_training_supported", lambda *_: True)
+    monkeypatch.setattr(operator_module, "srnl_spatial",
+                        lambda m, x, q, *_: seen.append(("module", x, q)) or x.float().clone())
+    monkeypatch.setattr(operator_module, "srnl_spatial_projected",
+                        lambda m, x, *_: seen.append(("projected", x, None)) or x.float().clone())
+    op = VisionHOPEOperator(HEADS * HEAD_DIM, HEAD_DIM).train()
+    op.seen = seen
+    return op
+
+
+def _channels_last():
+    return torch.randn(2, HEADS * HEAD_DIM, 3, 5).contiguous(memory_format=torch.channels_last)
+
+
+def test_query_projection_may_be_any_module(operator):
+    """``W_q`` replaced by a module without a ``weight`` of its own (an adapter around the
+    Linear, say): the call goes through, and the map kept for the backward is a copy, since
+    no Linear is known to keep it."""
+    operator.W_q = torch.nn.Sequential(operator.W_q, torch.nn.Identity())
+    x = _channels_last()
+    operator(x)
+    (route, kept, q), = operator.seen
+    assert route == "module" and kept.data_ptr() != x.data_ptr()
+    assert torch.equal(q, operator.W_q(x.permute(0, 2, 3, 1)))

@@ -183,7 +183,7 @@ class VisionHOPEOperator(nn.Module):
                 if spatial_training_supported(x, q_hw, self.head_dim, chunks):
                     states = self.srnl._validate_memories(x.device)
                     x_nhwc = x_nhwc.contiguous()
-                    if x_nhwc.data_ptr() == x.data_ptr() and not self.W_q.weight.requires_grad:
+                    if x_nhwc.data_ptr() == x.data_ptr() and not self._projection_keeps_x():
                         x_nhwc = x_nhwc.clone()   # nothing else keeps x for the backward: the caller may overwrite it
                     out = srnl_spatial(states, x_nhwc, q_hw.reshape(batch, height, width, self.dim),
                                        self.d_skip.float(), self.direction_weights().float(), chunks)
@@ -214,12 +214,15 @@ class VisionHOPEOperator(nn.Module):
                 and "project_queries" not in self.__dict__ and "forward" not in self.srnl.__dict__
                 and not _observed(self.srnl))
 
+    def _projection_keeps_x(self):
+        """Whether autograd keeps x for the gradient of ``W_q``: a plain Linear in training."""
+        return type(self.W_q) is nn.Linear and self.W_q.weight.requires_grad
+
     def _projection_fused(self, x, x_nhwc, chunks):
         """Whether a training step runs ``W_q`` inside the spatial Function: a plain Linear
-        whose calls nothing watches, with everything differentiable in the usual case (its
-        weight trained, so that autograd's own linear would keep x as it is, too)."""
-        return (torch.is_grad_enabled() and type(self.W_q) is nn.Linear and "forward" not in self.W_q.__dict__
-                and not _observed(self.W_q) and self.W_q.bias is not None and self.W_q.weight.requires_grad
+        whose calls nothing watches and whose gradient would keep x, too."""
+        return (torch.is_grad_enabled() and self._projection_keeps_x() and "forward" not in self.W_q.__dict__
+                and not _observed(self.W_q) and self.W_q.bias is not None
                 and spatial_training_supported(x, x, self.head_dim, chunks)
                 and projected_training_supported(x_nhwc, self.W_q))
 
