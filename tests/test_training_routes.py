@@ -94,3 +94,17 @@ def test_query_projection_may_be_any_module(operator):
     (route, kept, q), = operator.seen
     assert route == "module" and kept.data_ptr() != x.data_ptr()
     assert torch.equal(q, operator.W_q(x.permute(0, 2, 3, 1)))
+
+
+@pytest.mark.parametrize("frozen", [True, False])
+def test_projection_route_does_not_depend_on_gradients(operator, frozen):
+    """The same projection with and without gradients, and no copy of the map where nothing
+    is kept for a backward."""
+    operator.W_q.requires_grad_(not frozen)
+    x = _channels_last()
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            operator(x)
+    (route, without, _), (route_grad, _, _) = operator.seen
+    assert route == route_grad == ("module" if frozen else "projected")
+    assert without.data_ptr() == x.data_ptr()

@@ -183,7 +183,7 @@ class VisionHOPEOperator(nn.Module):
                 if spatial_training_supported(x, q_hw, self.head_dim, chunks):
                     states = self.srnl._validate_memories(x.device)
                     x_nhwc = x_nhwc.contiguous()
-                    if x_nhwc.data_ptr() == x.data_ptr() and not self._projection_keeps_x():
+                    if torch.is_grad_enabled() and x_nhwc.data_ptr() == x.data_ptr() and not self._projection_keeps_x():
                         x_nhwc = x_nhwc.clone()   # nothing else keeps x for the backward: the caller may overwrite it
                     out = srnl_spatial(states, x_nhwc, q_hw.reshape(batch, height, width, self.dim),
                                        self.d_skip.float(), self.direction_weights().float(), chunks)
@@ -219,9 +219,10 @@ class VisionHOPEOperator(nn.Module):
         return type(self.W_q) is nn.Linear and self.W_q.weight.requires_grad
 
     def _projection_fused(self, x, x_nhwc, chunks):
-        """Whether a training step runs ``W_q`` inside the spatial Function: a plain Linear
-        whose calls nothing watches and whose gradient would keep x, too."""
-        return (torch.is_grad_enabled() and self._projection_keeps_x() and "forward" not in self.W_q.__dict__
+        """Whether the ordinary path runs ``W_q`` inside the spatial Function: a plain Linear
+        whose calls nothing watches and whose gradient would keep x, too.  With gradients
+        enabled or not: a checkpointed step must find the queries of its first forward again."""
+        return (self._projection_keeps_x() and "forward" not in self.W_q.__dict__
                 and not _observed(self.W_q) and self.W_q.bias is not None
                 and spatial_training_supported(x, x, self.head_dim, chunks)
                 and projected_training_supported(x_nhwc, self.W_q))
