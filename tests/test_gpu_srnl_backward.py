@@ -300,3 +300,37 @@ def test_srnl_backward_block_inputs(device, head_dim, directions, dtype):
     chunks = [19, 40][:directions]
     _block_form_case(device, head_dim, chunks, 90, heads=3, batch=2, dtype=dtype, offset=1)
     _block_form_case(device, head_dim, chunks, 90, dtype=dtype, kind="strong", gate_scale=4.0, offset=3, q_raw=False)
+
+
+@pytest.mark.parametrize("head_dim", [16, 32])
+def test_retention_products_of_saturated_gates(device, head_dim):
+    """The gain of a chunk of 16 tokens whose keys are zero is the product of its retentions
+    times the identity: 2^-100 here, in every entry within the roundings of 16 gates (three
+    each: the exponential, the sum and the reciprocal) and of the five products.  As a
+    difference of sums of logarithms it would carry 2^-24 of 100."""
+    from visionhope_amd.models.srnl_core import chunk
+    from visionhope_amd.models.srnl_core.spatial import srnl_spatial_training_forward
+
+    heads, tokens, batch = 4, 16, 8
+    channels = heads * head_dim
+    gen = torch.Generator().manual_seed(head_dim)
+    gates = -7.0 + torch.rand(4, heads, head_dim, generator=gen)
+    mats = [torch.randn(4, heads, head_dim, head_dim, generator=gen), *torch.zeros(2, 4, heads, head_dim, head_dim)]
+    # token t of a row selects gate entry perm[t]; two rows, so that a second chunk exists
+    perms = torch.stack([torch.randperm(head_dim, generator=gen)[:tokens] for _ in range(batch * heads)])
+    x = torch.zeros(batch, 2, tokens, heads, head_dim)
+    for i, perm in enumerate(perms):
+        x[i // heads, :, torch.arange(tokens), i % heads, perm] = 1.0
+    x = x.reshape(batch, 2, tokens, channels)
+    mems = [m.to(device) for m in (*mats, torch.zeros_like(gates), gates)]
+    _, gains = srnl_spatial_training_forward(mems, x.to(device), x.to(device), torch.zeros(channels, device=device),
+                                             torch.ones(4, channels, device=device), (tokens,) * 4)
+    gains = gains.cpu()[:batch * 4 * heads * 2 * head_dim ** 2].double()
+    got = gains.reshape(batch, 4, heads, 2, head_dim, head_dim)[:, 0, :, 1]
+    bias = np.float32(chunk.RETENTION_BIAS)
+    for i, perm in enumerate(perms):
+        pre = (gates[0, i % heads, perm].numpy() + bias).astype(np.float64)
+        retention = chunk.MIN_RETENTION + (1 - chunk.MIN_RETENTION) / (1 + np.exp(-pre))
+        want = torch.eye(head_dim, dtype=torch.float64) * retention.prod()
+        bound = (3 * tokens + 5) * 2.0 ** -24 * retention.prod()
+        assert (got[i // heads, i % heads] - want).abs().max() <= bound

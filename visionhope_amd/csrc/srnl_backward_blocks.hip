@@ -77,12 +77,8 @@ __device__ __forceinline__ void store_io4(void* p, int64_t idx, int io, v4f v) {
     *reinterpret_cast<us4_any*>(static_cast<uint16_t*>(p) + idx) = u;
 }
 
-// 1 / x and e^x within about one ulp for the normal ranges met here, in 3 and 6 instructions
-// (hardware approximation and one correction) instead of the library's 10 and more.
-__device__ __forceinline__ float rcp1(float x) {
-    const float r = __builtin_amdgcn_rcpf(x);
-    return fmaf(fmaf(-x, r, 1.f), r, r);
-}
+// e^x within about one ulp for the normal ranges met here, in 6 instructions (hardware
+// approximation and one correction) instead of the library's 10 and more.
 __device__ __forceinline__ float exp1(float x) {
     constexpr float kLog2e = 1.44269504088896341f, kLog2eLow = 1.925963033500e-8f, kLn2 = 0.69314718055994531f;
     const float t = x * kLog2e, rest = fmaf(x, kLog2e, -t) + x * kLog2eLow, e = __builtin_amdgcn_exp2f(t);
@@ -659,7 +655,7 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
             }
             rr = xor16_32_sum(rr);
             rd = xor16_32_sum(rd);
-            const float phi = phi0 + time_prefix(rd, c).incl;
+            const float phi = phi0 + time_prefix(rd, c);
             const float d_eff = t.eff > 0.f ? rr * rcp1(t.eff) : 0.f;
             const float d_cap = d_eff * t.deff_dcap;
             const float d_alpha = (phi - rr) * rcp1(t.alpha) - d_cap * p.k.injection_margin * t.inv_denom + d_eff * t.deff_dalpha;
