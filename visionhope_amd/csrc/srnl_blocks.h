@@ -42,23 +42,6 @@ __device__ __forceinline__ float rcp1(float x) {
     return fmaf(fmaf(-x, r, 1.f), r, r);
 }
 
-// Inclusive prefix sum over the 16 slots of a block in time order (slot c = time 4 (c % 4) +
-// c / 4), the same in every row of lanes.
-__device__ __forceinline__ float time_prefix(float v, int c) {
-    float in = v + dpp0<0x114>(v);              // row_shr 4: the previous time of the same group of four
-    in += dpp0<0x118>(in);                      // row_shr 8
-    float t = v + dpp0<0x128>(v);               // row_ror 8, 4: the group's total
-    t += dpp0<0x124>(t);
-    // every lane moves before the selects: a move inside a branch would read inactive lanes
-    const int j = c & 3;
-    const float t1 = dpp0<0x90>(t);             // quad_perm [0, 0, 1, 2]
-    float s = t + (j >= 1 ? t1 : 0.f);
-    const float s2 = dpp0<0x40>(s);             // quad_perm [0, 0, 0, 1]
-    s += j >= 2 ? s2 : 0.f;
-    const float s1 = dpp0<0x90>(s);
-    return (j >= 1 ? s1 : 0.f) + in;
-}
-
 // Wave-private LDS of a block.
 struct Scratch {
     float tr[16 * kTrStride];   // transposes
@@ -120,6 +103,15 @@ struct Block {
         return r;
     }
     __device__ __forceinline__ v4f rows_of(const float* p) const { return *reinterpret_cast<const v4f*>(p + 4 * g); }
+    // Two values per slot column (the same in every row of lanes) as those of the lane's rows.
+    __device__ __forceinline__ void rows(float u, float v, v4f& u_r, v4f& v_r) const {
+        s.sc[0][c] = u;
+        s.sc[1][c] = v;
+        __builtin_amdgcn_wave_barrier();
+        u_r = rows_of(s.sc[0]);
+        v_r = rows_of(s.sc[1]);
+        __builtin_amdgcn_wave_barrier();
+    }
     __device__ __forceinline__ int row_time(int i) const { return 4 * i + g; }
     __device__ __forceinline__ v4f diagonal(float v) const {   // v I as a tile
         v4f r;
@@ -143,12 +135,7 @@ struct Block {
         const float num = j == 3 ? t2 : 1.f, den = j == 0 ? d.head : j == 1 ? t1 : 1.f;
         d.kappa = num * excl * rcp1(den);
         d.rho = eff * den * rcp1(num * incl);
-        s.sc[0][c] = d.rho;
-        s.sc[1][c] = d.kappa;
-        __builtin_amdgcn_wave_barrier();
-        d.rho_r = rows_of(s.sc[0]);
-        d.kappa_r = rows_of(s.sc[1]);
-        __builtin_amdgcn_wave_barrier();
+        rows(d.rho, d.kappa, d.rho_r, d.kappa_r);
         return d;
     }
     // v scaled by eta^_s a_t / a_{s+1} of the earlier slot s and the later slot t of (row,
