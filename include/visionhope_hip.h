@@ -74,7 +74,7 @@ const char* vh_last_error(void);
  *                                     blocks over the waves of one workgroup per line, never /
  *                                     whenever the chunks allow (default: head_dim 16 chunks
  *                                     of up to 16, or below 2048 lines, up to 128; head_dim 32
- *                                     always, chunks up to 128)
+ *                                     always, chunks up to 128, up to 64 of fp16 and FP32 x)
  *   pw_cfg, pw_resident               1x1 convolution kernel variants
  *   dw_tile, dw_tile_cs, dw_tile_p, dw_launch_bytes   depthwise kernel variants
  *   ln_stage         "0" | "1"        LayerNorm staged stores

@@ -132,8 +132,9 @@ def test_line_per_workgroup_scan_edges(oracle, device, batch, height, width, hea
     (1, 5, 127, 2), (1, 128, 3, 1), (64, 16, 16, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_line_per_workgroup_scan_edges_wide_heads(oracle, device, batch, height, width, heads, dtype):
-    """The same at head_dim 32: 1 to 8 blocks per chunk, full, ragged and single-token, rows and
-    columns with different wave counts."""
+    """The same at head_dim 32: 1 to 8 blocks per chunk (fp16 and FP32 maps with more than 4 run
+    the stepped and the wide scan), full, ragged and single-token, rows and columns with
+    different wave counts."""
     from visionhope_amd.models.srnl_core.fused import srnl_spatial_inference
 
     channels = 32 * heads
@@ -146,3 +147,24 @@ def test_line_per_workgroup_scan_edges_wide_heads(oracle, device, batch, height,
     expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 32)
     r, m = rel_err(got, expected), max_rel_err(got, expected)
     assert r <= BLOCK_TOL and m <= BLOCK_TOL, f"{dtype} {height}x{width}: normwise {r:.3e}, elementwise {m:.3e}"
+
+
+@pytest.mark.parametrize("batch,height,width,heads", [(1, 65, 65, 2), (1, 100, 80, 2), (1, 128, 128, 1)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_wide_heads_long_chunks_keep_fp32_products(oracle, device, batch, height, width, heads, dtype):
+    """head_dim 32, chunks of 65 to 128 tokens of fp16 and FP32 maps, saturated gates: FP32
+    products throughout.  The output is two chained sums of 32 FP32 products, so with random
+    roundings it is within sqrt(2 x 32) 2^-24 normwise (observed 1.6e-7); operands split into
+    bf16 hi + lo gave 7e-7 to 1.1e-6 for the first two maps."""
+    from visionhope_amd.models.srnl_core.fused import srnl_spatial_inference
+
+    channels = 32 * heads
+    seed = 1000 * height + width
+    mems = list(memories(4, heads, 32, kind="strong", seed=seed))
+    mems[3:] = [4.0 * m for m in mems[3:]]
+    x, q = (randn(batch, height, width, channels, seed=7 * height + width + i).to(dtype) for i in (1, 2))
+    skip, wts = torch.zeros(channels), torch.ones(4, channels)
+    got = srnl_spatial_inference(tuple(torch.from_numpy(m).to(device) for m in mems), x.to(device), q.to(device),
+                                 skip.to(device), wts.to(device), (width, width, height, height)).cpu().numpy()
+    expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 32)
+    assert rel_err(got, expected) <= 64 ** 0.5 * 2.0 ** -24

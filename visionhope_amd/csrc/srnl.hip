@@ -1326,10 +1326,11 @@ void launch_scan(const ScanParams& sp, hipStream_t stream) {
         }
         if constexpr (D == 32) {
             // head_dim 32: the block form with one workgroup per line (srnl_utw32.hip) for
-            // chunks of up to 128 tokens (ahead of the wide scan at every line count measured, 8 to
-            // 4,096: 1.25 times at 4,096 lines of 40, 2.6 at 8 lines of 128; 2,048
-            // lines of 80: 2,316 against 3,378 us), unless an override forces the wide scan (scan_wide),
-            // the stepped forms (scan_ut "0") or turns it off (scan_utw "0").
+            // chunks of up to 128 tokens of bf16 maps (ahead of the wide scan at every line count
+            // measured, 8 to 4,096: 1.25 times at 4,096 lines of 40, 2.6 at 8 lines of 128; 2,048
+            // lines of 80: 2,316 against 3,378 us) and up to 64 of fp16 and FP32 ones (longer chunks
+            // keep FP32 products), unless an override forces the wide scan (scan_wide), the stepped
+            // forms (scan_ut "0") or turns it off (scan_utw "0").
             const Override utw("scan_utw");
             const bool utw_on = !(utw.set() && utw.value[0] == '0');
             if (utw_on && scan_ut_enabled() && !Override("scan_wide").set() && launch_scan32_utw<T>(sp, stream))

@@ -372,8 +372,8 @@ bool launch_scan16_ut(const ScanParams& sp, hipStream_t stream);
 // launched) when the chunks or the input alignment do not allow it.
 template <typename T>
 bool launch_scan16_utw(const ScanParams& sp, hipStream_t stream);
-// head_dim 32, chunks of at most 128 tokens (srnl_utw32.hip); false when the call does not
-// qualify.
+// head_dim 32, chunks of at most 128 tokens (64 unless bf16; srnl_utw32.hip); false when the
+// call does not qualify.
 template <typename T>
 bool launch_scan32_utw(const ScanParams& sp, hipStream_t stream);
 bool launch_scan_wide(const ScanParams& sp, int io_dtype, int head_dim, int waves, int token_blocks,

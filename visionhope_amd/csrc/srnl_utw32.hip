@@ -15,8 +15,12 @@
 // carried the whole 112 x 32 state, solved (I + L) by columns on the vector unit and met at
 // a barrier for every block of a chunk: 384 lines of 3,136 tokens (chunks of 56) 274 -> 204 us,
 // 128 lines 215 -> 149, 1,024 lines of 784 (28) 222 -> 110, 4,096 of 196 (14) 212 -> 102, 8 of
-// 196 (14) 50 -> 33; with chunks of more than 64 tokens (8 waves, one workgroup per CU; it was
-// the wide scan) 1,024 lines of 6,400 (80) 1,692 -> 1,157, 384 of 16,384 (128) 1,699 -> 1,018.
+// 196 (14) 50 -> 33; bf16 with chunks of more than 64 tokens (8 waves, one workgroup per CU; it
+// was the wide scan) 1,024 lines of 6,400 (80) 1,692 -> 1,157, 384 of 16,384 (128) 1,699 -> 1,018.
+// Those lines of fp16 and FP32 keep the stepped and the wide scan: their products are FP32, and
+// this form's split operands were 1.1 (small gates) to 7 times (saturated ones) as far from 64
+// bits (maps of 65 x 65 to 128 x 128).  A bf16 map's error is that of its split chunk states
+// either way (2.5e-6, within 1%).
 #include <algorithm>
 
 #include "srnl_block_form.h"
@@ -281,13 +285,18 @@ __global__ __launch_bounds__(64 * W, 2) void srnl_scan32_utw_kernel(const ScanPa
 }
 
 // Waves per line of the head_dim-32 block-form scan: the chunk's 16-slot blocks rounded up to
-// a power of two; 0 when a chunk exceeds 8 blocks (128 tokens) or the input rows are not
-// aligned for vector loads.
+// a power of two; 0 when a chunk exceeds 8 blocks (128 tokens; 4 blocks for fp16 and FP32
+// activations, whose longer chunks keep FP32 products) or the input rows are not aligned for
+// vector loads.
+template <typename T>
+constexpr int kMaxBlocks = std::is_same<T, bf16_t>::value ? 8 : 4;
+
+template <typename T>
 int scan32_utw_waves(const ScanParams& sp) {
     int max_chunk = 0;
     for (int r = 0; r < sp.R; ++r) max_chunk = std::max(max_chunk, sp.chunk[r]);
     const int blocks = (max_chunk + 15) / 16;
-    if (blocks > 8 || !sp.x_vec) return 0;
+    if (blocks > kMaxBlocks<T> || !sp.x_vec) return 0;
     int w = 1;
     while (w < blocks) w *= 2;
     return w;
@@ -295,7 +304,7 @@ int scan32_utw_waves(const ScanParams& sp) {
 
 template <typename T>
 bool launch_scan32_utw(const ScanParams& sp, hipStream_t stream) {
-    const int waves = scan32_utw_waves(sp);
+    const int waves = scan32_utw_waves<T>(sp);
     if (waves == 0) return false;
     const unsigned grid = static_cast<unsigned>(sp.B * sp.R * sp.heads);
     auto go = [&](auto wc, auto spc) {
@@ -308,7 +317,9 @@ bool launch_scan32_utw(const ScanParams& sp, hipStream_t stream) {
             case 1: go(std::integral_constant<int, 1>{}, spc); break;
             case 2: go(std::integral_constant<int, 2>{}, spc); break;
             case 4: go(std::integral_constant<int, 4>{}, spc); break;
-            default: go(std::integral_constant<int, 8>{}, spc); break;
+            default:
+                if constexpr (kMaxBlocks<T> == 8) go(std::integral_constant<int, 8>{}, spc);
+                break;
         }
     };
     if (sp.x.spatial) pick(std::true_type{});
