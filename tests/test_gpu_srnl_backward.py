@@ -287,6 +287,14 @@ def test_srnl_backward_block_edges(device, head_dim, chunks, length):
     _block_form_case(device, head_dim, chunks, length, heads=2)
 
 
+@pytest.mark.parametrize("head_dim,chunks,length", [(16, [97, 112, 96, 81], 230), (16, [65, 80, 33, 48], 170),
+                                                    (32, [33, 48, 32, 17], 100)])
+def test_srnl_backward_spare_waves(device, head_dim, chunks, length):
+    """7, 6, 5 and 3 blocks on 8 waves, 3 and 2 on 4: few spare waves leave the readout's
+    gradients to the waves of their blocks, more of them take them all."""
+    _block_form_case(device, head_dim, chunks, length, heads=2)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("head_dim,directions", [(16, 1), (32, 2)])
 def test_srnl_backward_block_inputs(device, head_dim, directions, dtype):

@@ -43,8 +43,6 @@
 // -> 19 + 52 us.  With the forward repeated inside the backward kernel the first three took 249,
 // 710 and 745 us after a separate forward scan of 54, 125 and 130 us; with every wave walking all
 // of a chunk's maps and forming all of H, and transposes as products: 193, 540, 558 and 57 us.
-// The third also has waves without a block of their own, which take the readout's gradients
-// while the others form theirs (512 us with each wave doing its own block's afterwards).
 // Fetching the next chunk's operands ahead changed these by under 3% either way.
 #include <algorithm>
 #include <cmath>
@@ -517,6 +515,13 @@ __device__ __forceinline__ void copy_tiles(const v4f (&from)[ND][ND], v4f (&to)[
         for (int j = 0; j < ND; ++j) to[i][j] = from[i][j];
 }
 
+// Readouts' gradients a wave without a block takes at most.  256 lines, backward of 8 chunks,
+// d = 16, against every wave taking those of its own block: 2 of 4 waves spare, 1 readout each,
+// 67 -> 60 us; 3 of 8, 2 each, 97 -> 89; 2 of 8, 3 each, 100 -> 97; 1 of 8, 7 readouts, 103 ->
+// 124.  d = 32 (12 chunks): 2 of 4, 1 each, 206 -> 178; 1 of 4, 3 readouts, 218 -> 225.
+template <int D>
+constexpr int kSpareReadouts = D == 16 ? 3 : 2;
+
 // Waves per SIMD the register budget is cut for.
 template <int D, int W>
 constexpr int kMinWaves = D == 16 ? (W == 1 ? 3 : 2) : 1;
@@ -861,9 +866,11 @@ __global__ __launch_bounds__(64 * W, (kMinWaves<D, W>)) void srnl_backward_block
         }
 
         // Readout: y = M_m Gamma q^ of every token of the chunk.
-        // Waves without a block of the chunk take it, while the others are in their gradients.
-        const int idle = ch < nc - 1 ? W - nb : 0;
-        const int first = idle <= 0 ? w : w >= nb ? w - nb : nb;
+        // Waves without a block of the chunk take it while the others are in their gradients, where
+        // that leaves a wave few enough of them (kSpareReadouts).
+        const int spare = ch < nc - 1 ? W - nb : 0;
+        const int idle = spare > 0 && nb <= kSpareReadouts<D> * spare ? spare : 0;
+        const int first = idle == 0 ? w : w >= nb ? w - nb : nb;
         for (int blk = first; blk < nb; blk += idle > 0 ? idle : W) {
             const int tl = 16 * blk + tau;
             const Index tok = ch * C + tl;
