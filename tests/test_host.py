@@ -414,3 +414,30 @@ def test_audit_kernel_families_cover_every_scan_and_readout_kernel():
     for name in forward:
         hits = [f for f in SCAN_KERNELS + READOUT_KERNELS if re.fullmatch(re.escape(f), name)]
         assert len(hits) == 1, (name, hits)
+
+
+def test_host_tensors_reach_no_kernel(monkeypatch):
+    """A tensor in host memory raises before the native call, whatever the runtime makes of
+    device index -1 (it takes it as the current device, whose kernel would then read host
+    pointers)."""
+    from visionhope_amd.models.srnl_core import chunk, fused
+    from visionhope_amd.utils import hip
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                assert name.endswith("_bytes"), f"{name} was called"
+                return 1024
+            return call
+
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0)
+    monkeypatch.setattr(hip, "load_library", lambda *_: Library())
+    mems = [torch.zeros(4, 1, 16, 16)] * 3 + [torch.zeros(4, 1, 16)] * 2
+    x = torch.zeros(1, 3, 5, 16)
+    lines = torch.zeros(1, 4, 1, 15, 16)
+    with pytest.raises(ValueError, match="CUDA"):
+        hip.stream_of(x)
+    with pytest.raises(ValueError, match="CUDA"):
+        fused.srnl_spatial_inference(mems, x, x, torch.zeros(16), torch.zeros(4, 16), (5, 5, 3, 3))
+    with pytest.raises(ValueError, match="CUDA"):
+        chunk.srnl_packed_forward(mems, lines, torch.zeros(1, 4, 15, 16), [5] * 4, q_raw=True)

@@ -188,8 +188,12 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_of(tensor: torch.Tensor):
-    """The raw current stream of the tensor's device."""
-    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
+    """The raw current stream of the tensor's device.  Every native call asks for it, so this
+    is also where a tensor in host memory stops short of a kernel."""
+    device = tensor.get_device()
+    if device < 0:
+        raise ValueError(f"Expected a CUDA tensor, got one on {tensor.device}")
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def ptr(tensor):
