@@ -108,3 +108,35 @@ def test_projection_route_does_not_depend_on_gradients(operator, frozen):
     (route, without, _), (route_grad, _, _) = operator.seen
     assert route == route_grad == ("module" if frozen else "projected")
     assert without.data_ptr() == x.data_ptr()
+
+
+class _Recorder:
+    """A native library that runs nothing and records the pointers of each call."""
+
+    def __init__(self):
+        self.pointers = {}
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.pointers[name] = args
+            return 4096 if name.endswith("_bytes") else 0
+        return call
+
+
+def test_backward_takes_saved_tensors_of_any_strides(monkeypatch):
+    """Saved-tensor hooks may hand tensors back with other strides than they were saved with;
+    kernels that read them by pointer get contiguous copies."""
+    lib = _Recorder()
+    monkeypatch.setattr(spatial.hip, "load_library", lambda *_: lib)
+    monkeypatch.setattr(spatial.hip, "stream_of", lambda _: 0)
+    mems, x, q, skip, weights, chunks = _inputs()
+    gains = torch.zeros(64, 2)[:, 0]
+    spatial.srnl_spatial_backward(mems, x, q, skip, weights, chunks, gains, torch.ones_like(x))
+    assert gains.data_ptr() not in lib.pointers["vh_srnl_spatial_backward"]
+    x = torch.zeros(*x.shape, 2)[..., 0]
+    operands = torch.zeros(66, 32, 2)[..., 0]
+    dq = torch.zeros(1, 3, 5, 32)
+    spatial.project_queries_backward(x, operands, dq, dq, True, True)
+    assert x.data_ptr() not in lib.pointers["vh_linear_weight_grad"]
+    first, last = operands.data_ptr(), operands.data_ptr() + 4 * operands.numel()
+    assert not any(isinstance(p, int) and first <= p < last for p in lib.pointers["vh_pointwise_conv_nhwc_forward"])

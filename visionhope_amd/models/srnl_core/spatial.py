@@ -76,7 +76,8 @@ def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
     states = [as_fp32(m) for m in memories]
-    x_c, q_c, g = x.contiguous(), q.contiguous(), as_fp32(dout)
+    # saved tensors come back from hooks with whatever strides those give them
+    x_c, q_c, g, gains = x.contiguous(), q.contiguous(), as_fp32(dout), gains.contiguous()
     skip, wts = as_fp32(d_skip), as_fp32(weights)
     dx, dq = torch.empty_like(x_c), torch.empty_like(q_c)
     grads = [torch.empty_like(t) for t in (*states, skip, wts)]
@@ -156,6 +157,7 @@ def project_queries(x, w, b):
 def project_queries_backward(x, operands, dx, dq, need_dx, need_params):
     """dx + dq W (or None), dW and db (or None) of ``project_queries``."""
     channels = x.shape[-1]
+    x, operands = x.contiguous(), operands.contiguous()
     tokens, lib, stream = x.numel() // channels, hip.load_library(), hip.stream_of(x)
     total = dw = db = None
     if need_dx:
