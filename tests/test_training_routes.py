@@ -140,3 +140,18 @@ def test_backward_takes_saved_tensors_of_any_strides(monkeypatch):
     assert x.data_ptr() not in lib.pointers["vh_linear_weight_grad"]
     first, last = operands.data_ptr(), operands.data_ptr() + 4 * operands.numel()
     assert not any(isinstance(p, int) and first <= p < last for p in lib.pointers["vh_pointwise_conv_nhwc_forward"])
+
+
+@pytest.mark.parametrize("chunk,kept", [(7, True), (6, False)])
+def test_large_gains_are_not_kept(monkeypatch, chunk, kept):
+    """A step keeps its chunk gains up to a size in proportion to the map; beyond that the
+    backward forms them again."""
+    gains = torch.zeros(4 * 3 * -(-168 // chunk) * 32 * 32)   # 4 directions, 3 heads of 32, 168 tokens
+    monkeypatch.setattr(spatial, "srnl_spatial_training_forward", lambda m, x, *_: (x.detach().clone(), gains))
+    seen = []
+    monkeypatch.setattr(spatial, "srnl_spatial_backward", lambda m, x, q, s, w, c, gains, dout: seen.append(gains) or (
+        *m, x, q, s, w))
+    mems = [torch.zeros(4, 3, 32, 32) for _ in range(3)] + [torch.zeros(4, 3, 32) for _ in range(2)]
+    x = torch.zeros(1, 8, 21, 96, requires_grad=True)
+    spatial.srnl_spatial(mems, x, x.detach(), torch.zeros(96), torch.ones(4, 96), (chunk,) * 4).sum().backward()
+    assert len(seen) == 1 and (seen[0] is not None) == kept

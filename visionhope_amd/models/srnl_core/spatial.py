@@ -40,7 +40,7 @@ class SpatialSRNLFunction(torch.autograd.Function):
             raise RuntimeError("SRNL TorchScript tracing is unsupported; use eager or CUDA Graph inference.")
         memories = (M_m_0, M_v_0, M_k_0, M_eta_0, M_alpha_0)
         out, gains = srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks)
-        ctx.save_for_backward(*memories, x, q, d_skip, weights, gains)
+        ctx.save_for_backward(*memories, x, q, d_skip, weights, gains if keeps_gains(x, gains) else None)
         ctx.chunks = chunks
         return out
 
@@ -50,9 +50,23 @@ class SpatialSRNLFunction(torch.autograd.Function):
         return (*srnl_spatial_backward(memories, x, q, d_skip, weights, ctx.chunks, gains, dout), None)
 
 
+# Bytes of chunk gains per map element that a step keeps for its backward, at most.  A chunk of
+# c tokens leaves 16 d / c (four directions, d x d FP32 per head), so this covers chunks from 4
+# tokens at head_dim 16 and 7 at head_dim 32, the smallest maps of the backbones.  What would be
+# more (512 bytes for single-token chunks at head_dim 32, against 4 of a bf16 map and its
+# queries) the backward forms again: 6 x 6 x 256 maps, batch 128, d = 32, 101 MB of gains, 277
+# -> 374 us.
+KEPT_GAIN_BYTES = 80
+
+
+def keeps_gains(x, gains):
+    return gains.numel() * 4 <= KEPT_GAIN_BYTES * x.numel()
+
+
 @on_tensor_device
-def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
-    """The operator's output ``[B, H, W, C]`` FP32 and the gains its backward starts from."""
+def srnl_spatial_gains(memories, x, chunks):
+    """The products of the chunk gains that the backward starts from, and the workspace that
+    ``srnl_spatial_readout`` reads (the content memories at the chunk starts)."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
     states = [as_fp32(m) for m in memories]
@@ -65,17 +79,25 @@ def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
         x_c.data_ptr(), hip.dtype_code(x.dtype), *[m.data_ptr() for m in states], batch, height, width, channels,
         head_dim, chunk_ptr, srnl_consts(), gains.data_ptr(), gains.numel() * 4, ws.data_ptr(), ws.numel() * 4,
         hip.stream_of(x_c)), "vh_srnl_spatial_gains")
-    return srnl_spatial_readout(ws, x_c, q, d_skip, weights, chunks, head_dim), gains
+    return gains, ws
+
+
+def srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks):
+    """The operator's output ``[B, H, W, C]`` FP32 and the gains its backward starts from."""
+    gains, ws = srnl_spatial_gains(memories, x, chunks)
+    return srnl_spatial_readout(ws, x, q, d_skip, weights, chunks, memories[0].shape[-1]), gains
 
 
 @on_tensor_device
 def srnl_spatial_backward(memories, x, q, d_skip, weights, chunks, gains, dout):
     """Gradients of ``SpatialSRNLFunction`` for the output gradient ``dout [B, H, W, C]`` and
-    the ``gains`` of its forward: the five memories, x, q, d_skip and the weights, each
-    shaped and typed like its input."""
+    the ``gains`` of its forward (None: formed again): the five memories, x, q, d_skip and the
+    weights, each shaped and typed like its input."""
     batch, height, width, channels = x.shape
     head_dim = memories[0].shape[-1]
     states = [as_fp32(m) for m in memories]
+    if gains is None:
+        gains = srnl_spatial_gains(memories, x, chunks)[0]
     # saved tensors come back from hooks with whatever strides those give them
     x_c, q_c, g, gains = x.contiguous(), q.contiguous(), as_fp32(dout), gains.contiguous()
     skip, wts = as_fp32(d_skip), as_fp32(weights)
@@ -123,7 +145,7 @@ class ProjectedSpatialSRNLFunction(torch.autograd.Function):
         memories = (M_m_0, M_v_0, M_k_0, M_eta_0, M_alpha_0)
         operands, q = project_queries(x, w, b)
         out, gains = srnl_spatial_training_forward(memories, x, q, d_skip, weights, chunks)
-        ctx.save_for_backward(*memories, x, q, operands, d_skip, weights, gains)
+        ctx.save_for_backward(*memories, x, q, operands, d_skip, weights, gains if keeps_gains(x, gains) else None)
         ctx.chunks = chunks
         return out
 
