@@ -342,6 +342,72 @@ def test_srnl_spatial_backward_validates(lib):
     assert call(nbytes=64)[0] > 64 and call(nbytes=64)[1] == hip.VH_ERR_WORKSPACE
 
 
+def test_srnl_spatial_gains_validates(lib):
+    """The gains entry writes two buffers: it checks the size of both, and what the spatial
+    backward checks."""
+    p = ctypes.c_void_p(0x1000)
+
+    def call(head_dim=16, chunk=4, C=32, H=4, W=4, dtype=hip.VH_DTYPE_F32, gains=None, content=None, null=None,
+             consts=None):
+        arr, keep = hip.int64_array([chunk] * 4)
+        size = lib.vh_srnl_spatial_gains_bytes(1, H, W, C, head_dim, arr)
+        args = [p, dtype, p, p, p, p, p, 1, H, W, C, head_dim, arr, consts or _consts(), p,
+                size if gains is None else gains, p, 1 << 30 if content is None else content, None]
+        if null is not None:
+            args[null] = None
+        return size, lib.vh_srnl_spatial_gains(*args)
+
+    assert call(head_dim=8) == (0, hip.VH_ERR_HEAD_DIM)
+    assert call(head_dim=64, C=64) == (0, hip.VH_ERR_HEAD_DIM)
+    assert call(chunk=257) == (0, hip.VH_ERR_ARG)
+    assert call(chunk=0) == (0, hip.VH_ERR_ARG)
+    assert call(C=40) == (0, hip.VH_ERR_SHAPE)
+    assert call(H=0) == (0, hip.VH_ERR_SHAPE)
+    assert call(H=1 << 12, W=1 << 12)[1] == hip.VH_ERR_SHAPE
+    assert call(dtype=9)[1] == hip.VH_ERR_DTYPE
+    assert call(consts=hip.make_consts(0.025, 0.0, 2.197224577, 0.0, True, 0.999999))[1] == hip.VH_ERR_ARG
+    for pointer in (0, 2, 3, 4, 5, 6, 12, 14, 16):
+        assert call(null=pointer)[1] == hip.VH_ERR_ARG, pointer
+    # 8 lines of 16 tokens, 4 chunks each: 32 matrices of 16 x 16 floats in either buffer
+    size = call(gains=0)[0]
+    assert size == 32 * 1024
+    assert call(gains=size - 1)[1] == hip.VH_ERR_WORKSPACE
+    assert call(content=size - 1)[1] == hip.VH_ERR_WORKSPACE
+
+
+def test_linear_training_entries_validate(lib):
+    """vh_linear_operands and vh_linear_weight_grad check pointers, widths, dtype and workspace."""
+    p = ctypes.c_void_p(0x1000)
+
+    def operands(n=32, k=48, dtype=hip.VH_DTYPE_F32, null=None):
+        args = [p, p, dtype, n, k, p, p, p, None]
+        if null is not None:
+            args[null] = None
+        return lib.vh_linear_operands(*args)
+
+    for pointer in (0, 1, 5, 6, 7):
+        assert operands(null=pointer) == hip.VH_ERR_ARG
+    assert operands(n=0) == operands(k=-1) == operands(n=1 << 16, k=1 << 15) == hip.VH_ERR_SHAPE
+    assert operands(dtype=9) == hip.VH_ERR_DTYPE
+
+    def weight_grad(m=100, n=32, k=48, nbytes=None, null=None):
+        size = lib.vh_linear_weight_grad_workspace_bytes(m, n, k)
+        args = [p, p, m, n, k, p, p, p, size if nbytes is None else nbytes, None]
+        if null is not None:
+            args[null] = None
+        return size, lib.vh_linear_weight_grad(*args)
+
+    for pointer in (0, 1, 5, 6):
+        assert weight_grad(null=pointer)[1] == hip.VH_ERR_ARG
+    for bad in (dict(m=0), dict(n=40), dict(k=24), dict(n=0), dict(k=-16)):
+        assert weight_grad(**bad) == (0, hip.VH_ERR_SHAPE), bad
+    assert weight_grad(null=7)[1] == hip.VH_ERR_WORKSPACE
+    size = weight_grad(nbytes=0)[0]
+    assert size == (32 * 48 + 32) * 4
+    assert weight_grad(nbytes=size - 1)[1] == hip.VH_ERR_WORKSPACE
+    assert lib.vh_linear_weight_grad_workspace_bytes(1 << 20, 128, 128) <= 8 << 20
+
+
 def test_dispatch_overrides_are_validated(lib):
     """Kernel choices are forced only through vh_set_dispatch_override, which rejects unknown
     names and malformed values; nothing is read from the environment."""

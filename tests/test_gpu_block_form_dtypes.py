@@ -3,8 +3,8 @@ activations, through the spatial operator (``vh_srnl_spatial_forward``, FP32 out
 the sequence entry, against the C oracle on the same inputs.
 
 Each shape runs the library's own dispatch: one workgroup per line with a chunk's blocks over
-1 or 2 waves (head_dim 16: chunks of one block, or few lines), the packed one-wave form (2,048
-lines with longer chunks, in the edge cases) and the head_dim-32 form with chunks of 14 and 56
+1 or 2 waves (head_dim 16: chunks of one block, or few lines), the packed one-wave form (longer
+chunks from 2,048 lines, unaligned rows) and the head_dim-32 form with chunks of 14 and 56
 tokens (1 and 4 waves).  fp16 values are exact as bf16 hi + lo
 operands and FP32 values enter within 2^-16 of their value, so both are held to the bound of
 the bf16 block form, 2e-5 (about one hi + lo rounding of the output, five times inside the
@@ -168,3 +168,27 @@ def test_wide_heads_long_chunks_keep_fp32_products(oracle, device, batch, height
                                  skip.to(device), wts.to(device), (width, width, height, height)).cpu().numpy()
     expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 32)
     assert rel_err(got, expected) <= 64 ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("batch,height,width,heads,offset", [
+    (64, 17, 5, 8, 0), (128, 17, 5, 8, 0), (129, 5, 18, 8, 0), (114, 18, 20, 9, 0), (64, 3, 130, 4, 0),
+    (2, 17, 5, 4, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_packed_scan_by_default(oracle, device, batch, height, width, heads, offset, dtype):
+    """What the library gives to the packed scan by itself: chunks of more than 16 tokens from
+    2,048 lines (one line per wave), from 4,096 with an even and an odd number of heads (two
+    lines per wave, one), chunks of more than 128 from 1,024 lines, and rows that are not
+    aligned for vector loads."""
+    from visionhope_amd.models.srnl_core.fused import srnl_spatial_inference
+
+    channels = 16 * heads
+    seed = 1000 * height + width + heads
+    mems = memories(4, heads, 16, kind="strong", seed=seed)
+    x, q = (randn(batch, height, width, channels, seed=seed + i).to(dtype) for i in (1, 2))
+    skip, wts = randn(channels, seed=seed + 3, scale=0.1), 1 + randn(4, channels, seed=seed + 4, scale=0.1)
+    xd = torch.empty(x.numel() + offset, dtype=dtype, device=device)[offset:].view(x.shape).copy_(x)
+    got = srnl_spatial_inference(tuple(torch.from_numpy(m).to(device) for m in mems), xd, q.to(device),
+                                 skip.to(device), wts.to(device), (width, width, height, height)).cpu().numpy()
+    expected = oracle.operator_forward(x.float().numpy(), q.float().numpy(), mems, skip.numpy(), wts.numpy(), 16)
+    r, m = rel_err(got, expected), max_rel_err(got, expected)
+    assert r <= BLOCK_TOL and m <= BLOCK_TOL, f"{dtype} {height}x{width}: normwise {r:.3e}, elementwise {m:.3e}"

@@ -1,7 +1,7 @@
 """The spatial SRNL kernels at the Tiny B = 128 stage shapes, where the library's own
-dispatch (no override) picks the block-form scan with its per-stage packings (1 x 4 tiles
-at 1024 lines, 1 x 2 at 2048, 2 x 2 at 4096 and 8192) and the matrix-core readout on
-split chunk states, checked against the C oracle on the same bf16 inputs:
+dispatch (no override) picks a block-form scan (one workgroup per line at 56 x 56, 14 x 14
+and 7 x 7, packed with 1 x 2 tiles at the 2048 lines of 28 x 28) and the matrix-core readout
+on split chunk states, checked against the C oracle on the same bf16 inputs:
 
 * the fused entry (``vh_srnl_spatial_forward``, FP32 output) at a bound the block form's
   arithmetic supports: 2e-5, about one hi + lo rounding (2^-16 = 1.5e-5 relative) of the
