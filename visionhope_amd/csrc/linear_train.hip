@@ -170,9 +170,10 @@ __global__ __launch_bounds__(256) void linear_grad_reduce_kernel(const float* pa
     else db[idx - weights] = acc;
 }
 
-// Workgroups over the tokens: at least 256 tokens each, at most 512, and partial sums of at most
-// 8 MB, written and read once more (at 256 tokens and 128 + 128 channels a workgroup reads 128 KB
-// and writes 64).
+// Workgroups over the tokens: about 256 tokens each (whole steps of 64; M = 257 gives 192 and
+// 65), at most 512 of them, and partial sums of at most 8 MB unless a single part is larger,
+// written and read once more (at 256 tokens and 128 + 128 channels a workgroup reads 128 KB and
+// writes 64).
 int64_t weight_grad_parts(int64_t M, int64_t N, int64_t K) {
     const int64_t width = N * K + N;
     return std::max<int64_t>(1, std::min({(M + 255) / 256, static_cast<int64_t>(512), (int64_t(2) << 20) / width}));

@@ -1265,9 +1265,10 @@ constexpr int dtype_code_of() {
     return std::is_same<T, float>::value ? VH_DTYPE_F32 : std::is_same<T, bf16_t>::value ? VH_DTYPE_BF16 : VH_DTYPE_F16;
 }
 
-// Waves per line of the wide scan for this call: 0 = use the single-wave kernels.  Every
-// head_dim-32 scan and head_dim-16 scans with fewer lines than SIMDs use it.  The
-// scan_wide override (0 | 1 | 2 | 4) forces the choice (1 only for head_dim 16); a
+// Waves per line of the wide scan for this call where the block forms do not take it: 0 = use
+// the single-wave kernels.  By default head_dim-32 scans reach it with chunks beyond the block
+// form's (128 tokens for bf16, 64 for FP32; fp16 runs the stepped form), head_dim-16 scans with
+// chunks of more than 128 tokens and fewer lines than SIMDs.  The scan_wide override (0 | 1 | 2 | 4) forces the choice (1 only for head_dim 16); a
 // scan_pack override (a forced head_dim-16 packing) selects the single-wave kernels.
 int wide_waves(int64_t lines, int d) {
     const Override forced("scan_wide");
@@ -1303,7 +1304,8 @@ void launch_scan(const ScanParams& sp, hipStream_t stream) {
     if constexpr (D == 16 || D == 32) {
         const int waves = wide_waves(lines, D);
         // Token blocks (head_dim 16, chunks of 64 tokens or more, several waves): measured
-        // faster than the row split there, slower for shorter chunks and for head_dim 32.
+        // faster than the row split there, slower for shorter chunks (which get here only under
+        // an override) and for head_dim 32.
         // The scan_tb override (1 | 2) forces the row split or the blocks.
         int max_chunk = 0;
         for (int r = 0; r < sp.R; ++r) max_chunk = std::max(max_chunk, sp.chunk[r]);
@@ -1312,12 +1314,14 @@ void launch_scan(const ScanParams& sp, hipStream_t stream) {
         if (tb.set()) token_blocks = tb.as_int() == 1 ? 1 : 2;
         if constexpr (D == 16) {
             // One workgroup per line (srnl_utw.hip), unless a dispatch override forces another
-            // form: chunks of one 16-token block at any line count (4,096 lines of 14: 46.7
-            // against 51.7 us, 8,192 of 7: 40.7 against 48.5, 1,024 of 14: 21 against 46), longer
-            // chunks below 2,048 lines (1,024 lines of 56: 179 against 202 us, of 28: 59 against
-            // 96).  From there the waves of a chunk compete for the SIMDs and the packed form
-            // (srnl_ut.hip) is level or ahead: 2,048 lines of 28: 92 against 86 us, of 56: 323
-            // against 322, of 80: 828 against 646; 4,096 of 40: 368 against 345.
+            // form: chunks of one 16-token block at any line count (4,096 lines of 14: 44 against
+            // 52 us, 16,384 of 7: 70 against 86, 32,768 of 16: 332 against 394, 1,024 of 14: 21
+            // against 46), longer chunks below 2,048 lines (1,024 lines of 28: 58 against 96 us, of
+            // 56: 179 against 201, of 80: 421 against 522, of 128: 842 against 941; 1,536 of 80: 625
+            // against 1,053; 2,032 of 28: 93 against 186, of 80: 823 against 1,041, of 128: 1,625
+            // against 1,880; FP32 maps alike).  From 2,048 the packed form (srnl_ut.hip) gives every
+            // SIMD two waves and is level or ahead: 2,048 lines of 28: 92 against 86 us, of 32: 103
+            // against 97, of 56: 323 against 322, of 80: 828 against 646; 4,096 of 40: 368 against 345.
             const Override utw("scan_utw");   // "1": whenever the chunks allow, "0": never
             const bool utw_on = utw.set() ? utw.value[0] == '1'
                                           : !Override("scan_pack").set() && (max_chunk <= 16 || lines < 2048);
@@ -1433,10 +1437,12 @@ void scan16_packing(int64_t lines, int64_t heads, int* nl, int* tcw) {
     }
 }
 
-// Packing of the block-form scan (srnl_ut.hip, 200-310 VGPRs: one or two waves per SIMD).
-// Measured on MI355X at the Tiny stages (B = 128, scan launches alone): 1 x 4 for 1024
-// lines (chunk 56: 270 us; 1 x 2 301 us), 1 x 2 for 2048 (chunk 28: 104 us; 1 x 4 217 us),
-// 2 x 2 for 4096 and 8192 (chunks 14 and 7: 56.5 and 53 us; 4 x 4 71 and 68 us).
+// Packing of the block-form scan (srnl_ut.hip, 200-310 VGPRs: one or two waves per SIMD), which
+// by default takes chunks of more than 16 tokens from 2,048 lines, chunks of more than 128 from
+// 1,024, and rows that are not aligned for vector loads.  Scan launches alone on MI355X: 1 x 2
+// for 2,048 lines (chunk 28: 88 us; 1 x 4 187, 2 x 2 134), 2 x 2 for 4,096 and more (chunk 40:
+// 346 us; 1 x 2 422; chunk 80: 1,123 against 1,265; chunks of 28 and 56 level: 171 against 163
+// and 634 against 625), 1 x 4 below 2,048 (1,024 lines of 136: 1,357 us; 1 x 2 1,418).
 // The scan_pack override applies as for the stepped form.
 void scan16_ut_packing(int64_t lines, int64_t heads, int* nl, int* tcw) {
     if (Override("scan_pack").set()) {

@@ -1,6 +1,6 @@
 // The 16-token block form on the FP32 matrix cores: tile products, token order, decays and
-// triangular solves shared by the few-line scan (srnl_utw.hip) and the backward
-// (srnl_backward_blocks.hip).
+// triangular solves shared by the scans with one workgroup per line (srnl_utw.hip,
+// srnl_utw32.hip) and the backward (srnl_backward_blocks.hip).
 //
 // A tile is 4 registers: lane (g = l / 16, c = l % 16) holds rows 4g..4g+3 of column c, which
 // is what the matrix core returns, the B operand of that matrix and the A operand of its

@@ -18,9 +18,10 @@
 //
 // Keys, differences and coefficients of a 64-token segment are double-buffered in LDS, so
 // one barrier separates a segment's token phase from its recurrence; the state is
-// double-buffered, so the refresh needs two barriers per chunk.  Used when there are too
-// few lines to give every SIMD a wave of its own (VisionHOPE-Base at 512^2, the d = 32
-// operator of config 3) and for every head_dim-32 scan.
+// double-buffered, so the refresh needs two barriers per chunk.  Used for chunks beyond the
+// block forms with one workgroup per line (srnl_utw.hip, srnl_utw32.hip): head_dim 32 with
+// chunks of more than 128 tokens (bf16) or 64 (FP32), head_dim 16 with more than 128 where the
+// lines are too few to give every SIMD a wave of its own.
 //
 // Operands of the matrix products: lane l = 16 q + n supplies, for column n (a token, or
 // a column of G), the K-range [q D/4, (q+1) D/4), and receives rows 4q..4q+3 of column n
