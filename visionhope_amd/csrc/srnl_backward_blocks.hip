@@ -37,10 +37,10 @@
 // Bound: the dependency chain of a chunk, and within it the issue of the FP32 products, which
 // hold the vector pipe (34 cycles each, srnl_utw.hip); the bytes take under a tenth of the time.
 // Times on MI355X against the token-by-token kernel (which head_dim 4 and 8 still run), gains +
-// backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 78 + 186 us; 512 lines of
-// 3,136 tokens, d = 16, chunks of 56: 24,500 -> 185 + 501 us; 48 lines of 960 tokens, d = 32,
-// chunks of 40 and 24: 11,800 -> 174 + 424 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
-// -> 19 + 52 us.  With the forward repeated inside the backward kernel the first three took 249,
+// backward: 4,096 lines of 196 tokens, d = 16, chunks of 14: 2,480 -> 79 + 192 us; 512 lines of
+// 3,136 tokens, d = 16, chunks of 56: 24,500 -> 186 + 510 us; 48 lines of 960 tokens, d = 32,
+// chunks of 40 and 24: 11,800 -> 172 + 422 us; 4 lines of 196 tokens, d = 32, chunks of 64: 1,690
+// -> 18 + 52 us.  With the forward repeated inside the backward kernel the first three took 249,
 // 710 and 745 us after a separate forward scan of 54, 125 and 130 us; with every wave walking all
 // of a chunk's maps and forming all of H, and transposes as products: 193, 540, 558 and 57 us.
 // Fetching the next chunk's operands ahead changed these by under 3% either way.

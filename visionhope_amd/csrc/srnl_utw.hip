@@ -24,10 +24,10 @@
 // 389 us where the split ones take 296.)  Bound by the dependency chain of a chunk.
 //
 // Per launch on MI355X, against the form that carried the whole 64 x 16 state and solved
-// (I + L) by columns on the vector unit: 96 lines of 16,384 tokens (chunks of 128) 370 -> 296
+// (I + L) by columns on the vector unit: 96 lines of 16,384 tokens (chunks of 128) 370 -> 288
 // us, 64 lines of 600 (30, 20) 64 -> 44, 32 lines of 196 (14) 30 -> 18; against the packed form
-// (srnl_ut.hip): 1,024 lines of 3,136 (56) 202 -> 179, 4,096 of 196 (14) 52 -> 47, 8,192 of 49
-// (7) 48 -> 42.
+// (srnl_ut.hip): 1,024 lines of 3,136 (56) 202 -> 179, 4,096 of 196 (14) 52 -> 44, 8,192 of 49
+// (7) 48 -> 40.
 #include <algorithm>
 
 #include "srnl_block_form.h"
